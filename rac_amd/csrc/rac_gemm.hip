@@ -1,5 +1,5 @@
-// rac_gemm.hip — rotate-project-accumulate GEMM for gfx950 (VALU; FAST mode
-// on the FP32 matrix cores where the launch is large enough).
+// rac_gemm.hip — rotate-project-accumulate GEMM for gfx950: the VALU tiles of
+// the CORDIC and SHIFTADD MACs, and the dispatch of every product.
 //
 // C[M,N] = alpha * op(A) @ op(B) (+ beta * C), row-major, with the MAC of
 // rac_fma_iters (rac_kernels.hip:204-219):
@@ -20,28 +20,21 @@
 // and reads only 2 ds_read_b128 per 16 MACs; the rotations of those MACs
 // advance step-major, so independent FMA chains interleave in each wave's
 // instruction stream.  FAST mode (1 FMA per MAC) runs on the matrix cores
-// (gemm_mfma_fast_kernel, below) when it has enough 128x128 blocks and
-// K >= 128; otherwise on VALU tiles of 8x8 or 16x8 per lane (8x8 split in
-// 4x4 groups 64 apart, conflict-free LDS reads), the k loop unrolled by 2,
-// bound by LDS bandwidth (128 B/clk/CU) as much as by the FMA rate.
-// Launches with fewer than 1024 block tiles step down to 64x64, then 32x32
-// (2x2 per lane; CORDIC and SHIFTADD below 2 blocks of 64x64 per CU) so
+// (rac_gemm_fast.hip), here only for what those cannot read (K < 4).
+// Launches with fewer than 2 blocks of 64x64 per CU step down to 32x32 (2x2
+// per lane) so
 // every SIMD holds several waves.  The next K-tile is
 // prefetched into registers while the current one is computed.
 #include <hip/hip_runtime.h>
 #include <atomic>
 #include "rac_act.hpp"
+#include "rac_gemm.hpp"
 
 namespace rac {
 
 // CORDIC mode: rotations of kGroupRows tile rows (x TN columns) advance
 // step-major (8 interleaved chains in the 4x4 register tile).
 constexpr int kGroupRows = 2;
-// Fewer block tiles than this (4 per CU) leave SIMDs with one wave or none;
-// such launches step down to a smaller tile (64x64, then 32x32; the CORDIC
-// and SHIFTADD 64x64 tile down to 2 blocks per CU).
-constexpr long kMinTiles = 1024;
-
 // Offset of a lane's i-th row (or column) inside the block tile, for the
 // lane's 16-way index t.  Register tiles of 4k are split into k groups of 4
 // spaced 64 apart, so a wave's float4 LDS reads of one group cover 256
@@ -52,10 +45,6 @@ __device__ __forceinline__ int lane_off(int t, int i) {
     if constexpr (TT % 4 == 0) return (i >> 2) * 64 + t * 4 + (i & 3);
     else return t * TT + i;
 }
-
-// FAST MACs are one FMA each: the k loop is unrolled by this so the next
-// k-step's LDS reads issue under the current step's FMAs.
-constexpr int kFastKUnroll = 2;
 
 template <int MODE, int NITER, bool TA, bool TB, int TM, int TN>
 struct GemmCfg {
@@ -90,16 +79,6 @@ __device__ __forceinline__ float mac(float a, float b, uint32_t bsign, float acc
     } else {
         return acc + shiftadd_mul(a, b, iters);
     }
-}
-
-// Column tiles of row tile r in a causal score trapezoid (query rows
-// row0 + r*BM .. row0 + r*BM + BM - 1, keys 0 .. N-1): those holding a key
-// position not past the row tile's last query position.
-__host__ __device__ __forceinline__ int trap_cols(int row0, int r, int BM, int BN, int N) {
-    const long last = (long)row0 + (long)(r + 1) * BM - 1;
-    const long c = last / BN + 1;
-    const long ntn = (N + BN - 1) / BN;
-    return (int)(c < ntn ? c : ntn);
 }
 
 template <int MODE, int NITER, bool TA, bool TB, int TM, int TN, bool FUSED, int SCHED>
@@ -250,7 +229,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(
             // per trip (measured: 1024^3 0.616 -> 0.542 ms, the attention
             // core with P kept 9.75 -> 9.36 ms; the 4096^3 NN launch 1%
             // slower, so it keeps one).  The accumulation order is unchanged.
-            constexpr int KU = (MODE == kModeFast) ? kFastKUnroll : ((TM * TN <= 4 || SCHED == 1 || SCHED == 2) ? 2 : 1);
+            constexpr int KU = (TM * TN <= 4 || SCHED == 1 || SCHED == 2) ? 2 : 1;
 #pragma unroll 1
             for (int kb = 0; kb < BK; kb += KU)
 #pragma unroll
@@ -381,216 +360,6 @@ __global__ __launch_bounds__(256) void gemm_kernel(
     }   // pass
 }
 
-// ── FAST mode on the matrix cores ───────────────────────────────────────
-//
-// v_mfma_f32_32x32x1_2b_f32 adds one product to each of its 2 x 32 x 32
-// accumulators: D = A_i * B_j + C_ij with a single IEEE rounding, denormals
-// kept — the same value as fmaf(a, b, acc) (checked on gfx950 over 8.4 M
-// random, subnormal, special and exactly cancelling operands, 0 differences,
-// where a separately rounded multiply and add differ in 37%).  Issued once
-// per k in k order, it therefore gives every output the FAST MAC's
-// accumulation chain bit for bit, at 2048 MACs per instruction for 3 LDS
-// floats per lane and k, where the VALU form is bound by LDS bandwidth
-// (4096^3: 1.06-1.15 ms against 1.48-1.53 ms on the 16x8 VALU tile).
-//
-// Block tile 2 WR x 128, BK = 32, staged global -> registers -> LDS with
-// the next K-tile's loads in flight during the current one's MFMAs; 4
-// waves in 2 x 2, each owning WR x 64 outputs (WR = 64 or 128) as 2 WR / 32
-// instructions per k on independent accumulators (a dependent MFMA waits
-// ~100 cycles for its predecessor, ~65 cycles of issue, so more chains per
-// wave keep the matrix core busier).  For each 64-row group of the wave
-// tile, lane l supplies A row l (lanes 0-31 feed the instruction's block 0,
-// lanes 32-63 its block 1) and B column l % 32 of a 32-column half (both
-// blocks read the same 32 columns), so block b covers rows 32 b .. 32 b + 31.
-// Accumulator register r of lane l holds block r / 16, row
-// ((r % 16) / 4) * 8 + (l / 32) * 4 + r % 4 of that block, column l % 32.
-typedef float v32f __attribute__((ext_vector_type(32)));
-constexpr int kMfBN = 128, kMfBK = 32, kMfMinK = 128;
-
-// One operand's K-tile (32 k x ROWS rows) in LDS.  An operand stored with k
-// contiguous in memory (A, or B^T of the NT layout) is kept as [row][k]
-// rows of 36 floats, so a lane reads 4 consecutive k of its row in one
-// ds_read_b128 (rows 144 B apart: 16 lanes cover all 64 banks); the other
-// layout stays [k][row] (rows of ROWS + 4 floats) and is read one k at a time.
-template <bool KC, int ROWS>
-struct MfTile {
-    static constexpr int kRows = KC ? ROWS : kMfBK;
-    static constexpr int kCols = KC ? kMfBK + 4 : ROWS + 4;
-    static constexpr int kVecs = ROWS * kMfBK / 4 / 256;      // float4 per lane
-};
-
-// Global -> registers: the 32 x ROWS tile at k0 (rows r0.. of an operand
-// with `rows` rows, leading dimension ld) as float4 per lane, zero outside
-// the matrix.  k-contiguous: 8 consecutive lanes read a row's 128
-// contiguous bytes; otherwise ROWS / 4 consecutive lanes read one k's
-// 4 ROWS contiguous bytes.  `vec`: 16-byte loads are aligned (base and ld
-// multiples of 4 floats); otherwise every element is loaded on its own.
-template <bool KC, int ROWS>
-__device__ __forceinline__ void mf_load(const float* __restrict__ P, long ld, long rows, long K, long r0, int k0,
-                                        bool vec, float4 (&v)[MfTile<KC, ROWS>::kVecs]) {
-    constexpr int kPerK = ROWS / 4;
-    const int tid = threadIdx.x;
-#pragma unroll
-    for (int r = 0; r < MfTile<KC, ROWS>::kVecs; r++) {
-        const int idx = tid + r * 256;
-        float e[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        if constexpr (KC) {
-            const long gr = r0 + (idx >> 3), gk = (long)k0 + (idx & 7) * 4;
-            const float* q = P + gr * ld + gk;
-            if (vec && gr < rows && gk + 3 < K) {
-                v[r] = *reinterpret_cast<const float4*>(q);
-                continue;
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (gr < rows && gk + j < K) e[j] = q[j];
-        } else {
-            const long gk = (long)k0 + idx / kPerK, gr = r0 + (idx % kPerK) * 4;
-            const float* q = P + gk * ld + gr;
-            if (vec && gk < K && gr + 3 < rows) {
-                v[r] = *reinterpret_cast<const float4*>(q);
-                continue;
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (gk < K && gr + j < rows) e[j] = q[j];
-        }
-        v[r] = make_float4(e[0], e[1], e[2], e[3]);
-    }
-}
-
-// S: the tile's LDS array (kRows x kCols floats, row-major)
-template <bool KC, int ROWS>
-__device__ __forceinline__ void mf_store(float* S, const float4 (&v)[MfTile<KC, ROWS>::kVecs]) {
-    constexpr int kPerK = ROWS / 4, kC = MfTile<KC, ROWS>::kCols;
-    const int tid = threadIdx.x;
-#pragma unroll
-    for (int r = 0; r < MfTile<KC, ROWS>::kVecs; r++) {
-        const int idx = tid + r * 256;
-        if constexpr (KC) *reinterpret_cast<float4*>(&S[(idx >> 3) * kC + (idx & 7) * 4]) = v[r];
-        else *reinterpret_cast<float4*>(&S[(idx / kPerK) * kC + (idx % kPerK) * 4]) = v[r];
-    }
-}
-
-// k = 4q .. 4q+3 of tile row `row`
-template <bool KC, int ROWS>
-__device__ __forceinline__ float4 mf_read4(const float* S, int row, int q) {
-    constexpr int kC = MfTile<KC, ROWS>::kCols;
-    if constexpr (KC) return *reinterpret_cast<const float4*>(&S[row * kC + 4 * q]);
-    else return make_float4(S[4 * q * kC + row], S[(4 * q + 1) * kC + row], S[(4 * q + 2) * kC + row],
-                            S[(4 * q + 3) * kC + row]);
-}
-
-// WR: rows of a wave's tile (64: 2 accumulator chains per wave, 128: 4);
-// the block tile is 2 WR x 128.  TRAP: causal attention scores of query
-// rows row0 .. row0 + M - 1 against keys 0 .. N - 1, only the tiles on or
-// below the diagonal (trap_cols per row tile, numbered row by row along
-// grid x, as gemm_kernel's schedule 3); the masked softmax overwrites the
-// scores above the diagonal, so the others are never read.
-template <bool TA, bool TB, bool FUSED, int WR, bool TRAP = false>
-__global__ __launch_bounds__(256, WR == 128 ? 2 : 1) void gemm_mfma_fast_kernel(
-    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
-    int M, int N, int K, float alpha, float beta, int iters, long sa, long sb, long sc, GemmEpilogue ep,
-    int vec_a, int vec_b, const int* k_causal, int row0)
-{
-    constexpr bool KA = !TA, KB = TB;     // operand stored with k contiguous
-    constexpr int BM = 2 * WR, BN = kMfBN, WI = WR / 64;
-    using TAt = MfTile<KA, BM>;
-    using TBt = MfTile<KB, BN>;
-    int tm = blockIdx.y, tn = blockIdx.x;
-    if constexpr (TRAP) {
-        int l = blockIdx.x;
-        tm = 0;
-        for (;;) {
-            const int c = trap_cols(row0, tm, BM, BN, N);
-            if (l < c) break;
-            l -= c;
-            tm++;
-        }
-        tn = l;
-    }
-    const long m0 = (long)tm * BM, n0 = (long)tn * BN;
-    A += (long)blockIdx.z * sa;
-    B += (long)blockIdx.z * sb;
-    C += (long)blockIdx.z * sc;
-    __shared__ __attribute__((aligned(16))) float sA[TAt::kRows][TAt::kCols];
-    __shared__ __attribute__((aligned(16))) float sB[TBt::kRows][TBt::kCols];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = (wave >> 1) * WR, wc = (wave & 1) * 64;
-    const long lda = TA ? M : K, ldb = TB ? K : N;
-
-    v32f acc[WI][2];
-#pragma unroll
-    for (int i = 0; i < WI; i++)
-#pragma unroll
-        for (int r = 0; r < 32; r++) {
-            acc[i][0][r] = 0.0f;
-            acc[i][1][r] = 0.0f;
-        }
-    float4 va[TAt::kVecs], vb[TBt::kVecs];
-    // Zero operands past K leave an accumulator unchanged: fma(0, 0, acc)
-    // == acc because acc starts at +0 and never becomes -0.  Causal P V
-    // (*k_causal == 1: every v finite) stops after the tile's last query
-    // position, as gemm_kernel does.
-    int kend = K;
-    if (k_causal && *k_causal == 1) kend = (int)min((long)K, (long)row0 + m0 + BM);
-    mf_load<KA, BM>(A, lda, M, K, m0, 0, vec_a, va);
-    mf_load<KB, BN>(B, ldb, N, K, n0, 0, vec_b, vb);
-    for (int k0 = 0; k0 < kend; k0 += kMfBK) {
-        __syncthreads();
-        mf_store<KA, BM>(&sA[0][0], va);
-        mf_store<KB, BN>(&sB[0][0], vb);
-        __syncthreads();
-        if (k0 + kMfBK < kend) {
-            mf_load<KA, BM>(A, lda, M, K, m0, k0 + kMfBK, vec_a, va);
-            mf_load<KB, BN>(B, ldb, N, K, n0, k0 + kMfBK, vec_b, vb);
-        }
-#pragma unroll
-        for (int q = 0; q < kMfBK / 4; q++) {
-            float4 a[WI];
-#pragma unroll
-            for (int i = 0; i < WI; i++) a[i] = mf_read4<KA, BM>(&sA[0][0], wr + 64 * i + lane, q);
-            const float4 b0 = mf_read4<KB, BN>(&sB[0][0], wc + (lane & 31), q);
-            const float4 b1 = mf_read4<KB, BN>(&sB[0][0], wc + 32 + (lane & 31), q);
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-#pragma unroll
-                for (int i = 0; i < WI; i++) {
-                    const float aj = j == 0 ? a[i].x : j == 1 ? a[i].y : j == 2 ? a[i].z : a[i].w;
-                    const float b0j = j == 0 ? b0.x : j == 1 ? b0.y : j == 2 ? b0.z : b0.w;
-                    const float b1j = j == 0 ? b1.x : j == 1 ? b1.y : j == 2 ? b1.z : b1.w;
-                    acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x1f32(aj, b0j, acc[i][0], 0, 0, 0);
-                    acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x1f32(aj, b1j, acc[i][1], 0, 0, 0);
-                }
-        }
-    }
-
-    const long col0 = n0 + wc + (lane & 31);
-#pragma unroll
-    for (int i = 0; i < WI; i++)
-#pragma unroll
-    for (int r = 0; r < 32; r++) {
-        const long gm = m0 + wr + 64 * i + (r / 16) * 32 + ((r % 16) / 4) * 8 + (lane / 32) * 4 + (r % 4);
-        if (gm >= M) continue;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const long gn = col0 + 32 * h;
-            if (gn >= N) continue;
-            float* cp = C + gm * N + gn;
-            const float x = acc[i][h][r];
-            // rac_kernels.hip:267-272
-            float v = (beta != 0.0f) ? __builtin_fmaf(alpha, x, beta * *cp) : alpha * x;
-            if constexpr (FUSED) {
-                // rac_torch.cu:770-775
-                if (ep.bias) v = v + ep.bias[gn];
-                if (ep.pre) ep.pre[gm * N + gn] = v;
-                v = act_rt(v, ep.act, iters, ep.khinv);
-            }
-            *cp = v;
-        }
-    }
-}
-
 // flag = 1 unless some x[i] is inf or NaN (flag must be 1 on entry; lanes
 // only ever store 0, so concurrent stores agree).
 __global__ __launch_bounds__(256) void all_finite_kernel(const float* __restrict__ x, long n,
@@ -613,23 +382,6 @@ hipError_t all_finite_launch(const float* x, long n, int* flag, hipStream_t s) {
     return hipGetLastError();
 }
 
-struct GemmArgs {
-    const float* A;
-    const float* B;
-    float* C;
-    int M, N, K;
-    float alpha, beta;
-    int iters;
-    int batch;
-    long sa, sb, sc;
-    GemmEpilogue ep;
-    bool fused;
-    int sched;
-    const int* k_causal;
-    int exact_specials;
-    int row0;
-};
-
 template <int MODE, int NITER, bool TA, bool TB, bool FUSED, int SCHED, int TM, int TN = TM>
 static hipError_t launch_cfg(const GemmArgs& g, hipStream_t stream) {
     using Cfg = GemmCfg<MODE, NITER, TA, TB, TM, TN>;
@@ -646,27 +398,6 @@ static hipError_t launch_cfg(const GemmArgs& g, hipStream_t stream) {
     hipLaunchKernelGGL((gemm_kernel<MODE, NITER, TA, TB, TM, TN, FUSED, SCHED>), grid, dim3(256), 0, stream,
                        g.A, g.B, g.C, g.M, g.N, g.K, g.alpha, g.beta, g.iters, kinv, g.sa, g.sb, g.sc,
                        g.ep, g.k_causal, g.exact_specials, g.row0);
-    return hipGetLastError();
-}
-
-template <bool TA, bool TB, bool FUSED, int WR, bool TRAP = false>
-static hipError_t launch_mfma_fast(const GemmArgs& g, hipStream_t stream) {
-    constexpr int BM = 2 * WR;
-    dim3 grid((unsigned)((g.N + kMfBN - 1) / kMfBN), (unsigned)((g.M + BM - 1) / BM), (unsigned)g.batch);
-    if constexpr (TRAP) {
-        long t = 0;
-        for (int r = 0; r < (int)grid.y; r++) t += trap_cols(g.row0, r, BM, kMfBN, g.N);
-        grid = dim3((unsigned)t, 1, (unsigned)g.batch);
-    }
-    // 16-byte loads need 16-byte aligned rows in every batch item
-    auto aligned = [](const float* p, long ld, long stride) {
-        return ((uintptr_t)p % 16 == 0) && ld % 4 == 0 && stride % 4 == 0;
-    };
-    const int vec_a = aligned(g.A, TA ? g.M : g.K, g.batch > 1 ? g.sa : 0);
-    const int vec_b = aligned(g.B, TB ? g.K : g.N, g.batch > 1 ? g.sb : 0);
-    hipLaunchKernelGGL((gemm_mfma_fast_kernel<TA, TB, FUSED, WR, TRAP>), grid, dim3(256), 0, stream, g.A, g.B, g.C,
-                       g.M, g.N, g.K, g.alpha, g.beta, g.iters, g.sa, g.sb, g.sc, g.ep, vec_a, vec_b, g.k_causal,
-                       g.row0);
     return hipGetLastError();
 }
 
@@ -691,37 +422,12 @@ long device_cus() {
     return v;
 }
 
-// Register tile: 8x8 per lane (128x128 block) for FAST (16x8 when that fills
-// the CUs better), 4x4 (64x64) for the
-// CORDIC and SHIFTADD MACs, stepping down while the launch would have fewer
-// than kMinTiles blocks; the triangular and paired-row schedules keep the
-// 64x64 tile they are written for.  The tile never changes a result: each
-// output is one accumulator over k in order.
+// Register tile: 4x4 per lane (64x64 block), stepping down to 2x2 (32x32)
+// while the launch would have too few blocks; the triangular and paired-row
+// schedules keep the 64x64 tile they are written for.  The tile never
+// changes a result: each output is one accumulator over k in order.
 template <int MODE, int NITER, bool TA, bool TB, bool FUSED, int SCHED = 0>
 static hipError_t launch_tiles(const GemmArgs& g, hipStream_t s) {
-    constexpr int kBig = (MODE == kModeFast) ? 8 : 4;
-    if constexpr (MODE == kModeFast && SCHED != 0) {
-        // Causal attention products on the matrix cores under the rule of
-        // the plain schedule below: the scores (1: square, row0 = 0; 3: a
-        // chunk of query rows) over the tiles on or below the diagonal,
-        // P V (2) as a plain launch whose row tiles stop at their causal
-        // K limit (pairing row tiles for balance is not needed at MFMA
-        // block counts).
-        const long cus = device_cus();
-        if (g.K >= kMfMinK) {
-            if constexpr (SCHED == 2) {
-                const long t = ((g.M + 127) / 128) * ((g.N + kMfBN - 1) / kMfBN) * (long)g.batch;
-                if (4 * t >= cus && (double)g.M * g.N * g.batch >= 0.5 * (double)t * 128.0 * kMfBN)
-                    return launch_mfma_fast<TA, TB, FUSED, 64>(g, s);
-            } else {
-                GemmArgs h = g;
-                if constexpr (SCHED == 1) h.row0 = 0;
-                long t = 0;
-                for (int r = 0; r < (int)((g.M + 127) / 128); r++) t += trap_cols(h.row0, r, 128, kMfBN, g.N);
-                if (g.M >= 64 && 4 * t * (long)g.batch >= cus) return launch_mfma_fast<TA, TB, FUSED, 64, true>(h, s);
-            }
-        }
-    }
     if constexpr (SCHED == 2) {
         // Causal P V, row tiles p and nt-1-p per workgroup (equal K sums): on
         // 64x64 tiles while that gives 2 workgroups per CU, else on 32x32
@@ -738,63 +444,19 @@ static hipError_t launch_tiles(const GemmArgs& g, hipStream_t s) {
     } else if constexpr (SCHED == 1) {
         return launch_cfg<MODE, NITER, TA, TB, FUSED, SCHED, 4>(g, s);
     } else {
-        auto tiles = [&](long bm, long bn) {
-            if constexpr (SCHED == 3) {      // the causal trapezoid's tiles only
-                long t = 0;
-                for (long r = 0; r < (g.M + bm - 1) / bm; r++) t += trap_cols(g.row0, (int)r, (int)bm, (int)bn, g.N);
-                return t * (long)g.batch;
-            }
-            return ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * (long)g.batch;
-        };
-        if constexpr (MODE == kModeFast && SCHED == 0) {
-            // The matrix cores, once there are cus / 4 blocks of 128 x 128,
-            // at least half of their outputs real and K >= 128.  An MFMA
-            // block costs K x 128 cycles of its SIMDs whatever its fill:
-            // measured against the VALU tiles (bit-identical), 64 blocks
-            // (1024^2 x 1024, 32 x 256 x 128 x 2048) are 5-8% faster, 128
-            // blocks (the attention P V chunks 32 x 512 x 128 x K, 512 x
-            // 4096 x 4096 NT) 65-84% faster, while 32 blocks of a short M
-            // (128 x 4096 x 4096) are 3x slower, and K = 37 (2050 x 2049)
-            // 20 us against 16.
-            // Wave tiles of 128 x 64 (4 accumulator chains per wave, 2
-            // blocks of 256 x 128 per CU) beat 64 x 64 (2 chains, 3 blocks
-            // of 128 x 128 per CU) by 5-7% when they fill a round of the CUs
-            // and their rounds of resident blocks are fuller (4096^3,
-            // 8192^3), and lose up to 19% when a partial last round remains
-            // (2048 x 12288: 1.5 rounds against 2), so the fuller one is
-            // taken, 64 x 64 on a tie.  The fused epilogue keeps 64 x 64
-            // (with 4 chains it no longer fits the registers).
-            const long cus = device_cus();
-            auto fill = [&](long t, long per_cu) {
-                const long slots = per_cu * cus, rounds = (t + slots - 1) / slots;
-                return (double)t / (double)(rounds * slots);
-            };
-            const long t128 = tiles(128, kMfBN), t256 = tiles(256, kMfBN);
-            const double used = (double)g.M * (double)g.N * (double)g.batch / ((double)t128 * kMfBN * 128.0);
-            if (g.K >= kMfMinK && 4 * t128 >= cus && used >= 0.5) {
-                if constexpr (!FUSED) {
-                    if (t256 >= cus && fill(t256, 2) > fill(t128, 3)) return launch_mfma_fast<TA, TB, FUSED, 128>(g, s);
-                }
-                return launch_mfma_fast<TA, TB, FUSED, 64>(g, s);
-            }
-            // 16x8 per lane (256x128 blocks, 2 per CU at its register count)
-            // reads 25% fewer LDS bytes per FMA than 8x8 (128x128, 3 per
-            // CU); it is taken when it fills its rounds of resident blocks
-            // at least as completely as 8x8 does
-            if (t256 >= 2 * cus && fill(t256, 2) >= fill(t128, 3))
-                return launch_cfg<MODE, NITER, TA, TB, FUSED, 0, 16, 8>(g, s);
+        long tiles = 0;                      // of 64x64
+        if constexpr (SCHED == 3) {          // the causal trapezoid's only
+            for (long r = 0; r < (g.M + 63) / 64; r++) tiles += trap_cols(g.row0, (int)r, 64, 64, g.N);
+        } else {
+            tiles = (long)((g.M + 63) / 64) * ((g.N + 63) / 64);
         }
-        if (tiles(16 * kBig, 16 * kBig) >= kMinTiles) return launch_cfg<MODE, NITER, TA, TB, FUSED, SCHED, kBig>(g, s);
-        if constexpr (kBig == 4) {
-            // CORDIC / SHIFTADD: two 64x64 blocks per CU (2 waves per SIMD,
-            // 16 MAC chains each) still beat 32x32 blocks (measured, same
-            // bits: 512-1023 blocks 5-6% faster, e.g. the attention core's
-            // P V chunks 32 x 512 x 128 x K; at one block per CU 43% slower)
-            if (tiles(64, 64) >= 2 * device_cus()) return launch_cfg<MODE, NITER, TA, TB, FUSED, SCHED, 4>(g, s);
-        }
-        if constexpr (kBig == 8) {
-            if (tiles(64, 64) >= kMinTiles) return launch_cfg<MODE, NITER, TA, TB, FUSED, SCHED, 4>(g, s);
-        }
+        tiles *= g.batch;
+        // two 64x64 blocks per CU (2 waves per SIMD, 16 MAC chains each)
+        // still beat 32x32 blocks (measured, same bits: 512-1023 blocks 5-6%
+        // faster, e.g. the attention core's P V chunks 32 x 512 x 128 x K; at
+        // one block per CU 43% slower)
+        if (tiles >= 2 * device_cus())
+            return launch_cfg<MODE, NITER, TA, TB, FUSED, SCHED, 4>(g, s);
         return launch_cfg<MODE, NITER, TA, TB, FUSED, SCHED, 2>(g, s);
     }
 }
@@ -823,7 +485,12 @@ static hipError_t dispatch(int ta, int tb, int mode, const GemmArgs& g, hipStrea
                            g.ep, g.fused, tb != 0, g.k_causal, g.exact_specials, g.row0};
         return gemm_skinny_launch(k, mode, s);
     }
-    if (mode == kModeFast) return launch_layout<kModeFast, 0>(ta, tb, g, s);
+    if (mode == kModeFast) {
+        // the matrix cores; what they cannot read (fewer than 4 k, or 4 rows
+        // of an operand whose rows are contiguous) on the VALU tiles
+        if (g.K >= 4 && (!ta || g.M >= 4) && (tb || g.N >= 4)) return gemm_fast_launch(ta, tb, g, s);
+        return launch_layout<kModeFast, 0>(ta, tb, g, s);
+    }
     if (mode == kModeShiftAdd) return launch_layout<kModeShiftAdd, 0>(ta, tb, g, s);
     switch (g.iters) {
         case 8: return launch_layout<kModeCordic, 8>(ta, tb, g, s);
@@ -838,13 +505,13 @@ hipError_t gemm_launch(int ta, int tb, const float* A, const float* B, float* C,
                        hipStream_t s, int batch, long sa, long sb, long sc, int sched,
                        const int* k_causal, bool exact_specials, int row0) {
     const GemmArgs g{A, B, C, M, N, K, alpha, beta, clamp_iters(iters), batch, sa, sb, sc,
-                     GemmEpilogue(), false, sched, k_causal, exact_specials ? 1 : 0, row0};
+                     GemmEpilogue(), false, sched, k_causal, exact_specials ? 1 : 0, row0, 1};
     return dispatch(ta, tb, mode, g, s);
 }
 
 hipError_t gemm_fused_launch(const float* A, const float* W, float* C, int M, int N, int K,
                              const GemmEpilogue& ep, int iters, int mode, hipStream_t s) {
-    const GemmArgs g{A, W, C, M, N, K, 1.0f, 0.0f, clamp_iters(iters), 1, 0, 0, 0, ep, true, 0, nullptr, 1, 0};
+    const GemmArgs g{A, W, C, M, N, K, 1.0f, 0.0f, clamp_iters(iters), 1, 0, 0, 0, ep, true, 0, nullptr, 1, 0, 0};
     return dispatch(0, 1, mode, g, s);
 }
 

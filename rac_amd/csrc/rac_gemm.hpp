@@ -1,0 +1,44 @@
+// rac_gemm.hpp — what the GEMM kernel files share: a launch's arguments and
+// the causal score trapezoid.
+#pragma once
+#include <hip/hip_runtime.h>
+#include "rac_internal.hpp"
+
+namespace rac {
+
+struct GemmArgs {
+    const float* A;
+    const float* B;
+    float* C;
+    int M, N, K;
+    float alpha, beta;
+    int iters;
+    int batch;
+    long sa, sb, sc;
+    GemmEpilogue ep;
+    bool fused;
+    int sched;
+    const int* k_causal;
+    int exact_specials;
+    int row0;
+    // with k_causal: 1, row tile m sums k only up to its last query position
+    // row0 + m*BM + BM - 1 (P V); 2, only from k = m*BM - row0 on (P^T dO: row
+    // s of P^T is 0 before query position s, k = 0 being position row0)
+    int k_side;
+};
+
+// Column tiles of row tile r in a causal score trapezoid (query rows
+// row0 + r*BM .. row0 + r*BM + BM - 1, keys 0 .. N-1): those holding a key
+// position not past the row tile's last query position.
+__host__ __device__ __forceinline__ int trap_cols(int row0, int r, int BM, int BN, int N) {
+    const long last = (long)row0 + (long)(r + 1) * BM - 1;
+    const long c = last / BN + 1;
+    const long ntn = (N + BN - 1) / BN;
+    return (int)(c < ntn ? c : ntn);
+}
+
+// FAST mode on the matrix cores (rac_gemm_fast.hip): K >= 4 and, for an
+// operand stored with its rows contiguous (A of ta, B of !tb), at least 4 rows.
+hipError_t gemm_fast_launch(int ta, int tb, const GemmArgs& g, hipStream_t s);
+
+}  // namespace rac

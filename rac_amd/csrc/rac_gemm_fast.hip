@@ -1,0 +1,473 @@
+// rac_gemm_fast.hip — the FAST-mode GEMM (one fmaf per MAC, k in order) on
+// the FP32 matrix cores of gfx950.
+//
+// v_mfma_f32_16x16x4_f32 adds four products to each of its 16 x 16
+// accumulators, one after the other in k order, each with a single IEEE
+// rounding and denormals kept: the value of the chain
+//   fmaf(a3, b3, fmaf(a2, b2, fmaf(a1, b1, fmaf(a0, b0, acc))))
+// (checked on gfx950 against glibc's fmaf over 21 M random, subnormal,
+// special and cancelling operand sets: 0 differences; the reverse order and
+// separate roundings differ in millions).  Issued in k order it therefore
+// gives every output the FAST MAC's accumulation chain (rac_fma_iters,
+// rac_kernels.hip:204-219) bit for bit.  A single dependent chain issues at
+// the full rate (32.2 cycles per instruction, measured), so a wave needs
+// only one 16 x 16 tile to keep its matrix core busy, 8 cycles per k and 256
+// outputs, where the 32x32x1_2b form needs 2048 outputs for it.
+#include <hip/hip_runtime.h>
+#include <type_traits>
+#include "rac_act.hpp"
+#include "rac_gemm.hpp"
+
+namespace rac {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+// a float4 at any 4-byte boundary (global_load / store_dwordx4 need no more)
+typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ void store4(float* p, v4f v, int n) {
+    if (n >= 4) {
+        *reinterpret_cast<v4u*>(p) = v4u{v.x, v.y, v.z, v.w};
+        return;
+    }
+    if (n > 0) p[0] = v.x;
+    if (n > 1) p[1] = v.y;
+    if (n > 2) p[2] = v.z;
+}
+
+// One operand's K-tile (KT k x ROWS rows) of a workgroup: global ->
+// registers -> LDS -> matrix-core operands.  Lane l of the instruction
+// holds element (row l % 16, k = 4 t + l / 16) of step t.
+//
+// KC (k contiguous in memory: A, or B^T of the NT layout): LDS rows of KT +
+// 4 floats, each 16-k group stored with k = 4 t + q at 4 q + t, so one
+// ds_read_b128 gives a lane its elements of four consecutive steps; both the
+// reads (8 lanes on 8 rows, 4 KT + 16 bytes apart) and the scattering writes
+// touch every bank once.  Otherwise LDS rows are k rows of ROWS + pad floats
+// (= 16 mod 32: the two k of a half wave on opposite banks), read a step at
+// a time.
+template <bool KC, int ROWS, int KT, int NL>
+struct FastTile {
+    static constexpr int kStride = KC ? KT + 4 : ROWS + ((48 - ROWS % 32) % 32);
+    static constexpr int kFloats = (KC ? ROWS : KT) * kStride;
+    static constexpr int kVecs = ROWS * KT / 4;                     // float4 of the tile
+    static constexpr int kVPT = (kVecs + NL - 1) / NL;              // per lane
+    static constexpr int kPer = KC ? KT / 4 : ROWS / 4;             // float4 per LDS row
+
+    // this lane's global addresses at the next K-tile to load; rows past the
+    // matrix read rows inside it (their outputs are never stored)
+    const float* p[kVPT];
+    long step;                                                      // one K-tile further
+    int shift;                                                      // !KC: see fix_rows()
+
+    __device__ __forceinline__ static bool on(int i) { return kVecs % NL == 0 || (int)threadIdx.x + i * NL < kVecs; }
+    __device__ __forceinline__ void init(const float* P, long ld, long rows, long r0, long k0) {
+        const int tid = threadIdx.x;
+        step = KC ? KT : (long)KT * ld;
+        shift = 0;
+        long r = 0;
+        if constexpr (!KC) {
+            // four rows inside the matrix (it has more than 16)
+            const long want = r0 + (tid % kPer) * 4;
+            r = min(want, rows - 4);
+            shift = (int)min(want - r, 3L);
+        }
+#pragma unroll
+        for (int i = 0; i < kVPT; i++) {
+            const int idx = tid + i * NL;
+            if constexpr (KC) p[i] = P + min(r0 + idx / kPer, rows - 1) * ld + k0 + (idx % kPer) * 4;
+            else p[i] = P + (k0 + idx / kPer) * ld + r;
+        }
+    }
+    // The K-tile at hand has only `kn` (1 .. KT - 1) of its k, and the matrix
+    // at least 4: addresses move back inside K; fix_k() then puts the
+    // elements where they belong and zeroes those past K (a zero product
+    // leaves an accumulator as it is: it starts at +0 and never becomes -0).
+    __device__ __forceinline__ void retreat(int kn, long ld) {
+#pragma unroll
+        for (int i = 0; i < kVPT; i++) {
+            const int idx = threadIdx.x + i * NL;
+            if constexpr (KC) p[i] -= max(0, (idx % kPer) * 4 + 4 - kn);
+            else p[i] -= max(0, idx / kPer + 1 - kn) * ld;
+        }
+    }
+    __device__ __forceinline__ void load(v4f (&v)[kVPT], int i) const {
+        if (on(i)) {
+            const v4u t = *reinterpret_cast<const v4u*>(p[i]);
+            v[i] = v4f{t.x, t.y, t.z, t.w};
+        }
+    }
+    __device__ __forceinline__ void advance(long by) {
+#pragma unroll
+        for (int i = 0; i < kVPT; i++) p[i] += by;
+    }
+    __device__ __forceinline__ static v4f shifted(v4f v, int sh) {
+        if (sh & 1) v = v4f{v.y, v.z, v.w, 0.0f};
+        if (sh & 2) v = v4f{v.z, v.w, 0.0f, 0.0f};
+        if (sh & 4) v = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        return v;
+    }
+    __device__ __forceinline__ static void fix_k(v4f (&v)[kVPT], int kn) {
+#pragma unroll
+        for (int i = 0; i < kVPT; i++) {
+            const int idx = threadIdx.x + i * NL;
+            if constexpr (KC) v[i] = shifted(v[i], min(4, max(0, (idx % kPer) * 4 + 4 - kn)));
+            else v[i] = shifted(v[i], idx / kPer >= kn ? 4 : 0);
+        }
+    }
+    // !KC, tiles past the last row: lanes that moved back to stay inside
+    // the matrix put their rows where they belong
+    __device__ __forceinline__ void fix_rows(v4f (&v)[kVPT]) const {
+#pragma unroll
+        for (int i = 0; i < kVPT; i++) v[i] = shifted(v[i], shift);
+    }
+    __device__ __forceinline__ static void store(float* S, const v4f (&v)[kVPT], int i) {
+        const int idx = threadIdx.x + i * NL;
+        if (!on(i)) return;
+        if constexpr (KC) {
+            const int c = idx % kPer;
+            float* s = S + (idx / kPer) * kStride + (c / 4) * 16 + c % 4;
+            s[0] = v[i].x;
+            s[4] = v[i].y;
+            s[8] = v[i].z;
+            s[12] = v[i].w;
+        } else {
+            *reinterpret_cast<v4f*>(S + (idx / kPer) * kStride + (idx % kPer) * 4) = v[i];
+        }
+    }
+    // the lane's elements of steps 4 g .. 4 g + 3 (k = 16 g .. 16 g + 15)
+    // for the 16 rows at `row`
+    __device__ __forceinline__ static v4f frag(const float* S, int row, int g) {
+        const int l = threadIdx.x & 63;
+        if constexpr (KC) {
+            return *reinterpret_cast<const v4f*>(S + (row + l % 16) * kStride + 16 * g + 4 * (l / 16));
+        } else {
+            const float* s = S + (16 * g + l / 16) * kStride + row + l % 16;
+            return v4f{s[0], s[4 * kStride], s[8 * kStride], s[12 * kStride]};
+        }
+    }
+};
+
+struct FastGeom {
+    int M, N, K;
+    long sa, sb, sc;
+    float alpha, beta;
+    int iters;
+    GemmEpilogue ep;
+    const int* k_causal;
+    int k_side;           // 0: every k; 1, 2: the causal limits of GemmArgs, when *k_causal holds 1
+    int row0;
+    int tiles, tiles_m;   // output tiles of one batch item, rows of them
+    int batch;
+    long total;           // tiles * batch
+};
+
+// Output tile BM x BN, WR x WC waves, K-tiles of KT in two LDS buffers, PD
+// K-tiles in flight in registers.  Per K-tile and buffer one barrier: while
+// the MACs of one run, the next is written into the other buffer and the
+// one PD further is requested.  SPREAD 0 does that ahead of the MACs, 1
+// between them, 2 between them with the order held by scheduling barriers
+// (a lone wave per SIMD issues them in the shadow of its matrix
+// instructions: 32x4096x4096 on 32x32 tiles 34.7 -> 24.9 us).
+template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD>
+__global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const float* __restrict__ A,
+                                                                 const float* __restrict__ B, float* __restrict__ C,
+                                                                 FastGeom g)
+{
+    constexpr int NL = 64 * WR * WC;
+    using TAt = FastTile<!TA, BM, KT, NL>;
+    using TBt = FastTile<TB, BN, KT, NL>;
+    constexpr int TM = BM / WR, TN = BN / WC, MT = TM / 16, NT = TN / 16;
+    __shared__ __attribute__((aligned(16))) float sA[2][TAt::kFloats];
+    __shared__ __attribute__((aligned(16))) float sB[2][TBt::kFloats];
+
+    const long L = blockIdx.x + (long)blockIdx.y * gridDim.x;
+    if (L >= g.total) return;
+    const int tiles_n = TRAP ? 1 : g.tiles / g.tiles_m;
+    int z, tm, tn;
+    if (g.k_side) {
+        // tiles of unequal K: the longest first, one of every batch item in
+        // turn (an item's tiles stay on one XCD where 8 divides the batch)
+        z = (int)(L % g.batch);
+        const int t = (int)(L / g.batch);
+        tm = t / tiles_n;
+        tn = t - tm * tiles_n;
+        if (g.k_side == 1) tm = g.tiles_m - 1 - tm;
+    } else {
+        // The dispatcher puts workgroup L on XCD L % 8: each XCD takes one
+        // contiguous range of tiles, numbered in groups of 8 row tiles
+        // down, then across, so tiles that share operand panels share an L2.
+        const long q = g.total / 8, r = g.total % 8, x = L % 8;
+        const long id = x * q + min(x, r) + L / 8;
+        z = (int)(id / g.tiles);
+        int t = (int)(id - (long)z * g.tiles);
+        if constexpr (TRAP) {
+            tm = 0;
+            for (;;) {
+                const int c = trap_cols(g.row0, tm, BM, BN, g.N);
+                if (t < c) break;
+                t -= c;
+                tm++;
+            }
+            tn = t;
+        } else {
+            const int grp = t / (8 * tiles_n), first = grp * 8, rows = min(8, g.tiles_m - first);
+            t -= grp * 8 * tiles_n;
+            tm = first + t % rows;
+            tn = t / rows;
+        }
+    }
+    const int M = g.M, N = g.N;
+    const long m0 = (long)tm * BM, n0 = (long)tn * BN;
+    A += z * g.sa;
+    B += z * g.sb;
+    C += z * g.sc;
+    int kbeg = 0, kend = g.K;
+    if (g.k_side && *g.k_causal == 1) {
+        if (g.k_side == 1) kend = (int)min((long)g.K, (long)g.row0 + m0 + BM);
+        else kbeg = (int)min((long)g.K - 4, max(0L, m0 - g.row0));
+    }
+
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = (wave / WC) * TM, wn = (wave % WC) * TN;
+    v4f acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+    TAt ta;
+    TBt tb;
+    const long lda = TA ? M : g.K, ldb = TB ? g.K : N;
+    ta.init(A, lda, M, m0, kbeg);
+    tb.init(B, ldb, N, n0, kbeg);
+    constexpr int VA = TAt::kVPT, VB = TBt::kVPT;
+    v4f va[PD][VA], vb[PD][VB];
+    const int kn = kend - kbeg, nfull = kn / KT, tail = kn - nfull * KT, nst = nfull + (tail ? 1 : 0);
+    const bool edge_a = TA && m0 + BM > M, edge_b = !TB && n0 + BN > N;
+    // before K-tile s is loaded / after (tiles past the last reload it: the
+    // loads stay unconditional, so the waits stay exact)
+    auto before = [&](int s) {
+        if (tail && s == nfull) {
+            ta.retreat(tail, lda);
+            tb.retreat(tail, ldb);
+        }
+    };
+    auto after = [&](int s) {
+        const bool more = s + 1 < nst;
+        ta.advance(more ? ta.step : 0);
+        tb.advance(more ? tb.step : 0);
+    };
+    auto fix = [&](int s, int slot) {
+        if (tail && s == nfull) {
+            TAt::fix_k(va[slot], tail);
+            TBt::fix_k(vb[slot], tail);
+        }
+        if constexpr (TA) if (edge_a) ta.fix_rows(va[slot]);
+        if constexpr (!TB) if (edge_b) tb.fix_rows(vb[slot]);
+    };
+    auto frags = [&](int buf, int q, v4f (&fa)[MT], v4f (&fb)[NT]) {
+#pragma unroll
+        for (int i = 0; i < MT; i++) fa[i] = TAt::frag(sA[buf], wm + 16 * i, q);
+#pragma unroll
+        for (int j = 0; j < NT; j++) fb[j] = TBt::frag(sB[buf], wn + 16 * j, q);
+    };
+    // item x of a K-tile's staging: registers -> the other LDS buffer, and
+    // the slot's next load
+    auto stage = [&](int buf, int slot, int x, bool ld) {
+        if (x < VA) {
+            TAt::store(sA[buf], va[slot], x);
+            if (ld) ta.load(va[slot], x);
+        } else if (x < VA + VB) {
+            TBt::store(sB[buf], vb[slot], x - VA);
+            if (ld) tb.load(vb[slot], x - VA);
+        }
+    };
+    // the MACs of the K-tile in LDS buffer `buf`; `staged`: with the
+    // next tile's staging, ahead of them (SPREAD 0) or spread over them
+    auto compute = [&](int buf, auto staged, int slot, bool ld) {
+        constexpr int Q = KT / 16, X = VA + VB;
+        v4f fa[2][MT], fb[2][NT];
+        if constexpr (SPREAD == 0 && decltype(staged)::value) {
+#pragma unroll
+            for (int x = 0; x < X; x++) stage(buf ^ 1, slot, x, ld);
+        }
+        frags(buf, 0, fa[0], fb[0]);
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            if (q + 1 < Q) frags(buf, q + 1, fa[(q + 1) & 1], fb[(q + 1) & 1]);
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[q & 1][j][t], fa[q & 1][i][t], acc[i][j], 0, 0, 0);
+                if constexpr (SPREAD > 0 && decltype(staged)::value) {
+                    const int c = 4 * q + t;
+#pragma unroll
+                    for (int x = c * X / (4 * Q); x < (c + 1) * X / (4 * Q); x++) stage(buf ^ 1, slot, x, ld);
+                }
+                if constexpr (SPREAD == 2) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < PD; s++) {
+        before(s);
+#pragma unroll
+        for (int x = 0; x < VA; x++) ta.load(va[s], x);
+#pragma unroll
+        for (int x = 0; x < VB; x++) tb.load(vb[s], x);
+        after(s);
+    }
+    fix(0, 0);
+    before(PD);
+#pragma unroll
+    for (int x = 0; x < VA + VB; x++) stage(0, 0, x, true);
+    after(PD);
+    __syncthreads();
+    int s = 0;
+    for (; s + 2 < nst; s += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            fix(s + u + 1, (u + 1) % PD);
+            before(s + u + 1 + PD);
+            compute(u, std::true_type(), (u + 1) % PD, true);
+            after(s + u + 1 + PD);
+            __syncthreads();
+        }
+    }
+    if (s + 1 < nst) {
+        fix(s + 1, 1 % PD);
+        compute(0, std::true_type(), 1 % PD, false);
+        __syncthreads();
+        compute(1, std::false_type(), 0, false);
+    } else {
+        compute(0, std::false_type(), 0, false);
+    }
+
+    // the operands are passed B first, so a lane holds four consecutive
+    // columns of one row: n = 4 (lane / 16) + r, m = lane % 16 of each tile
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        const long gm = m0 + wm + 16 * i + lane % 16;
+        if (gm >= M) continue;
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            const long gn = n0 + wn + 16 * j + 4 * (lane / 16);
+            const int left = (int)min(4L, (long)N - gn);
+            if (left <= 0) continue;
+            float* cp = C + gm * N + gn;
+            v4f v;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                // rac_kernels.hip:267-272
+                v[r] = g.alpha * acc[i][j][r];
+                if (g.beta != 0.0f && r < left) v[r] = __builtin_fmaf(g.alpha, acc[i][j][r], g.beta * cp[r]);
+            }
+            if constexpr (FUSED) {
+                // rac_torch.cu:770-775
+                if (g.ep.bias) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (r < left) v[r] = v[r] + g.ep.bias[gn + r];
+                }
+                if (g.ep.pre) store4(g.ep.pre + gm * N + gn, v, left);
+                if (g.ep.act != kActNone) {
+                    // one copy of the activation per tile: v rotates
+#pragma unroll 1
+                    for (int r = 0; r < 4; r++) {
+                        const float x = act_rt(v.x, g.ep.act, g.iters, g.ep.khinv);
+                        v = v4f{v.y, v.z, v.w, x};
+                    }
+                }
+            }
+            store4(cp, v, left);
+        }
+    }
+}
+
+template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD>
+static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
+    FastGeom g{a.M, a.N, a.K, a.sa, a.sb, a.sc, a.alpha, a.beta, a.iters, a.ep, a.k_causal, a.k_causal ? a.k_side : 0,
+               a.row0, 0, (a.M + BM - 1) / BM, a.batch, 0};
+    if constexpr (TRAP) {
+        for (int r = 0; r < g.tiles_m; r++) g.tiles += trap_cols(g.row0, r, BM, BN, g.N);
+    } else {
+        g.tiles = g.tiles_m * ((g.N + BN - 1) / BN);
+    }
+    g.total = (long)g.tiles * g.batch;
+    // a grid dimension holds fewer than 2^32 lanes
+    const long gx = g.total < (1L << 22) ? g.total : (1L << 22);
+    hipLaunchKernelGGL((gemm_fast_kernel<TA, TB, FUSED, TRAP, BM, BN, WR, WC, KT, PD, SPREAD>),
+                       dim3((unsigned)gx, (unsigned)((g.total + gx - 1) / gx)), dim3(64 * WR * WC), 0, s, a.A, a.B,
+                       a.C, g);
+    return hipGetLastError();
+}
+
+// The output tile: the one with the least matrix-core time on the fullest
+// CU.  A CU works through BM x BN x K MACs of a tile at 128 per cycle times
+// the share `eff` of that rate which the tile sustains, and the fullest CU
+// has ceil(tiles / CUs) of them: large tiles reuse operands best but leave
+// CUs idle in the last round.  eff and the shapes inside a tile size are
+// measured (K 1000-11008, all layouts): e.g. 2048 x 11008 x 4096 NT 1.39 ms
+// on 64x128 (128x128: 1.47, 64x64: 1.46), 500 x 2048 x 5632 NT 99 us on
+// 64x64 (32x64: 101, 32x32: 105), 128 x 11008 x 4096 NT 107 us on 32x64
+// (32x32: 113, 64x64: 124), 1500^3 NT 68 us on 32x32 (64x64: 80).  With a
+// causal limit the tiles' work is unequal and dispatched longest first: the
+// CUs share it evenly but for about one longest tile.
+template <bool TA, bool TB, bool FUSED, bool TRAP>
+static hipError_t fast_tile(const GemmArgs& a, hipStream_t s) {
+    struct Shape { int bm, bn; double eff; };
+    constexpr Shape shapes[5] = {{128, 128, 0.93}, {64, 128, 0.91}, {64, 64, 0.83}, {32, 64, 0.81}, {32, 32, 0.76}};
+    const long cus = device_cus();
+    int best = 0;
+    double best_cost = 0.0;
+    for (int i = 0; i < 5; i++) {
+        const long bm = shapes[i].bm, bn = shapes[i].bn, tm = (a.M + bm - 1) / bm;
+        double cost;
+        if (TRAP) {
+            long t = 0;
+            for (long r = 0; r < tm; r++) t += trap_cols(a.row0, (int)r, (int)bm, (int)bn, a.N);
+            t *= a.batch;
+            cost = (double)((t + cus - 1) / cus) * bm * bn / shapes[i].eff;
+        } else if (a.k_causal && a.k_side) {
+            // about half of the k of all tiles, in units of K
+            const double per_cu = 0.5 * tm * ((a.N + bn - 1) / bn) * a.batch / cus;
+            cost = (per_cu + 1.0) * bm * bn / shapes[i].eff;
+        } else {
+            const long t = tm * ((a.N + bn - 1) / bn) * a.batch;
+            cost = (double)((t + cus - 1) / cus) * bm * bn / shapes[i].eff;
+        }
+        if (i == 0 || cost < best_cost) {
+            best = i;
+            best_cost = cost;
+        }
+    }
+    constexpr bool KC2 = !TA && TB, KC0 = TA && !TB;      // both / neither operand k-contiguous
+    switch (best) {
+    case 0:
+        if constexpr (KC2) return fast_launch<TA, TB, FUSED, TRAP, 128, 128, 2, 4, 16, 1, 0>(a, s);
+        else if constexpr (KC0) return fast_launch<TA, TB, FUSED, TRAP, 128, 128, 2, 4, 32, 1, 0>(a, s);
+        else return fast_launch<TA, TB, FUSED, TRAP, 128, 128, 2, 2, 16, 1, 0>(a, s);
+    case 1:
+        if constexpr (KC0) return fast_launch<TA, TB, FUSED, TRAP, 64, 64, 2, 2, 32, 1, 1>(a, s);
+        else return fast_launch<TA, TB, FUSED, TRAP, 64, 128, 2, 2, 16, 1, 1>(a, s);
+    case 2:
+        if constexpr (KC0) return fast_launch<TA, TB, FUSED, TRAP, 64, 64, 2, 2, 32, 1, 1>(a, s);
+        else return fast_launch<TA, TB, FUSED, TRAP, 64, 64, 2, 4, 64, 2, 2>(a, s);
+    case 3: return fast_launch<TA, TB, FUSED, TRAP, 32, 64, 2, 2, 64, 2, 2>(a, s);
+    default: return fast_launch<TA, TB, FUSED, TRAP, 32, 32, 2, 2, 64, 2, 2>(a, s);
+    }
+}
+
+hipError_t gemm_fast_launch(int ta, int tb, const GemmArgs& g, hipStream_t s) {
+    if (g.fused) return fast_tile<false, true, true, false>(g, s);                      // NT only
+    if (g.sched == 1 || g.sched == 3) return fast_tile<false, true, false, true>(g, s);  // NT only
+    if (!ta && !tb) return fast_tile<false, false, false, false>(g, s);
+    if (!ta && tb) return fast_tile<false, true, false, false>(g, s);
+    if (ta && !tb) return fast_tile<true, false, false, false>(g, s);
+    return fast_tile<true, true, false, false>(g, s);
+}
+
+}  // namespace rac
