@@ -478,18 +478,20 @@ static hipError_t launch_layout(int ta, int tb, const GemmArgs& g, hipStream_t s
 }
 
 static hipError_t dispatch(int ta, int tb, int mode, const GemmArgs& g, hipStream_t s) {
+    if (mode == kModeFast) {
+        // the matrix cores; the VALU tiles for fewer than 4 k, which the
+        // 16-byte loads cannot read, and where both operands hold 2 or 3 rows
+        // side by side
+        const bool thin_a = ta && g.M > 1 && g.M < 4, thin_b = !tb && g.N > 1 && g.N < 4;
+        if (g.K >= 4 && !(thin_a && thin_b)) return gemm_fast_launch(ta, tb, g, s);
+        return launch_layout<kModeFast, 0>(ta, tb, g, s);
+    }
     // few rows or columns (schedule 2, the causal P V, is then the plain
     // product with its causal K limit, which those kernels apply)
     if ((g.sched == 0 || g.sched == 2) && !ta && (g.M <= kSkinnyMaxRows || g.N <= kSkinnyMaxRows)) {
         const SkinnyArgs k{g.A, g.B, g.C, g.M, g.N, g.K, g.alpha, g.beta, g.iters, g.batch, g.sa, g.sb, g.sc,
                            g.ep, g.fused, tb != 0, g.k_causal, g.exact_specials, g.row0};
         return gemm_skinny_launch(k, mode, s);
-    }
-    if (mode == kModeFast) {
-        // the matrix cores; what they cannot read (fewer than 4 k, or 4 rows
-        // of an operand whose rows are contiguous) on the VALU tiles
-        if (g.K >= 4 && (!ta || g.M >= 4) && (tb || g.N >= 4)) return gemm_fast_launch(ta, tb, g, s);
-        return launch_layout<kModeFast, 0>(ta, tb, g, s);
     }
     if (mode == kModeShiftAdd) return launch_layout<kModeShiftAdd, 0>(ta, tb, g, s);
     switch (g.iters) {

@@ -37,8 +37,8 @@ __host__ __device__ __forceinline__ int trap_cols(int row0, int r, int BM, int B
     return (int)(c < ntn ? c : ntn);
 }
 
-// FAST mode on the matrix cores (rac_gemm_fast.hip): K >= 4 and, for an
-// operand stored with its rows contiguous (A of ta, B of !tb), at least 4 rows.
+// FAST mode on the matrix cores (rac_gemm_fast.hip): K >= 4; at most one
+// operand stored with its rows side by side (A of ta, B of !tb) has 2 or 3.
 hipError_t gemm_fast_launch(int ta, int tb, const GemmArgs& g, hipStream_t s);
 
 }  // namespace rac

@@ -45,7 +45,7 @@ __device__ __forceinline__ void store4(float* p, v4f v, int n) {
 // touch every bank once.  Otherwise LDS rows are k rows of ROWS + pad floats
 // (= 16 mod 32: the two k of a half wave on opposite banks), read a step at
 // a time.
-template <bool KC, int ROWS, int KT, int NL>
+template <bool KC, int ROWS, int KT, int NL, bool THIN = false>
 struct FastTile {
     static constexpr int kStride = KC ? KT + 4 : ROWS + ((48 - ROWS % 32) % 32);
     static constexpr int kFloats = (KC ? ROWS : KT) * kStride;
@@ -66,10 +66,10 @@ struct FastTile {
         shift = 0;
         long r = 0;
         if constexpr (!KC) {
-            // four rows inside the matrix (it has more than 16)
+            // four rows inside the matrix (it has at least 4)
             const long want = r0 + (tid % kPer) * 4;
-            r = min(want, rows - 4);
-            shift = (int)min(want - r, 3L);
+            r = THIN ? 0 : min(want, rows - 4);
+            shift = THIN ? (int)rows - 1 : (int)min(want - r, 3L);      // THIN: the last row
         }
 #pragma unroll
         for (int i = 0; i < kVPT; i++) {
@@ -91,7 +91,9 @@ struct FastTile {
         }
     }
     __device__ __forceinline__ void load(v4f (&v)[kVPT], int i) const {
-        if (on(i)) {
+        if constexpr (THIN) {
+            if (on(i)) v[i] = v4f{p[i][0], p[i][min(1, shift)], p[i][min(2, shift)], 0.0f};
+        } else if (on(i)) {
             const v4u t = *reinterpret_cast<const v4u*>(p[i]);
             v[i] = v4f{t.x, t.y, t.z, t.w};
         }
@@ -118,7 +120,8 @@ struct FastTile {
     // the matrix put their rows where they belong
     __device__ __forceinline__ void fix_rows(v4f (&v)[kVPT]) const {
 #pragma unroll
-        for (int i = 0; i < kVPT; i++) v[i] = shifted(v[i], shift);
+        for (int i = 0; i < kVPT; i++)
+            if constexpr (!THIN) v[i] = shifted(v[i], shift);
     }
     __device__ __forceinline__ static void store(float* S, const v4f (&v)[kVPT], int i) {
         const int idx = threadIdx.x + i * NL;
@@ -161,6 +164,40 @@ struct FastGeom {
     long total;           // tiles * batch
 };
 
+// alpha / beta, bias and activation of outputs (gm, gn .. gn + 3)
+template <bool FUSED>
+__device__ __forceinline__ void fast_epilogue(float* __restrict__ C, int M, int N, long gm, long gn, v4f acc,
+                                              const FastGeom& g) {
+    const int left = (int)min(4L, (long)N - gn);
+    if (gm >= M || left <= 0) return;
+    float* cp = C + gm * N + gn;
+    v4f v;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        // rac_kernels.hip:267-272
+        v[r] = g.alpha * acc[r];
+        if (g.beta != 0.0f && r < left) v[r] = __builtin_fmaf(g.alpha, acc[r], g.beta * cp[r]);
+    }
+    if constexpr (FUSED) {
+        // rac_torch.cu:770-775
+        if (g.ep.bias) {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (r < left) v[r] = v[r] + g.ep.bias[gn + r];
+        }
+        if (g.ep.pre) store4(g.ep.pre + gm * N + gn, v, left);
+        if (g.ep.act != kActNone) {
+            // one copy of the activation per tile: v rotates
+#pragma unroll 1
+            for (int r = 0; r < 4; r++) {
+                const float x = act_rt(v.x, g.ep.act, g.iters, g.ep.khinv);
+                v = v4f{v.y, v.z, v.w, x};
+            }
+        }
+    }
+    store4(cp, v, left);
+}
+
 // Output tile BM x BN, WR x WC waves, K-tiles of KT in two LDS buffers, PD
 // K-tiles in flight in registers.  Per K-tile and buffer one barrier: while
 // the MACs of one run, the next is written into the other buffer and the
@@ -168,14 +205,14 @@ struct FastGeom {
 // between them, 2 between them with the order held by scheduling barriers
 // (a lone wave per SIMD issues them in the shadow of its matrix
 // instructions: 32x4096x4096 on 32x32 tiles 34.7 -> 24.9 us).
-template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD>
+template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD, bool THIN>
 __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const float* __restrict__ A,
                                                                  const float* __restrict__ B, float* __restrict__ C,
                                                                  FastGeom g)
 {
     constexpr int NL = 64 * WR * WC;
-    using TAt = FastTile<!TA, BM, KT, NL>;
-    using TBt = FastTile<TB, BN, KT, NL>;
+    using TAt = FastTile<!TA, BM, KT, NL, TA && THIN && BM == 16>;
+    using TBt = FastTile<TB, BN, KT, NL, !TB && THIN && BN == 16>;
     constexpr int TM = BM / WR, TN = BN / WC, MT = TM / 16, NT = TN / 16;
     __shared__ __attribute__((aligned(16))) float sA[2][TAt::kFloats];
     __shared__ __attribute__((aligned(16))) float sB[2][TBt::kFloats];
@@ -349,45 +386,14 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const float* __
     // the operands are passed B first, so a lane holds four consecutive
     // columns of one row: n = 4 (lane / 16) + r, m = lane % 16 of each tile
 #pragma unroll
-    for (int i = 0; i < MT; i++) {
-        const long gm = m0 + wm + 16 * i + lane % 16;
-        if (gm >= M) continue;
+    for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int j = 0; j < NT; j++) {
-            const long gn = n0 + wn + 16 * j + 4 * (lane / 16);
-            const int left = (int)min(4L, (long)N - gn);
-            if (left <= 0) continue;
-            float* cp = C + gm * N + gn;
-            v4f v;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                // rac_kernels.hip:267-272
-                v[r] = g.alpha * acc[i][j][r];
-                if (g.beta != 0.0f && r < left) v[r] = __builtin_fmaf(g.alpha, acc[i][j][r], g.beta * cp[r]);
-            }
-            if constexpr (FUSED) {
-                // rac_torch.cu:770-775
-                if (g.ep.bias) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (r < left) v[r] = v[r] + g.ep.bias[gn + r];
-                }
-                if (g.ep.pre) store4(g.ep.pre + gm * N + gn, v, left);
-                if (g.ep.act != kActNone) {
-                    // one copy of the activation per tile: v rotates
-#pragma unroll 1
-                    for (int r = 0; r < 4; r++) {
-                        const float x = act_rt(v.x, g.ep.act, g.iters, g.ep.khinv);
-                        v = v4f{v.y, v.z, v.w, x};
-                    }
-                }
-            }
-            store4(cp, v, left);
-        }
-    }
+        for (int j = 0; j < NT; j++)
+            fast_epilogue<FUSED>(C, M, N, m0 + wm + 16 * i + lane % 16, n0 + wn + 16 * j + 4 * (lane / 16), acc[i][j],
+                                 g);
 }
 
-template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD>
+template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD, bool THIN = false>
 static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
     FastGeom g{a.M, a.N, a.K, a.sa, a.sb, a.sc, a.alpha, a.beta, a.iters, a.ep, a.k_causal, a.k_causal ? a.k_side : 0,
                a.row0, 0, (a.M + BM - 1) / BM, a.batch, 0};
@@ -399,7 +405,7 @@ static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
     g.total = (long)g.tiles * g.batch;
     // a grid dimension holds fewer than 2^32 lanes
     const long gx = g.total < (1L << 22) ? g.total : (1L << 22);
-    hipLaunchKernelGGL((gemm_fast_kernel<TA, TB, FUSED, TRAP, BM, BN, WR, WC, KT, PD, SPREAD>),
+    hipLaunchKernelGGL((gemm_fast_kernel<TA, TB, FUSED, TRAP, BM, BN, WR, WC, KT, PD, SPREAD, THIN>),
                        dim3((unsigned)gx, (unsigned)((g.total + gx - 1) / gx)), dim3(64 * WR * WC), 0, s, a.A, a.B,
                        a.C, g);
     return hipGetLastError();
@@ -461,13 +467,52 @@ static hipError_t fast_tile(const GemmArgs& a, hipStream_t s) {
     }
 }
 
+// At most 16 rows (decode-time linears) or columns: one 16 x 16 block of
+// outputs per wave, which runs at the instruction's latency, K x 8 cycles
+// for any number of rows up to 16 (1 x 4096 x 4096: 23.4 us, of which 14.5
+// that chain).  Four waves side by side, one per SIMD, with the deeper
+// K-tile once a CU has more than one such block (1 x 32000 x 4096: 90.1
+// against 95.3 us; 1 x 11008 x 4096, 172 blocks: 31.5 against 27.8); pairs
+// of waves where those still fit one to a CU (4096 columns: 23.4 against
+// 26.9 us; 11008, 344 blocks: 39.6, a second pair shares the first's SIMDs).
+template <bool TA, bool TB, bool FUSED>
+static hipError_t fast_few(const GemmArgs& a, hipStream_t s) {
+    const long cus = device_cus();
+    const bool rows = a.M <= 16;
+    const long n = rows ? a.N : a.M, b4 = (n + 63) / 64 * a.batch, b2 = (n + 31) / 32 * a.batch;
+    // fewer than 4 rows stored side by side (1 is a vector, read as k-contiguous)
+    if constexpr (TA) {
+        if (a.M < 4) return fast_launch<TA, TB, FUSED, false, 16, 64, 1, 4, 64, 2, 2, true>(a, s);
+    }
+    if constexpr (!TB) {
+        if (a.N < 4) return fast_launch<TA, TB, FUSED, false, 64, 16, 4, 1, 64, 2, 2, true>(a, s);
+    }
+    if (rows) {
+        if (b2 <= cus) return fast_launch<TA, TB, FUSED, false, 16, 32, 1, 2, 128, 1, 2>(a, s);
+        if (b4 <= cus) return fast_launch<TA, TB, FUSED, false, 16, 64, 1, 4, 64, 2, 2>(a, s);
+        return fast_launch<TA, TB, FUSED, false, 16, 64, 1, 4, 128, 1, 2>(a, s);
+    }
+    if (b2 <= cus) return fast_launch<TA, TB, FUSED, false, 32, 16, 2, 1, 128, 1, 2>(a, s);
+    if (b4 <= cus) return fast_launch<TA, TB, FUSED, false, 64, 16, 4, 1, 64, 2, 2>(a, s);
+    return fast_launch<TA, TB, FUSED, false, 64, 16, 4, 1, 128, 1, 2>(a, s);
+}
+
+template <bool TA, bool TB, bool FUSED>
+static hipError_t fast_shape(const GemmArgs& a, hipStream_t s) {
+    if (a.M <= 16 || a.N <= 16) return fast_few<TA, TB, FUSED>(a, s);
+    return fast_tile<TA, TB, FUSED, false>(a, s);
+}
+
 hipError_t gemm_fast_launch(int ta, int tb, const GemmArgs& g, hipStream_t s) {
-    if (g.fused) return fast_tile<false, true, true, false>(g, s);                      // NT only
+    // one row or column is a vector: as well k-contiguous
+    if (g.M == 1) ta = 0;
+    if (g.N == 1) tb = 1;
+    if (g.fused) return fast_shape<false, true, true>(g, s);                             // NT only
     if (g.sched == 1 || g.sched == 3) return fast_tile<false, true, false, true>(g, s);  // NT only
-    if (!ta && !tb) return fast_tile<false, false, false, false>(g, s);
-    if (!ta && tb) return fast_tile<false, true, false, false>(g, s);
-    if (ta && !tb) return fast_tile<true, false, false, false>(g, s);
-    return fast_tile<true, true, false, false>(g, s);
+    if (!ta && !tb) return fast_shape<false, false, false>(g, s);
+    if (!ta && tb) return fast_shape<false, true, false>(g, s);
+    if (ta && !tb) return fast_shape<true, false, false>(g, s);
+    return fast_shape<true, true, false>(g, s);
 }
 
 }  // namespace rac

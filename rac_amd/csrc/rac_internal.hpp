@@ -54,9 +54,9 @@ hipError_t act_grad_launch(const float* g, const float* pre, float* d, long coun
 // keeps the strength-reduced chain for every input (callers whose parity
 // bar is a summation bound, where subnormal-rounding differences of tiny
 // products are far below it).
-// The same product for M <= 16 rows or N <= 16 columns, A row-major (not
-// transposed): gemm_launch hands such launches (schedules 0 and 2) to the
-// few-row / few-column kernels.
+// The CORDIC and SHIFTADD products for M <= 16 rows or N <= 16 columns, A
+// row-major (not transposed): gemm_launch hands such launches (schedules 0
+// and 2) to the few-row / few-column kernels.
 struct SkinnyArgs {
     const float* A;
     const float* B;

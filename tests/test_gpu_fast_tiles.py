@@ -41,7 +41,11 @@ def run(A, B, C0, M, N, K, ta, tb, alpha, beta):
 
 SHAPES = [(17, 17, 4), (17, 33, 3), (20, 18, 1), (31, 32, 63), (33, 65, 64), (32, 31, 65), (63, 129, 15),
           (65, 64, 129), (127, 200, 16), (128, 257, 17), (129, 8200, 37), (300, 5633, 31), (500, 2049, 70),
-          (1000, 777, 131), (2047, 2177, 19), (2049, 4095, 33)]
+          (1000, 777, 131), (2047, 2177, 19), (2049, 4095, 33),
+          # few rows or columns: one, the 2 and 3 of a thin operand, 16; blocks
+          # of 32 and of 64, with both K-tiles
+          (1, 1, 5), (1, 31, 130), (2, 3, 70), (3, 2100, 129), (16, 33, 127), (5, 8300, 65), (2, 16500, 131),
+          (33, 1, 64), (2100, 3, 129), (31, 16, 257), (8300, 2, 65), (16500, 7, 131)]
 
 
 @pytest.mark.parametrize("layout", [(0, 0), (0, 1), (1, 0), (1, 1)])
