@@ -215,6 +215,18 @@ int rac_attention_probs_rows_dev(const float *q, const float *k, const float *ma
                                  float *P, int batch, int n_heads, int seq, int head_dim, int row0,
                                  int rows, int iters, int mode, void *stream);
 
+/* The attention core's gradients for query rows row0 .. row0+rows-1, from
+ * their probabilities P [batch*n_heads, rows, seq]: dq rows row0 .. (null:
+ * not wanted), dk (null: not wanted) and dv [batch*n_heads, seq, head_dim],
+ * overwritten, or added to when `accumulate` (later chunks of rows).
+ * causal_unmasked: P is that of is_causal with no additive mask.  workspace:
+ * rac_attention_backward_workspace_bytes bytes. */
+long rac_attention_backward_workspace_bytes(int batch, int n_heads, int seq, int rows);
+int rac_attention_backward_dev(const float *q, const float *k, const float *v, const float *P,
+                               const float *grad_out, int causal_unmasked, float *dq, float *dk, float *dv,
+                               int batch, int n_heads, int seq, int head_dim, int row0, int rows,
+                               int accumulate, float *workspace, int iters, int mode, void *stream);
+
 /* ── reference launcher ABI (rac_kernels.hip:822-909; bound by
  *    rac_torch_bind.cpp:16-45 with the stream as void*) ──────────────────── */
 

@@ -91,6 +91,9 @@ _SIGNATURES = {
     "rac_attention_ws_dev": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _vp, _l, _i, _i, _vp]),
     "rac_attention_probs_dev": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _vp, _i, _i, _vp]),
     "rac_attention_probs_rows_dev": (_i, [_vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),
+    "rac_attention_backward_workspace_bytes": (_l, [_i, _i, _i, _i]),
+    "rac_attention_backward_dev": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _i,
+                                        _i, _vp]),
     # rac_decode.h — decode step pieces, cache position in device memory
     "rac_decode_attention_dev": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _l, _vp, _f, _i, _vp]),
     "rac_kv_append_dev": (_i, [_vp, _vp, _vp, _i, _i, _l, _vp, _vp]),

@@ -992,6 +992,68 @@ RAC_EXPORT int rac_attention_probs_rows_dev(const float* q, const float* k, cons
                                  clamp_iters(iters), mode, (hipStream_t)stream);
 }
 
+// The attention core's gradients for query rows row0 .. row0+rows-1, from
+// their probabilities P [batch*n_heads, rows, seq]: dV (+)= P^T dO, dP = dO
+// V^T, dS = P (dP - rowsum(dP P)), dQ = s dS K, dK (+)= s dS^T Q, every
+// product on the RAC GEMM.  A causal P without an additive mask is exactly
+// zero past the diagonal; in FAST mode the products then skip that half (a
+// zero term leaves an accumulator as it is) when a device check finds every
+// operand bounded (0 * inf is NaN), and take every k otherwise.
+RAC_EXPORT long rac_attention_backward_workspace_bytes(int batch, int n_heads, int seq, int rows) {
+    if (batch <= 0 || n_heads <= 0 || seq <= 0 || rows <= 0) return 0;
+    return attention_scores_bytes((long)batch * n_heads, seq, rows) + 256;
+}
+
+RAC_EXPORT int rac_attention_backward_dev(const float* q, const float* k, const float* v, const float* P,
+                                          const float* grad_out, int causal_unmasked, float* dq, float* dk, float* dv,
+                                          int batch, int n_heads, int seq, int head_dim, int row0, int rows,
+                                          int accumulate, float* workspace, int iters, int mode, void* stream) {
+    int rc = check_attention(q, k, v, grad_out, batch, n_heads, seq, head_dim);
+    if (rc) return rc;
+    if (!P || !dv || !workspace) return fail(RAC_ERR_NULL_PTR, "rac_attention_backward_dev: null buffer");
+    if (mode < 0 || mode > 2) return fail(RAC_ERR_INVALID_DIM, "rac_attention_backward_dev: mode must be 0, 1 or 2");
+    if (row0 < 0 || rows <= 0 || (long)row0 + rows > seq)
+        return fail(RAC_ERR_INVALID_DIM, "rac_attention_backward_dev: rows %d .. %ld outside 0 .. %d", row0,
+                    (long)row0 + rows - 1, seq - 1);
+    const hipStream_t s = (hipStream_t)stream;
+    const int bh = batch * n_heads, t = seq, d = head_dim, c = rows;
+    const long td = (long)t * d, ct = (long)c * t, off = (long)row0 * d;
+    const float scale = 1.0f / sqrtf((float)d), beta = accumulate ? 1.0f : 0.0f;
+    iters = clamp_iters(iters);
+    // the sizes the FAST tiles take with a causal limit (K and side-by-side
+    // rows of at least 4), and head_dim within the bound check's 4096 terms
+    int* flag = nullptr;
+    if (causal_unmasked && mode == kModeFast && t >= 4 && c >= 4 && d >= 4 && d <= 4096) {
+        flag = reinterpret_cast<int*>(reinterpret_cast<char*>(workspace) + attention_scores_bytes(bh, t, c));
+        rc = check_hip(all_bounded_launch(q, k, v, grad_out, bh * td, flag, s), "rac_attention_backward bound check");
+        if (rc) return rc;
+    }
+    rc = check_hip(gemm_launch(1, 0, P, grad_out + off, dv, t, d, c, 1.0f, beta, iters, mode, s, bh, ct, td, td, 0,
+                               flag, true, row0, 2),
+                   "rac_attention_backward dV launch");
+    if (rc || (!dq && !dk)) return rc;
+    rc = check_hip(gemm_launch(0, 1, grad_out + off, v, workspace, c, t, d, 1.0f, 0.0f, iters, mode, s, bh, td, td, ct,
+                               0, flag, true, row0, 3),
+                   "rac_attention_backward dP launch");
+    if (rc) return rc;
+    rc = check_hip(attn_dscore_launch(P, workspace, (long)bh * c, t, c, row0, flag, s),
+                   "rac_attention_backward dS launch");
+    if (rc) return rc;
+    if (dq) {
+        rc = check_hip(gemm_launch(0, 0, workspace, k, dq + off, c, d, t, scale, 0.0f, iters, mode, s, bh, ct, td, td,
+                                   0, flag, true, row0, 1),
+                       "rac_attention_backward dQ launch");
+        if (rc) return rc;
+    }
+    if (dk) {
+        rc = check_hip(gemm_launch(1, 0, workspace, q + off, dk, t, d, c, scale, beta, iters, mode, s, bh, ct, td, td,
+                                   0, flag, true, row0, 2),
+                       "rac_attention_backward dK launch");
+        if (rc) return rc;
+    }
+    return RAC_OK;
+}
+
 // ── Q8_0 weights and decode GEMV (lib/c/rac_q8_0.h) ─────────────────────
 
 static int check_q8(const char* who, const void* a, const void* b, long rows, long K) {

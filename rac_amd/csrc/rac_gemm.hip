@@ -373,6 +373,36 @@ __global__ __launch_bounds__(256) void all_finite_kernel(const float* __restrict
 
 __global__ void set_flag_kernel(int* flag, int v) { *flag = v; }
 
+// flag = 1 unless some element of the four arrays (n each) is 2^58 or more
+// in magnitude, infinite or NaN: then no product of two of them over up to
+// 4096 k overflows, and what a causal backward pass may skip is exactly zero.
+__global__ __launch_bounds__(256) void all_bounded_kernel(const float* __restrict__ a, const float* __restrict__ b,
+                                                          const float* __restrict__ c, const float* __restrict__ d,
+                                                          long n, int* __restrict__ flag) {
+    const float* x = blockIdx.y == 0 ? a : blockIdx.y == 1 ? b : blockIdx.y == 2 ? c : d;
+    typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
+    float m = 0.0f;                                      // the largest magnitude; a NaN stays
+    const long n4 = n / 4, stride = (long)gridDim.x * 256;
+#pragma unroll 4
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n4; i += stride) {
+        const v4u q = reinterpret_cast<const v4u*>(x)[i];
+#pragma unroll
+        for (int e = 0; e < 4; e++) m = __builtin_elementwise_maximum(m, __builtin_fabsf(q[e]));
+    }
+    if (blockIdx.x == 0 && threadIdx.x < n - 4 * n4)
+        m = __builtin_elementwise_maximum(m, __builtin_fabsf(x[4 * n4 + threadIdx.x]));
+    if (!(m < 0x1p58f)) *flag = 0;
+}
+
+hipError_t all_bounded_launch(const float* a, const float* b, const float* c, const float* d, long n, int* flag,
+                              hipStream_t s) {
+    hipLaunchKernelGGL(set_flag_kernel, dim3(1), dim3(1), 0, s, flag, 1);
+    const long blocks = n / 4096 + 1;
+    hipLaunchKernelGGL(all_bounded_kernel, dim3((unsigned)(blocks < 1024 ? blocks : 1024), 4), dim3(256), 0, s, a, b,
+                       c, d, n, flag);
+    return hipGetLastError();
+}
+
 hipError_t all_finite_launch(const float* x, long n, int* flag, hipStream_t s) {
     hipLaunchKernelGGL(set_flag_kernel, dim3(1), dim3(1), 0, s, flag, 1);
     long blocks = (n + 255) / 256;
@@ -505,9 +535,9 @@ static hipError_t dispatch(int ta, int tb, int mode, const GemmArgs& g, hipStrea
 hipError_t gemm_launch(int ta, int tb, const float* A, const float* B, float* C,
                        int M, int N, int K, float alpha, float beta, int iters, int mode,
                        hipStream_t s, int batch, long sa, long sb, long sc, int sched,
-                       const int* k_causal, bool exact_specials, int row0) {
+                       const int* k_causal, bool exact_specials, int row0, int k_side) {
     const GemmArgs g{A, B, C, M, N, K, alpha, beta, clamp_iters(iters), batch, sa, sb, sc,
-                     GemmEpilogue(), false, sched, k_causal, exact_specials ? 1 : 0, row0, 1};
+                     GemmEpilogue(), false, sched, k_causal, exact_specials ? 1 : 0, row0, k_side};
     return dispatch(ta, tb, mode, g, s);
 }
 

@@ -23,7 +23,9 @@ struct GemmArgs {
     int row0;
     // with k_causal: 1, row tile m sums k only up to its last query position
     // row0 + m*BM + BM - 1 (P V); 2, only from k = m*BM - row0 on (P^T dO: row
-    // s of P^T is 0 before query position s, k = 0 being position row0)
+    // s of P^T is 0 before query position s, k = 0 being position row0); 3,
+    // tiles wholly above the diagonal are left unwritten (dO V^T, rows from
+    // query position row0).  2 and 3 in FAST mode only.
     int k_side;
 };
 

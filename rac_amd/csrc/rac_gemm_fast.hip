@@ -14,6 +14,7 @@
 // only one 16 x 16 tile to keep its matrix core busy, 8 cycles per k and 256
 // outputs, where the 32x32x1_2b form needs 2048 outputs for it.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <type_traits>
 #include "rac_act.hpp"
 #include "rac_gemm.hpp"
@@ -157,7 +158,7 @@ struct FastGeom {
     int iters;
     GemmEpilogue ep;
     const int* k_causal;
-    int k_side;           // 0: every k; 1, 2: the causal limits of GemmArgs, when *k_causal holds 1
+    int k_side;           // 0: every k; 1-3: the causal limits of GemmArgs, when *k_causal holds 1
     int row0;
     int tiles, tiles_m;   // output tiles of one batch item, rows of them
     int batch;
@@ -221,7 +222,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const float* __
     if (L >= g.total) return;
     const int tiles_n = TRAP ? 1 : g.tiles / g.tiles_m;
     int z, tm, tn;
-    if (g.k_side) {
+    if (g.k_side == 1 || g.k_side == 2) {
         // tiles of unequal K: the longest first, one of every batch item in
         // turn (an item's tiles stay on one XCD where 8 divides the batch)
         z = (int)(L % g.batch);
@@ -259,9 +260,14 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const float* __
     B += z * g.sb;
     C += z * g.sc;
     int kbeg = 0, kend = g.K;
+    bool any_k = true;
     if (g.k_side && *g.k_causal == 1) {
         if (g.k_side == 1) kend = (int)min((long)g.K, (long)g.row0 + m0 + BM);
-        else kbeg = (int)min((long)g.K - 4, max(0L, m0 - g.row0));
+        else if (g.k_side == 3 && n0 > (long)g.row0 + m0 + BM - 1) return;
+        else if (g.k_side == 2) {
+            kbeg = (int)min((long)g.K - 4, max(0L, m0 - g.row0));
+            any_k = m0 - g.row0 < g.K;
+        }
     }
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -348,39 +354,41 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const float* __
             }
         }
     };
+    if (any_k) {
 #pragma unroll
-    for (int s = 0; s < PD; s++) {
-        before(s);
+        for (int s = 0; s < PD; s++) {
+            before(s);
 #pragma unroll
-        for (int x = 0; x < VA; x++) ta.load(va[s], x);
+            for (int x = 0; x < VA; x++) ta.load(va[s], x);
 #pragma unroll
-        for (int x = 0; x < VB; x++) tb.load(vb[s], x);
-        after(s);
-    }
-    fix(0, 0);
-    before(PD);
-#pragma unroll
-    for (int x = 0; x < VA + VB; x++) stage(0, 0, x, true);
-    after(PD);
-    __syncthreads();
-    int s = 0;
-    for (; s + 2 < nst; s += 2) {
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            fix(s + u + 1, (u + 1) % PD);
-            before(s + u + 1 + PD);
-            compute(u, std::true_type(), (u + 1) % PD, true);
-            after(s + u + 1 + PD);
-            __syncthreads();
+            for (int x = 0; x < VB; x++) tb.load(vb[s], x);
+            after(s);
         }
-    }
-    if (s + 1 < nst) {
-        fix(s + 1, 1 % PD);
-        compute(0, std::true_type(), 1 % PD, false);
+        fix(0, 0);
+        before(PD);
+#pragma unroll
+        for (int x = 0; x < VA + VB; x++) stage(0, 0, x, true);
+        after(PD);
         __syncthreads();
-        compute(1, std::false_type(), 0, false);
-    } else {
-        compute(0, std::false_type(), 0, false);
+        int s = 0;
+        for (; s + 2 < nst; s += 2) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                fix(s + u + 1, (u + 1) % PD);
+                before(s + u + 1 + PD);
+                compute(u, std::true_type(), (u + 1) % PD, true);
+                after(s + u + 1 + PD);
+                __syncthreads();
+            }
+        }
+        if (s + 1 < nst) {
+            fix(s + 1, 1 % PD);
+            compute(0, std::true_type(), 1 % PD, false);
+            __syncthreads();
+            compute(1, std::false_type(), 0, false);
+        } else {
+            compute(0, std::false_type(), 0, false);
+        }
     }
 
     // the operands are passed B first, so a lane holds four consecutive
@@ -419,32 +427,33 @@ static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
 // measured (K 1000-11008, all layouts): e.g. 2048 x 11008 x 4096 NT 1.39 ms
 // on 64x128 (128x128: 1.47, 64x64: 1.46), 500 x 2048 x 5632 NT 99 us on
 // 64x64 (32x64: 101, 32x32: 105), 128 x 11008 x 4096 NT 107 us on 32x64
-// (32x32: 113, 64x64: 124), 1500^3 NT 68 us on 32x32 (64x64: 80).  With a
-// causal limit the tiles' work is unequal and dispatched longest first: the
-// CUs share it evenly but for about one longest tile.
+// (32x32: 113, 64x64: 124), 1500^3 NT 68 us on 32x32 (64x64: 80).  With few
+// k a 128x128 tile is mostly start and end (32 x 2048 x 2048 x 128, causal:
+// 195 us, 64x128 190, 64x64 189).  A causal limit on k makes the tiles'
+// work unequal (half of K on average, dispatched longest first), so a CU
+// needs at least the longest tile's time: 32 x 2048 x 128 x 2048 150 us on
+// 64x64 (64x128 159, 128x128 162, 32x64 227), 8 x 1000 x 64 x 1000 15.5 us
+// on 32x64 (64x64 22).
 template <bool TA, bool TB, bool FUSED, bool TRAP>
 static hipError_t fast_tile(const GemmArgs& a, hipStream_t s) {
-    struct Shape { int bm, bn; double eff; };
-    constexpr Shape shapes[5] = {{128, 128, 0.93}, {64, 128, 0.91}, {64, 64, 0.83}, {32, 64, 0.81}, {32, 32, 0.76}};
+    struct Shape { int bm, bn; double eff, eff_causal; };
+    constexpr Shape shapes[5] = {{128, 128, 0.93, 0.80}, {64, 128, 0.91, 0.85}, {64, 64, 0.83, 0.88},
+                                 {32, 64, 0.81, 0.70}, {32, 32, 0.76, 0.65}};
     const long cus = device_cus();
+    const bool causal_k = a.k_causal && (a.k_side == 1 || a.k_side == 2);
     int best = 0;
     double best_cost = 0.0;
     for (int i = 0; i < 5; i++) {
         const long bm = shapes[i].bm, bn = shapes[i].bn, tm = (a.M + bm - 1) / bm;
-        double cost;
+        long t = tm * ((a.N + bn - 1) / bn);
         if (TRAP) {
-            long t = 0;
+            t = 0;
             for (long r = 0; r < tm; r++) t += trap_cols(a.row0, (int)r, (int)bm, (int)bn, a.N);
-            t *= a.batch;
-            cost = (double)((t + cus - 1) / cus) * bm * bn / shapes[i].eff;
-        } else if (a.k_causal && a.k_side) {
-            // about half of the k of all tiles, in units of K
-            const double per_cu = 0.5 * tm * ((a.N + bn - 1) / bn) * a.batch / cus;
-            cost = (per_cu + 1.0) * bm * bn / shapes[i].eff;
-        } else {
-            const long t = tm * ((a.N + bn - 1) / bn) * a.batch;
-            cost = (double)((t + cus - 1) / cus) * bm * bn / shapes[i].eff;
         }
+        t *= a.batch;
+        const double work = (double)bm * bn;
+        double cost = (double)((t + cus - 1) / cus) * work / (i == 0 && a.K < 512 ? 0.80 : shapes[i].eff);
+        if (causal_k) cost = std::max(0.5 * t / cus, 1.0) * work / shapes[i].eff_causal;
         if (i == 0 || cost < best_cost) {
             best = i;
             best_cost = cost;

@@ -82,9 +82,19 @@ hipError_t gemm_launch(int ta, int tb, const float* A, const float* B, float* C,
                        int M, int N, int K, float alpha, float beta, int iters, int mode,
                        hipStream_t s, int batch = 1, long sa = 0, long sb = 0, long sc = 0,
                        int sched = 0, const int* k_causal = nullptr, bool exact_specials = true,
-                       int row0 = 0);
+                       int row0 = 0, int k_side = 1);
 // *flag = 1 if every x[i] is finite, else 0 (stream-ordered).
 hipError_t all_finite_launch(const float* x, long n, int* flag, hipStream_t s);
+// *flag = 1 if every element of the four arrays is below 2^58 in magnitude,
+// else 0.
+hipError_t all_bounded_launch(const float* a, const float* b, const float* c, const float* d, long n, int* flag,
+                              hipStream_t s);
+// dS = P (dP - rowsum(dP P)) in place of dP, rows x seq each (query position
+// row0 + row % c); flag (may be null): when it holds 1, P is causal, only the
+// columns up to the query position are read, and the next 131 are written as
+// zeros.
+hipError_t attn_dscore_launch(const float* P, float* dP, long rows, long seq, long c, long row0, const int* flag,
+                              hipStream_t s);
 
 // Optional attention masking of each row r (query position t = row0 +
 // r % seq, column j): causal -> x = -inf for j > t; then x += mask[t*ld + j]

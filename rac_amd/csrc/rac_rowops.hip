@@ -108,7 +108,25 @@ __device__ __forceinline__ float softmax_lane_exps(float* v, float m, int iters,
     constexpr int E = 4 * VPT;
 #pragma unroll
     for (int e = 0; e < E; e++) v[e] = v[e] - m;
-    exp_lane<NITER, E>(v, iters, khinv);
+    if constexpr (MASKED) {
+        // the exps of -inf are +0: a wave skips the runs of its values that
+        // are -inf in every lane (past the diagonal of a causal row)
+        constexpr int G = E <= 8 ? 4 : 8;
+#pragma unroll
+        for (int b = 0; b < E; b += G) {
+            bool some = false;
+#pragma unroll
+            for (int e = 0; e < G; e++) some |= v[b + e] != -__builtin_inff();
+            if (__any(some)) {
+                exp_lane<NITER, G>(v + b, iters, khinv);
+            } else {
+#pragma unroll
+                for (int e = 0; e < G; e++) v[b + e] = 0.0f;
+            }
+        }
+    } else {
+        exp_lane<NITER, E>(v, iters, khinv);
+    }
     float s = 0.0f;
 #pragma unroll
     for (int e = 0; e < E; e++) s += v[e];
@@ -235,14 +253,16 @@ __device__ __forceinline__ void softmax_row_regs(float* v, long n4, long t, int 
     softmax_row_finish<VPT, NITER, MASKED>(v, m, iters, khinv, mk, red, zred);
 }
 
-template <int VPT, bool FULL>
-__device__ __forceinline__ void load_row_regs(const float* xrow, long n4, float* v) {
+// last: the last column needed (causal rows: the query position; the mask
+// puts -inf past it whatever was there).
+template <int VPT, bool FULL, bool MASKED = false>
+__device__ __forceinline__ void load_row_regs(const float* xrow, long n4, float* v, long last = 0) {
     const float4* xr = reinterpret_cast<const float4*>(xrow);
 #pragma unroll
     for (int i = 0; i < VPT; i++) {
         const long idx = threadIdx.x + (long)i * kRowThreads;
         float4 t = make_float4(-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff());
-        if (FULL || idx < n4) t = ld4_stream(&xr[idx]);
+        if ((FULL || idx < n4) && (!MASKED || 4 * idx <= last)) t = ld4_stream(&xr[idx]);
         v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
     }
 }
@@ -270,9 +290,9 @@ __global__ __launch_bounds__(kRowThreads) void softmax_reg_kernel(
     const long row = blockIdx.x;
     const long n4 = n / 4;
     float v[4 * VPT];
-    load_row_regs<VPT, FULL>(x + row * n, n4, v);
-    softmax_row_regs<VPT, NITER, MASKED, FULL>(v, n4, MASKED ? mk.row0 + row % mk.seq : 0, iters, khinv, mk,
-                                               red, zred);
+    const long t = MASKED ? mk.row0 + row % mk.seq : 0;
+    load_row_regs<VPT, FULL, MASKED>(x + row * n, n4, v, MASKED && mk.causal ? t : n);
+    softmax_row_regs<VPT, NITER, MASKED, FULL>(v, n4, t, iters, khinv, mk, red, zred);
     store_row_regs<VPT, FULL>(y + row * n, n4, v);
 }
 
@@ -663,6 +683,104 @@ hipError_t layernorm_launch(const float* x, float* y, const float* gamma, const 
         hipLaunchKernelGGL((layernorm_reg_kernel<16>), grid, block, 0, s, x, y, gamma, beta, eps, d, k);
     else
         hipLaunchKernelGGL(layernorm_loop_kernel, grid, block, 0, s, x, y, gamma, beta, eps, d, k);
+    return hipGetLastError();
+}
+
+// ── the attention backward's score gradients ─────────────────────────────
+
+// dS = P (dP - rowsum(dP P)), in place of dP, in one pass: both rows are held
+// in registers (4 VPT values of each per lane) between the sum and the
+// products, where separate elementwise passes move each matrix six times.
+// W waves per row (1: rows of up to 512, four to a workgroup).  Bound by
+// memory: [32, 2048, 2048] in 155 us causal (804 MB: half of each matrix).
+// With *flag == 1 (causal P, nothing past the diagonal but zeros) row t reads
+// columns 0 .. t and also writes zeros to t + 131, as far as the products'
+// 128-wide tiles and their last 4 k look past the diagonal.
+template <int W, int VPT>
+__global__ __launch_bounds__(256) void attn_dscore_kernel(const float* __restrict__ P, float* dP, long rows, long n,
+                                                          long c, long row0, const int* flag) {
+    constexpr int LANES = 64 * W;
+    __shared__ float red[kRowWaves];
+    const int lane = threadIdx.x % LANES;
+    const long row = (long)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+    if (W == 1 && row >= rows) return;
+    const bool causal = flag && *flag == 1;
+    const long t = row0 + row % c;
+    const long have = causal ? min(n, t + 1) : n, want = causal ? min(n, t + 132) : n;
+    const float* p = P + row * n;
+    float* d = dP + row * n;
+    // 16-byte accesses at any 4-byte boundary
+    typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
+    auto get = [&](const float* x, long j, float* v) {
+        if (j + 3 < have) {
+            const v4u q = *reinterpret_cast<const v4u*>(x + j);
+            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = j + e < have ? x[j + e] : 0.0f;
+        }
+    };
+    auto put = [&](long j, const float* pv, const float* dv, float s) {
+        v4u o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = j + e < have ? pv[e] * (dv[e] - s) : 0.0f;
+        if (j + 3 < want) {
+            *reinterpret_cast<v4u*>(d + j) = o;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; e++)
+                if (j + e < want) d[j + e] = o[e];
+        }
+    };
+    float s = 0.0f;
+    if constexpr (VPT > 0) {
+        float pv[4 * VPT], dv[4 * VPT];
+#pragma unroll
+        for (int i = 0; i < VPT; i++) {
+            const long j = 4L * (lane + i * LANES);
+            get(p, j, pv + 4 * i);
+            get(d, j, dv + 4 * i);
+        }
+#pragma unroll
+        for (int e = 0; e < 4 * VPT; e++) s = __builtin_fmaf(dv[e], pv[e], s);
+        if constexpr (W == 1) s = wave_sum(s);
+        else s = block_sum<false>(s, red);
+#pragma unroll
+        for (int i = 0; i < VPT; i++) {
+            const long j = 4L * (lane + i * LANES);
+            if (j < want) put(j, pv + 4 * i, dv + 4 * i, s);
+        }
+    } else {
+        for (long j = 4L * lane; j < have; j += 4L * LANES) {
+            float pv[4], dv[4];
+            get(p, j, pv);
+            get(d, j, dv);
+#pragma unroll
+            for (int e = 0; e < 4; e++) s = __builtin_fmaf(dv[e], pv[e], s);
+        }
+        s = block_sum<false>(s, red);
+        for (long j = 4L * lane; j < want; j += 4L * LANES) {
+            float pv[4], dv[4];
+            get(p, j, pv);
+            get(d, j, dv);
+            put(j, pv, dv, s);
+        }
+    }
+}
+
+hipError_t attn_dscore_launch(const float* P, float* dP, long rows, long seq, long c, long row0, const int* flag,
+                              hipStream_t s) {
+#define RAC_DSCORE(W, VPT)                                                                                     \
+    hipLaunchKernelGGL((attn_dscore_kernel<W, VPT>), dim3((unsigned)((rows * W + 3) / 4)), dim3(256), 0, s, P, \
+                       dP, rows, seq, c, row0, flag)
+    if (seq <= 256) RAC_DSCORE(1, 1);
+    else if (seq <= 512) RAC_DSCORE(1, 2);
+    else if (seq <= 1024) RAC_DSCORE(4, 1);
+    else if (seq <= 2048) RAC_DSCORE(4, 2);
+    else if (seq <= 4096) RAC_DSCORE(4, 4);
+    else if (seq <= 8192) RAC_DSCORE(4, 8);
+    else RAC_DSCORE(4, 0);
+#undef RAC_DSCORE
     return hipGetLastError();
 }
 

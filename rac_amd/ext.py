@@ -674,6 +674,38 @@ def attention_probs_rows(q: torch.Tensor, k: torch.Tensor, mask: Optional[torch.
     return P
 
 
+def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, P: torch.Tensor, grad_out: torch.Tensor,
+                       causal_unmasked: bool, dq: Optional[torch.Tensor], dk: Optional[torch.Tensor],
+                       dv: torch.Tensor, row0: int = 0, accumulate: bool = False, iters: int = 0,
+                       mode: int = -1) -> None:
+    """Gradients of attention() for query rows row0 .. row0 + rows - 1 from
+    their probabilities P [B, H, rows, T], through
+    rac_attention_backward_dev: dq's rows, dk and dv (contiguous [B, H, T, D];
+    dq and dk may be None), dk and dv added to when `accumulate`.
+    causal_unmasked: P is that of is_causal without an additive mask."""
+    for t, n in ((q, "q"), (k, "k"), (v, "v"), (P, "P"), (grad_out, "grad_out"), (dq, "dq"), (dk, "dk"), (dv, "dv")):
+        if t is not None:
+            _require_f32(t, n)
+            if t.dim() != 4 or not t.is_contiguous():
+                raise RuntimeError(f"RAC: attention_backward needs a contiguous 4-D {n}")
+            if n != "P" and t.shape != q.shape:
+                raise RuntimeError(f"RAC: {n} must have q's shape")
+    B, H, T, D = q.shape
+    rows = P.size(2)
+    if P.shape != (B, H, rows, T):
+        raise RuntimeError("RAC: P must be [B, H, rows, T]")
+    iters, mode = _resolve(iters, mode)
+    lib = _lib.load()
+    ws = torch.empty(lib.rac_attention_backward_workspace_bytes(B, H, T, rows) // 4, device=q.device,
+                     dtype=torch.float32)
+    check(lib.rac_attention_backward_dev(q.data_ptr(), k.data_ptr(), v.data_ptr(), P.data_ptr(), grad_out.data_ptr(),
+                                         int(bool(causal_unmasked)), dq.data_ptr() if dq is not None else None,
+                                         dk.data_ptr() if dk is not None else None, dv.data_ptr(), B, H, T, D,
+                                         int(row0), rows, int(bool(accumulate)), ws.data_ptr(), iters, mode,
+                                         _stream(dv)),
+          "rac_attention_backward_dev")
+
+
 # ── vector primitives (rac.h:101-250) ───────────────────────────────────────
 
 VEC2_OPS = {
@@ -1104,7 +1136,7 @@ __all__ = [
     "matmul_forward", "matmul_backward", "linear_forward", "linear_backward",
     "softmax", "rmsnorm", "layernorm", "exp", "silu", "sigmoid", "tanh", "gelu", "relu",
     "rsqrt", "sincos", "rope_inv_freq", "rope_cache", "rope_apply_", "rope_apply",
-    "bmm", "softmax_masked_", "attention", "attention_probs_rows", "vec2", "inner", "outer", "dct", "VEC2_OPS",
+    "bmm", "softmax_masked_", "attention", "attention_probs_rows", "attention_backward", "vec2", "inner", "outer", "dct", "VEC2_OPS",
     "fused_linear_forward", "fused_linear_backward", "act_grad", "attention_scale",
     "q8_quantize", "q8_dequantize", "q8_gemv", "Q8_BLOCK_BYTES",
     "dsp_eval", "dsp_systolic", "DSP_OPS", "SafeTensors",

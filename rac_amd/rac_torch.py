@@ -793,40 +793,20 @@ class RACAttentionFunction(Function):
     def backward(ctx, g):
         q, k, v, m, P = ctx.saved_tensors
         B, H, T, D = q.shape
-        Z = B * H
-        scale = _rac.attention_scale(D)
-        need_q, need_k = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        g3 = g.float().contiguous().view(Z, T, D)
-        q3, k3, v3 = q.view(Z, T, D), k.view(Z, T, D), v.view(Z, T, D)
+        g = g.float().contiguous()
+        bare = ctx.is_causal and m is None
+        dQ = torch.empty_like(q) if ctx.needs_input_grad[0] else None
+        dK = torch.empty_like(k) if ctx.needs_input_grad[1] else None
+        dV = torch.empty_like(v)
         if P is not None:
-            P3 = P.view(Z, T, T)
-            dV = _rac.bmm(P3, g3, trans_a=True, **_kw())
-            dP = _rac.bmm(g3, v3, trans_b=True, **_kw())
-            dS = P3 * (dP - (dP * P3).sum(-1, keepdim=True))
-            dQ = _rac.bmm(dS, k3, alpha=scale, **_kw()) if need_q else None
-            dK = _rac.bmm(dS, q3, trans_a=True, alpha=scale, **_kw()) if need_k else None
+            _rac.attention_backward(q, k, v, P, g, bare, dQ, dK, dV, **_kw())
         else:
-            rows = _ATTN_BWD_CHUNK_BYTES // (4 * Z * T)
+            rows = _ATTN_BWD_CHUNK_BYTES // (4 * B * H * T)
             rows = T if rows >= T else max(64, rows // 64 * 64)
-            dV = torch.zeros((Z, T, D), device=q.device, dtype=torch.float32)
-            dQ = torch.empty((Z, T, D), device=q.device, dtype=torch.float32) if need_q else None
-            dK = torch.zeros((Z, T, D), device=q.device, dtype=torch.float32) if need_k else None
             for t0 in range(0, T, rows):
-                r = min(rows, T - t0)
-                Pc = _rac.attention_probs_rows(q, k, m, ctx.is_causal, t0, r, **_kw()).view(Z, r, T)
-                gc = g3[:, t0:t0 + r].contiguous()
-                _rac.bmm(Pc, gc, trans_a=True, out=dV, beta=1.0, **_kw())
-                dP = _rac.bmm(gc, v3, trans_b=True, **_kw())
-                dS = Pc * (dP - (dP * Pc).sum(-1, keepdim=True))
-                del dP, Pc
-                if need_q:
-                    dQ[:, t0:t0 + r] = _rac.bmm(dS, k3, alpha=scale, **_kw())
-                if need_k:
-                    _rac.bmm(dS, q3[:, t0:t0 + r].contiguous(), trans_a=True, alpha=scale, out=dK, beta=1.0,
-                             **_kw())
-        shape = (B, H, T, D)
-        return (dQ.view(shape) if dQ is not None else None, dK.view(shape) if dK is not None else None,
-                dV.view(shape), None, None)
+                Pc = _rac.attention_probs_rows(q, k, m, ctx.is_causal, t0, min(rows, T - t0), **_kw())
+                _rac.attention_backward(q, k, v, Pc, g, bare, dQ, dK, dV, row0=t0, accumulate=t0 > 0, **_kw())
+        return dQ, dK, dV, None, None
 
 
 def rac_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optional[torch.Tensor] = None,
