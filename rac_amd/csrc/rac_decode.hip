@@ -9,7 +9,7 @@
 // arguments: the step can be recorded once as a HIP graph and replayed per
 // token, the position advancing inside the graph.
 //
-// Attention is one workgroup (256 lanes) per query head h, reading key /
+// Attention is one workgroup per query head h, reading key /
 // value head g = h / rep of a cache laid out [n_kv_heads, t_cap, d_head]
 // (each head's keys a row-major matrix).  Its arithmetic is that of the
 // composition  scores = alpha * (q K^T) (FAST MAC: one fmaf chain over
@@ -44,23 +44,23 @@ __device__ __forceinline__ void dec_exp4(float* v, int iters, float khinv) {
 // V tile staged in LDS for the P V chains: kDecTile floats (16 KB)
 constexpr int kDecTile = 4096;
 
-// Scores: lane t computes positions t, t + 256, ... (one fmaf chain each;
-// DH > 0: the row's DH / 4 16-byte loads are issued together).  Softmax:
+// Any d_head and alignment (the shapes the matrix-core kernel below does not
+// take): one workgroup per query head.
+// Scores: lane t computes positions t, t + 256, ... (one fmaf chain each).  Softmax:
 // lane l takes the groups l, l + 256, ... as the row kernel.  P V: the
 // value rows pass through LDS a tile at a time (every lane loads, the next
 // tile's loads are in flight during the chains), and lane c < d_head runs
 // output column c's chain over the tile.
-template <int NITER, int DH>
+template <int NITER>
 __global__ __launch_bounds__(kRowThreads) void decode_attention_kernel(
     const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
-    float* __restrict__ out, int rep, int dh_rt, long t_cap, const int* __restrict__ pos_dev, float scale,
+    float* __restrict__ out, int rep, int dh, long t_cap, const int* __restrict__ pos_dev, float scale,
     int iters, float khinv)
 {
     __shared__ __attribute__((aligned(16))) float sq[kDecodeMaxHead];
     __shared__ __attribute__((aligned(16))) float sp[kDecodeMaxLen];
     __shared__ __attribute__((aligned(16))) float sv[kDecTile];
     __shared__ float red[2 * kRowWaves];
-    const int dh = DH > 0 ? DH : dh_rt;
     const int tid = threadIdx.x;
     const int h = blockIdx.x;
     const long g = h / rep;
@@ -81,21 +81,7 @@ __global__ __launch_bounds__(kRowThreads) void decode_attention_kernel(
     for (int j = tid; j < n; j += kRowThreads) {
         const float* kr = K + (long)j * dh;
         float acc = 0.0f;
-        if constexpr (DH > 0) {
-            float4 kv[DH / 4];
-#pragma unroll
-            for (int k = 0; k < DH / 4; k++) kv[k] = reinterpret_cast<const float4*>(kr)[k];
-#pragma unroll
-            for (int k = 0; k < DH / 4; k++) {
-                const float4 a = reinterpret_cast<const float4*>(sq)[k];
-                acc = __builtin_fmaf(a.x, kv[k].x, acc);
-                acc = __builtin_fmaf(a.y, kv[k].y, acc);
-                acc = __builtin_fmaf(a.z, kv[k].z, acc);
-                acc = __builtin_fmaf(a.w, kv[k].w, acc);
-            }
-        } else {
-            for (int k = 0; k < dh; k++) acc = __builtin_fmaf(sq[k], kr[k], acc);
-        }
+        for (int k = 0; k < dh; k++) acc = __builtin_fmaf(sq[k], kr[k], acc);
         sp[j] = scale * acc;
     }
     if (tid < 4 * n4 - n) sp[n + tid] = -__builtin_inff();       // the row's -inf padding
@@ -149,7 +135,6 @@ __global__ __launch_bounds__(kRowThreads) void decode_attention_kernel(
     // out[c] = sum_j p_j V[j][c], one chain per output column in j order
     const int tj = kDecTile / dh;                        // value rows per tile
     constexpr int kF4 = kDecTile / 4 / kRowThreads;      // tile float4 per lane
-    const bool vec = DH > 0;
     float4 pre[kF4];
     auto fetch = [&](int j0) {                           // rows j0 .. of the tile into registers
         const int cnt = (n - j0 < tj ? n - j0 : tj) * dh;
@@ -157,14 +142,10 @@ __global__ __launch_bounds__(kRowThreads) void decode_attention_kernel(
 #pragma unroll
         for (int i = 0; i < kF4; i++) {
             const int e = (tid + i * kRowThreads) * 4;
-            if (vec) {
-                pre[i] = e < cnt ? *reinterpret_cast<const float4*>(src + e) : make_float4(0.f, 0.f, 0.f, 0.f);
-            } else {
-                pre[i].x = e < cnt ? src[e] : 0.0f;
-                pre[i].y = e + 1 < cnt ? src[e + 1] : 0.0f;
-                pre[i].z = e + 2 < cnt ? src[e + 2] : 0.0f;
-                pre[i].w = e + 3 < cnt ? src[e + 3] : 0.0f;
-            }
+            pre[i].x = e < cnt ? src[e] : 0.0f;
+            pre[i].y = e + 1 < cnt ? src[e + 1] : 0.0f;
+            pre[i].z = e + 2 < cnt ? src[e + 2] : 0.0f;
+            pre[i].w = e + 3 < cnt ? src[e + 3] : 0.0f;
         }
     };
     float acc = 0.0f;
@@ -188,17 +169,287 @@ __global__ __launch_bounds__(kRowThreads) void decode_attention_kernel(
     if (tid < dh) o[tid] = acc;
 }
 
+// ── the same on the matrix cores (d_head 32, 64, 128; 16-byte rows) ──────
+//
+// One workgroup of 16 waves per query head.  Every chain of the form above is
+// kept, four k per instruction: a 16x16x4 matrix instruction is four in-order
+// fmaf steps on each of 16 x 16 outputs (rac_gemm_fast.hip), here on 16
+// positions (scores) or 16 columns (P V) of one head.  What bounds a step of
+// a few hundred positions is latency, so each stage spreads over the waves
+// and its loads are requested stages ahead:
+//   scores   a wave takes 16 positions at a time, two such tiles in flight:
+//            its key rows come by 16-byte loads of whole rows and pass through
+//            a piece of LDS of its own (permuted as below; no barrier).
+//            Loaded as the instruction wants them, 16 rows by 64 bytes, four
+//            neighbouring lanes touch four cache lines: 132 KB of keys took
+//            4.7 us to request, against 3.1;
+//   softmax  one exp per lane and 1024 positions; the row sum on four waves
+//            in the row kernel's order; the probabilities go to LDS permuted,
+//            k = 4 t + q of a 16-k group at 4 q + t, so that one ds_read_b128
+//            feeds four instructions;
+//   P V      a wave per 16 columns; its values, kDecAhead groups of 16
+//            positions in flight from before the scores on, go straight to
+//            the instruction: 10-14 cycles per position of the chain, where a
+//            lane of the VALU form took ~35 (its fmaf, its LDS reads).
+// Replayed in a graph (32 heads over 4, d_head 64), before -> now: length 1
+// 4.0 -> 4.3, 256 8.6 -> 6.7, 516 14.7 -> 10.3, 2047 46.7 -> 29.1 us (d_head
+// 128: 4.4 -> 4.9, 11.8 -> 9.6, 21.5 -> 16.2, 75.3 -> 50.7).  Four heads to a
+// workgroup (one reading of the keys for them) were slower: 12.6 us at 516,
+// the exps of all four being on one CU.
+typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr int kDecWaves = 16, kDecThreads = 64 * kDecWaves;
+constexpr int kDecExps = kDecodeMaxLen / kDecThreads;       // positions per lane at most
+
+// EMAX: lanes hold up to EMAX positions (caches of up to 1024 EMAX)
+template <int NITER, int DH, int EMAX>
+__global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
+    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
+    float* __restrict__ out, int rep, long t_cap, const int* __restrict__ pos_dev, float scale, int iters,
+    float khinv)
+{
+    constexpr int DF = DH / 16, kDecTiles = DH == 128 ? 1 : 2, kDecAhead = DH == 128 ? 6 : 8;
+    // a wave's key staging: 16 rows of KP floats (a row, or half a long one)
+    constexpr int KP = DH < 64 ? DH : 64, KR = KP + 4, PARTS = DH / KP, VECS = KP / 16;
+    __shared__ __attribute__((aligned(16))) float sk[kDecWaves][16 * KR];
+    __shared__ __attribute__((aligned(16))) float sp[kDecThreads * EMAX];
+    __shared__ __attribute__((aligned(16))) float rmax[kDecWaves];
+    __shared__ __attribute__((aligned(16))) uint32_t rzero[kDecWaves];
+    __shared__ float rsum[kRowWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int li = lane % 16, lq = lane / 16;
+    // workgroup L runs on XCD L % 8: neighbouring heads, which share keys and
+    // values, on one XCD and its L2
+    const int nh = gridDim.x, h = nh % 8 ? blockIdx.x : (blockIdx.x % 8) * (nh / 8) + blockIdx.x / 8, g = h / rep;
+    const int pos = *pos_dev;
+    if (pos < 0 || pos >= t_cap || pos >= kDecodeMaxLen) {
+        // a position outside the cache: NaN output, nothing read
+        for (int c = tid; c < DH; c += kDecThreads) out[(long)h * DH + c] = __builtin_nanf("");
+        return;
+    }
+    const int n = pos + 1, n4 = (n + 3) / 4, n16 = (n + 15) / 16;
+    const float* K = kc + (long)g * t_cap * DH;
+    const float* V = vc + (long)g * t_cap * DH;
+
+    // keys of positions 16 b ..: part h (KP columns), 16-byte vector lane + 64 i
+    v4f kf[kDecTiles][DF];
+    auto kload = [&](int b, v4f (&f)[DF]) {
+#pragma unroll
+        for (int h = 0; h < PARTS; h++)
+#pragma unroll
+            for (int i = 0; i < VECS; i++) {
+                const int v = lane + 64 * i;
+                f[h * VECS + i] = *reinterpret_cast<const v4f*>(
+                    K + (long)min(16 * b + v / (KP / 4), n - 1) * DH + h * KP + 4 * (v % (KP / 4)));
+            }
+    };
+    float* skw = sk[wave];
+    const v4f q4 = *reinterpret_cast<const v4f*>(q + (long)h * DH + 4 * (lane % (DH / 4)));
+#pragma unroll
+    for (int u = 0; u < kDecTiles; u++)
+        if (wave + kDecWaves * u < n16) kload(wave + kDecWaves * u, kf[u]);
+
+    // P V's values, group of 16 positions b: V[16 b + 4 t + lq][16 wave + li],
+    // the last, partial group apart (zero past the row)
+    const bool pv_wave = wave < DF;
+    const int nf = n / 16;
+    v4f vr[kDecAhead], vt = {0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t voff = (uint32_t)(lq * DH + 16 * wave + li) * 4u;
+    auto vload = [&](int b) {
+        const char* base = reinterpret_cast<const char*>(V + (long)b * 16 * DH);
+        v4f v;
+#pragma unroll
+        for (int t = 0; t < 4; t++) v[t] = *reinterpret_cast<const float*>(base + 16 * t * DH + voff);
+        return v;
+    };
+    if (pv_wave) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int j = 16 * nf + 4 * t + lq;
+            if (j < n) vt[t] = V[(long)j * DH + 16 * wave + li];
+        }
+        if (nf) {
+#pragma unroll
+            for (int u = 0; u < kDecAhead; u++) vr[u] = vload(min(u, nf - 1));
+        }
+    }
+
+    // scores: every column of the instruction's output is this head; the
+    // query passes through the staging as the keys do
+    auto own_lds = [&]() {
+        // the wave's own writes, read back by other lanes
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    };
+    v4f qf[DF];                                                   // q[16 c + 4 t + lq]
+    if (lane < DH / 4) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) skw[(lane / 4) * 16 + lane % 4 + 4 * e] = q4[e];
+    }
+    own_lds();
+#pragma unroll
+    for (int c = 0; c < DF; c++) qf[c] = *reinterpret_cast<const v4f*>(skw + 16 * c + 4 * lq);
+    own_lds();
+    for (int b0 = wave; b0 < n16; b0 += kDecWaves * kDecTiles) {
+#pragma unroll
+        for (int u = 0; u < kDecTiles; u++) {
+            const int b = b0 + kDecWaves * u;
+            if (b < n16) {
+                v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int p = 0; p < PARTS; p++) {
+#pragma unroll
+                    for (int i = 0; i < VECS; i++) {
+                        const int v = lane + 64 * i, c = v % (KP / 4);
+                        float* o = skw + (v / (KP / 4)) * KR + (c / 4) * 16 + c % 4;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) o[4 * e] = kf[u][p * VECS + i][e];
+                    }
+                    own_lds();
+                    v4f a[VECS];
+#pragma unroll
+                    for (int c = 0; c < VECS; c++)
+                        a[c] = *reinterpret_cast<const v4f*>(skw + li * KR + 16 * c + 4 * lq);
+#pragma unroll
+                    for (int c = 0; c < VECS; c++)
+#pragma unroll
+                        for (int t = 0; t < 4; t++)
+                            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c][t], qf[p * VECS + c][t], acc, 0, 0, 0);
+                    own_lds();
+                }
+                if (b + kDecWaves * kDecTiles < n16) kload(b + kDecWaves * kDecTiles, kf[u]);
+                // positions j .. j + 3; -inf past the row
+                const int j = 16 * b + 4 * lq;
+                v4f v;
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[r] = j + r < n ? scale * acc[r] : -__builtin_inff();
+                if (li == 0) *reinterpret_cast<v4f*>(&sp[j]) = v;
+            }
+        }
+    }
+    __syncthreads();
+
+    // row maximum; a zero maximum takes the sign of the row's first zero
+    // (first_zero_max)
+    float e[EMAX];
+    float m = -__builtin_inff();
+#pragma unroll
+    for (int i = 0; i < EMAX; i++) {
+        const int j = tid + kDecThreads * i;
+        e[i] = j < n ? sp[j] : -__builtin_inff();
+        m = fmaxf(m, e[i]);
+    }
+    m = wave_max(m);
+    uint32_t key = ~0u;
+    if (m == 0.0f) {
+#pragma unroll
+        for (int i = EMAX - 1; i >= 0; i--)
+            if (e[i] == 0.0f) key = zero_key<uint32_t>(tid + kDecThreads * i, e[i]);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) key = min(key, (uint32_t)__shfl_xor((int)key, off, 64));
+    }
+    if (lane == 0) {
+        rmax[wave] = m;
+        rzero[wave] = key;
+    }
+    __syncthreads();
+    m = rmax[0];
+#pragma unroll
+    for (int i = 1; i < kDecWaves; i++) m = fmaxf(m, rmax[i]);
+    if (m == 0.0f) {
+        key = rzero[0];
+#pragma unroll
+        for (int i = 1; i < kDecWaves; i++) key = min(key, rzero[i]);
+        m = (key & 1) ? -0.0f : 0.0f;
+    }
+
+    // exps; a NaN score stays NaN and makes the row's sum, and every
+    // probability, NaN
+#pragma unroll
+    for (int i = 0; i < EMAX; i++) {
+        const int j = tid + kDecThreads * i;
+        if (j < 4 * n4) {
+            float v[1] = {e[i] - m};
+            const bool nan = v[0] != v[0];
+            if constexpr (NITER > 0) exp_cordic_vec<NITER, 1, kExpFlush | kExpNonPos>(v, khinv);
+            else v[0] = exp_cordic_rt(v[0], iters, khinv);
+            e[i] = nan ? __builtin_nanf("") : v[0];
+            sp[j] = e[i];
+        }
+    }
+    __syncthreads();
+    if (tid < kRowThreads) {
+        float s = 0.0f;
+        for (int gi = tid; gi < n4; gi += kRowThreads) {
+            const v4f v = *reinterpret_cast<const v4f*>(&sp[4 * gi]);
+#pragma unroll
+            for (int c = 0; c < 4; c++) s += v[c];
+        }
+        s = wave_sum(s);
+        if (lane == 0) rsum[wave] = s;
+    }
+    __syncthreads();
+    float s = rsum[0];
+#pragma unroll
+    for (int i = 1; i < kRowWaves; i++) s += rsum[i];
+    const float inv = 1.0f / s;
+#pragma unroll
+    for (int i = 0; i < EMAX; i++) {
+        const int j = tid + kDecThreads * i;
+        if (j < 16 * n16) sp[(j & ~15) + 4 * (j & 3) + ((j >> 2) & 3)] = j < n ? e[i] * inv : 0.0f;
+    }
+    __syncthreads();
+
+    if (pv_wave) {
+        const float* prow = sp + 4 * lq;
+        v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        auto mac = [&](v4f p, v4f v) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t], p[t], acc, 0, 0, 0);
+        };
+        auto probs = [&](int b) { return *reinterpret_cast<const v4f*>(prow + 16 * b); };
+        v4f p = probs(0);
+        int b0 = 0;
+        for (; b0 + kDecAhead < nf; b0 += kDecAhead) {
+#pragma unroll
+            for (int u = 0; u < kDecAhead; u++) {
+                const v4f pn = probs(b0 + u + 1);
+                mac(p, vr[u]);
+                vr[u] = vload(min(b0 + u + kDecAhead, nf - 1));
+                p = pn;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kDecAhead; u++)
+            if (b0 + u < nf) {
+                mac(p, vr[u]);
+                p = probs(min(b0 + u + 1, n16 - 1));
+            }
+        if (nf < n16) mac(p, vt);
+        if (li == 0) *reinterpret_cast<v4f*>(out + (long)h * DH + 16 * wave + 4 * lq) = acc;
+    }
+}
+
 template <int NITER>
 static hipError_t decode_attention_dh(int dh, bool vec, const float* q, const float* kc, const float* vc,
                                       float* out, int n_heads, int rep, long t_cap, const int* pos, float scale,
                                       int iters, float khinv, hipStream_t s) {
-#define RAC_DEC_ATT(D)                                                                                         \
-    hipLaunchKernelGGL((decode_attention_kernel<NITER, D>), dim3(n_heads), dim3(kRowThreads), 0, s, q, kc, vc, \
-                       out, rep, dh, t_cap, pos, scale, iters, khinv)
-    if (vec && dh == 64) RAC_DEC_ATT(64);
-    else if (vec && dh == 128) RAC_DEC_ATT(128);
-    else if (vec && dh == 32) RAC_DEC_ATT(32);
-    else RAC_DEC_ATT(0);
+#define RAC_DEC_ATT(D, E)                                                                                         \
+    hipLaunchKernelGGL((decode_attention_mfma_kernel<NITER, D, E>), dim3(n_heads), dim3(kDecThreads), 0, s, q, kc, \
+                       vc, out, rep, t_cap, pos, scale, iters, khinv)
+#define RAC_DEC_ATT_LEN(D)                         \
+    do {                                           \
+        if (t_cap <= 2 * kDecThreads) RAC_DEC_ATT(D, 2); \
+        else RAC_DEC_ATT(D, kDecExps);             \
+    } while (0)
+    if (vec && dh == 64) RAC_DEC_ATT_LEN(64);
+    else if (vec && dh == 128) RAC_DEC_ATT_LEN(128);
+    else if (vec && dh == 32) RAC_DEC_ATT_LEN(32);
+    else
+        hipLaunchKernelGGL((decode_attention_kernel<NITER>), dim3(n_heads), dim3(kRowThreads), 0, s, q, kc, vc, out,
+                           rep, dh, t_cap, pos, scale, iters, khinv);
+#undef RAC_DEC_ATT_LEN
 #undef RAC_DEC_ATT
     return hipGetLastError();
 }
@@ -209,9 +460,10 @@ hipError_t decode_attention_launch(const float* q, const float* kc, const float*
     iters = clamp_iters(iters);
     const float khinv = host_consts().exp_khinv[iters];
     const int rep = n_heads / n_kv_heads;
-    // 16-byte loads of key and value rows: rows on 16-byte boundaries
-    const bool vec = dh % 4 == 0 && (reinterpret_cast<uintptr_t>(kc) & 15) == 0 &&
-                     (reinterpret_cast<uintptr_t>(vc) & 15) == 0;
+    // 16-byte loads of query and key rows, 16-byte stores of the output
+    const uintptr_t any = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kc) |
+                          reinterpret_cast<uintptr_t>(vc) | reinterpret_cast<uintptr_t>(out);
+    const bool vec = (any & 15) == 0;
     switch (iters) {
         case 8: return decode_attention_dh<8>(dh, vec, q, kc, vc, out, n_heads, rep, t_cap, pos, scale, iters, khinv, s);
         case 16: return decode_attention_dh<16>(dh, vec, q, kc, vc, out, n_heads, rep, t_cap, pos, scale, iters, khinv, s);
