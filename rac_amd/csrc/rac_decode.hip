@@ -339,7 +339,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
         e[i] = j < n ? sp[j] : -__builtin_inff();
         m = fmaxf(m, e[i]);
     }
-    m = wave_max(m);
+    m = wave_max_valu(m);
     uint32_t key = ~0u;
     if (m == 0.0f) {
 #pragma unroll
@@ -385,7 +385,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
 #pragma unroll
             for (int c = 0; c < 4; c++) s += v[c];
         }
-        s = wave_sum(s);
+        s = wave_sum_valu(s);
         if (lane == 0) rsum[wave] = s;
     }
     __syncthreads();

@@ -166,20 +166,35 @@ __global__ __launch_bounds__(256, MX == 1 ? 4 : 2) void q8_gemv_kernel(const flo
     };
 
     float acc = 0.0f;          // lane tid < MX * R owns output (tid / R, j0 + tid % R)
-    fetch(chunk_start(0));
     float inv = 1.0f;
+    // NORM: the lane's first float4s of x are requested ahead of the weights:
+    // loads return in order, so behind them the norm would start only when
+    // the first chunk has come from memory (2560 x 2048 6.8 -> 5.9 us with
+    // the reduction on the VALU, 11264 x 2048 10.0 -> 9.4)
+    constexpr int kNX = 2;
+    float4 nx[NORM ? kNX : 1];
     if constexpr (NORM) {
+#pragma unroll
+        for (int i = 0; i < kNX; i++) nx[i] = reinterpret_cast<const float4*>(x)[min(tid + 256 * i, K / 4 - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    fetch(chunk_start(0));
+    if constexpr (NORM) {
+        __builtin_amdgcn_sched_barrier(0);
         __shared__ float red[kRowWaves];
         const float4* x4 = reinterpret_cast<const float4*>(x);
         float ss = 0.0f;
-        for (int i = tid; i < K / 4; i += 256) {
-            const float4 v = x4[i];
+        auto add = [&](float4 v) {
             ss = __builtin_fmaf(v.x, v.x, ss);
             ss = __builtin_fmaf(v.y, v.y, ss);
             ss = __builtin_fmaf(v.z, v.z, ss);
             ss = __builtin_fmaf(v.w, v.w, ss);
-        }
-        const float ms = block_sum(ss, red) / (float)K;
+        };
+#pragma unroll
+        for (int i = 0; i < kNX; i++)
+            if (tid + 256 * i < K / 4) add(nx[i]);
+        for (int i = tid + 256 * kNX; i < K / 4; i += 256) add(x4[i]);
+        const float ms = block_sum<true, true, true>(ss, red) / (float)K;
         inv = rsqrt_cordic(ms + fz.eps, fz.rs_khinv);
     }
     for (int c = 0; c < nch; c++) {
@@ -342,10 +357,13 @@ __global__ __launch_bounds__(256) void q8_gemv_generic_kernel(const float* __res
 
 // One input row on the fast path: the workgroup shape by the number of
 // rows.  16 rows per workgroup while that still gives two workgroups per
-// CU; below, 4 rows (8 when a row has fewer than 64 blocks) so that small
-// matrices spread over every CU (measured on MI355X with weights streamed
-// from HBM: 2560 x 2048 in 4.6 us instead of 5.2, 2048 x 5632 in 7.1
-// instead of 10.3).  The shape only changes which lane computes what.
+// CU; below, 4 rows (8 when a row has fewer than 64 blocks, or when every
+// workgroup computes the norm first) so that small matrices spread over
+// every CU (measured on MI355X with weights streamed from HBM: 2048 x 5632
+// in 6.0 us instead of 8.3; 2560 x 2048 behind a norm in 5.6 on 8 rows, 5.9 on
+// 4).  Rows of 16-31 blocks in chunks of 16 (512 x 512 2.7 us, in chunks of 8
+// with 32 rows 3.4; 3072 x 512 behind a norm 4.0 against 4.7).  The shape only
+// changes which lane computes what.
 template <bool NORM, int EPI>
 static void q8_launch_row(const float* x, const uint8_t* w, const float* bias, float* out, int N, int K, int act,
                           const Q8Fuse& fz, hipStream_t s) {
@@ -354,9 +372,10 @@ static void q8_launch_row(const float* x, const uint8_t* w, const float* bias, f
 #define RAC_Q8_ROW(CB, R)                                                                                   \
     hipLaunchKernelGGL((q8_gemv_kernel<1, CB, R, NORM, EPI>), dim3((unsigned)((N + R - 1) / R)), dim3(256), 0, \
                        s, x, w, bias, out, 1, N, K, act, fz)
-    if (nb < 32) RAC_Q8_ROW(8, 32);
+    if (nb < 16) RAC_Q8_ROW(8, 32);
+    else if (nb < 32) RAC_Q8_ROW(16, 16);
     else if ((N + 15) / 16 >= 2 * cus) RAC_Q8_ROW(32, 16);
-    else if (nb >= 64) RAC_Q8_ROW(64, 4);
+    else if (nb >= 64 && !NORM) RAC_Q8_ROW(64, 4);
     else RAC_Q8_ROW(32, 8);
 #undef RAC_Q8_ROW
 }

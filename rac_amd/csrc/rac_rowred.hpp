@@ -23,6 +23,45 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// op(v, v of lane ^ OFF) for the butterfly's steps, OFF = 32 .. 1 in turn, on
+// the VALU alone: the halves and the rows of 16 by v_permlane32_swap and
+// v_permlane16_swap (v with itself: one result holds the lower, the other the
+// upper part's value in every lane), the rest by a rotation inside the row:
+// once lanes i and i ^ 2 OFF agree, i + OFF and i ^ OFF do.  The same pairs,
+// and bits, as a shuffle by OFF, whose trip through LDS takes ~100 cycles a
+// step: for kernels that wait on one row's reduction (the decode attention:
+// 4.26 -> 3.96 us at one position).  The row kernels, which have other rows'
+// waves to run meanwhile, keep the shuffles: softmax 4096 x 4096 was slower
+// without (n = 16 28.5 -> 30.9 us, n = 24 32.1 -> 36.1).
+template <int OFF, class Op>
+__device__ __forceinline__ float butterfly_step(float v, Op op) {
+    const uint32_t u = __float_as_uint(v);
+    if constexpr (OFF == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else if constexpr (OFF == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else {
+        return op(v, __uint_as_float(__builtin_amdgcn_update_dpp(0, (int)u, 0x120 + OFF, 0xf, 0xf, false)));
+    }
+}
+template <class Op>
+__device__ __forceinline__ float butterfly(float v, Op op) {
+    v = butterfly_step<32>(v, op);
+    v = butterfly_step<16>(v, op);
+    v = butterfly_step<8>(v, op);
+    v = butterfly_step<4>(v, op);
+    v = butterfly_step<2>(v, op);
+    return butterfly_step<1>(v, op);
+}
+__device__ __forceinline__ float wave_sum_valu(float v) {
+    return butterfly(v, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float wave_max_valu(float v) {
+    return butterfly(v, [](float a, float b) { return fmaxf(a, b); });
+}
+
 // IEEE maximum (NaN-propagating; -0 < +0 like v_max_f32): no operand
 // canonicalisation, and a NaN anywhere reaches every lane.
 __device__ __forceinline__ float maximum(float a, float b) { return __builtin_elementwise_maximum(a, b); }
@@ -53,10 +92,10 @@ __device__ __forceinline__ void red_barrier() {
 // same value in every lane (fixed combination order).  TRAIL: end with a
 // barrier, so that `red` may be rewritten at once; callers that give each
 // reduction of a row its own `red` leave it off.  LDS_ONLY: the barriers
-// order LDS only (lds_barrier).
-template <bool TRAIL = true, bool LDS_ONLY = false>
+// order LDS only (lds_barrier).  VALU: wave_sum_valu's butterfly.
+template <bool TRAIL = true, bool LDS_ONLY = false, bool VALU = false>
 __device__ __forceinline__ float block_sum(float v, float* red) {
-    v = wave_sum(v);
+    v = VALU ? wave_sum_valu(v) : wave_sum(v);
     const int w = threadIdx.x / 64;
     if ((threadIdx.x & 63) == 0) red[w] = v;
     red_barrier<LDS_ONLY>();
