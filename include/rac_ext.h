@@ -74,6 +74,11 @@ int rac_gemm_batched_dev(const float *A, const float *B, float *C, int M, int N,
  * NULL; pre receives the pre-activation values when given. */
 int rac_fused_linear_dev(const float *input, const float *weight, const float *bias, float *out,
                          float *pre, int M, int N, int K, int act, int iters, int mode, void *stream);
+/* The same in FAST mode with input, weight, bias and out in bf16 (dtype 1) or
+ * fp16 (dtype 2): widened, computed in fp32 (pre is fp32) and rounded to
+ * nearest even.  K >= 4. */
+int rac_fused_linear_half_dev(const void *input, const void *weight, const void *bias, void *out,
+                              float *pre, int M, int N, int K, int act, int iters, int dtype, void *stream);
 /* d[i] = g[i] * act'(pre[i]) (rac_torch.cu:680-694), same activation ids. */
 int rac_act_grad_dev(const float *g, const float *pre, float *d, long count, int act, int iters,
                      void *stream);

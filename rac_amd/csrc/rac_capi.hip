@@ -413,6 +413,27 @@ RAC_EXPORT int rac_fused_linear_dev(const float* input, const float* weight, con
                      "rac_fused_linear_dev launch");
 }
 
+// rac_fused_linear_dev in FAST mode on 16-bit operands (dtype 1 bf16, 2
+// fp16: input, weight, bias and out), computed in fp32: the result of
+// widening them, running the fp32 layer and rounding its output to nearest
+// even, without those passes.
+RAC_EXPORT int rac_fused_linear_half_dev(const void* input, const void* weight, const void* bias, void* out,
+                                         float* pre, int M, int N, int K, int act, int iters, int dtype,
+                                         void* stream) {
+    int rc = check_gemm(input, weight, out, M, N, K);
+    if (rc) return rc;
+    if (K < 4) return fail(RAC_ERR_INVALID_DIM, "rac_fused_linear_half_dev: K must be at least 4");
+    if (act < 0 || act > 3) return fail(RAC_ERR_INVALID_DIM, "rac_fused_linear_half_dev: act must be 0..3");
+    if (dtype != 1 && dtype != 2)
+        return fail(RAC_ERR_INVALID_DIM, "rac_fused_linear_half_dev: dtype must be 1 (bf16) or 2 (fp16)");
+    GemmEpilogue ep;
+    ep.pre = pre;
+    ep.act = act;
+    ep.khinv = host_consts().exp_khinv[clamp_iters(iters)];
+    return check_hip(gemm_fused_half_launch(input, weight, bias, out, M, N, K, ep, iters, dtype, (hipStream_t)stream),
+                     "rac_fused_linear_half_dev launch");
+}
+
 // d[i] = g[i] * act'(pre[i]) for the activation ids of rac_fused_linear_dev.
 RAC_EXPORT int rac_act_grad_dev(const float* g, const float* pre, float* d, long count, int act, int iters,
                                 void* stream) {

@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
 {
     constexpr int DF = DH / 16, kDecTiles = DH == 128 ? 1 : 2, kDecAhead = DH == 128 ? 6 : 8;
     // a wave's key staging: 16 rows of KP floats (a row, or half a long one)
-    constexpr int KP = DH < 64 ? DH : 64, KR = KP + 4, PARTS = DH / KP, VECS = KP / 16;
+    constexpr int KP = DH < 64 ? DH : 64, KR = KP + 8, PARTS = DH / KP, VECS = KP / 16;
     __shared__ __attribute__((aligned(16))) float sk[kDecWaves][16 * KR];
     __shared__ __attribute__((aligned(16))) float sp[kDecThreads * EMAX];
     __shared__ __attribute__((aligned(16))) float rmax[kDecWaves];

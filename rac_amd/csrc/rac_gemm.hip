@@ -547,4 +547,13 @@ hipError_t gemm_fused_launch(const float* A, const float* W, float* C, int M, in
     return dispatch(0, 1, mode, g, s);
 }
 
+hipError_t gemm_fused_half_launch(const void* A, const void* W, const void* bias, void* C, int M, int N, int K,
+                                  const GemmEpilogue& ep, int iters, int dtype, hipStream_t s) {
+    GemmEpilogue e = ep;
+    e.bias = static_cast<const float*>(bias);                  // of the operands' type
+    const GemmArgs g{static_cast<const float*>(A), static_cast<const float*>(W), static_cast<float*>(C), M, N, K, 1.0f,
+                     0.0f, clamp_iters(iters), 1, 0, 0, 0, e, true, 0, nullptr, 1, 0, 0};
+    return gemm_fast_half_launch(dtype, g, s);
+}
+
 }  // namespace rac

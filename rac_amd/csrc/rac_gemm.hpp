@@ -42,5 +42,8 @@ __host__ __device__ __forceinline__ int trap_cols(int row0, int r, int BM, int B
 // FAST mode on the matrix cores (rac_gemm_fast.hip): K >= 4; at most one
 // operand stored with its rows side by side (A of ta, B of !tb) has 2 or 3.
 hipError_t gemm_fast_launch(int ta, int tb, const GemmArgs& g, hipStream_t s);
+// The fused linear layer (NT) with A, B, C and the bias in bf16 (dtype 1) or
+// fp16 (2), K >= 4; the products and sums in fp32, ep.pre in fp32.
+hipError_t gemm_fast_half_launch(int dtype, const GemmArgs& g, hipStream_t s);
 
 }  // namespace rac

@@ -25,30 +25,109 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // a float4 at any 4-byte boundary (global_load / store_dwordx4 need no more)
 typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
 
-__device__ __forceinline__ void store4(float* p, v4f v, int n) {
-    if (n >= 4) {
-        *reinterpret_cast<v4u*>(p) = v4u{v.x, v.y, v.z, v.w};
-        return;
+// Elements of the operands and the output: float, or the 16-bit formats of a
+// half-precision linear layer, widened (exactly) on the way to LDS and
+// rounded to nearest even on the way out: what converting whole tensors
+// before and after would give, without their passes over memory.
+// Q: four elements as loaded; shifted(): the first `sh` dropped, zeros behind.
+struct Bf16 { uint16_t bits; };
+struct F16 { uint16_t bits; };
+typedef uint32_t u2a __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+
+template <class T>
+struct Elem;
+template <>
+struct Elem<float> {
+    using Q = v4f;
+    static __device__ __forceinline__ Q load(const float* p) {
+        const v4u t = *reinterpret_cast<const v4u*>(p);
+        return v4f{t.x, t.y, t.z, t.w};
     }
-    if (n > 0) p[0] = v.x;
-    if (n > 1) p[1] = v.y;
-    if (n > 2) p[2] = v.z;
-}
+    static __device__ __forceinline__ v4f widen(Q v) { return v; }
+    static __device__ __forceinline__ Q shifted(Q v, int sh) {
+        if (sh & 1) v = v4f{v.y, v.z, v.w, 0.0f};
+        if (sh & 2) v = v4f{v.z, v.w, 0.0f, 0.0f};
+        if (sh & 4) v = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        return v;
+    }
+    static __device__ __forceinline__ float get(const float* p) { return *p; }
+    static __device__ __forceinline__ void store(float* p, v4f v, int n) {
+        if (n >= 4) {
+            *reinterpret_cast<v4u*>(p) = v4u{v.x, v.y, v.z, v.w};
+            return;
+        }
+        if (n > 0) p[0] = v.x;
+        if (n > 1) p[1] = v.y;
+        if (n > 2) p[2] = v.z;
+    }
+};
+template <class T>
+struct Elem16 {
+    using Q = u2v;
+    static __device__ __forceinline__ Q load(const T* p) {
+        const u2a t = *reinterpret_cast<const u2a*>(p);
+        return u2v{t.x, t.y};
+    }
+    static __device__ __forceinline__ Q shifted(Q v, int sh) {
+        const uint64_t x = sh >= 4 ? 0 : (((uint64_t)v.y << 32) | v.x) >> (16 * sh);
+        return u2v{(uint32_t)x, (uint32_t)(x >> 32)};
+    }
+};
+template <>
+struct Elem<Bf16> : Elem16<Bf16> {
+    static __device__ __forceinline__ v4f widen(Q v) {
+        return v4f{as_f(v.x << 16), as_f(v.x & 0xffff0000u), as_f(v.y << 16), as_f(v.y & 0xffff0000u)};
+    }
+    static __device__ __forceinline__ float get(const Bf16* p) { return as_f((uint32_t)p->bits << 16); }
+    static __device__ __forceinline__ void store(Bf16* p, v4f v, int n) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const uint32_t u = as_u(v[r]);
+            const uint32_t h = v[r] != v[r] ? 0x7fc0u : (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+            if (r < n) p[r].bits = (uint16_t)h;
+        }
+    }
+};
+template <>
+struct Elem<F16> : Elem16<F16> {
+    static __device__ __forceinline__ float widen1(uint32_t bits) {
+        const uint16_t h = (uint16_t)bits;
+        _Float16 f;
+        __builtin_memcpy(&f, &h, 2);
+        return (float)f;
+    }
+    static __device__ __forceinline__ v4f widen(Q v) {
+        return v4f{widen1(v.x), widen1(v.x >> 16), widen1(v.y), widen1(v.y >> 16)};
+    }
+    static __device__ __forceinline__ float get(const F16* p) { return widen1(p->bits); }
+    static __device__ __forceinline__ void store(F16* p, v4f v, int n) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const _Float16 f = (_Float16)v[r];
+            if (r < n) __builtin_memcpy(&p[r].bits, &f, 2);
+        }
+    }
+};
 
 // One operand's K-tile (KT k x ROWS rows) of a workgroup: global ->
 // registers -> LDS -> matrix-core operands.  Lane l of the instruction
 // holds element (row l % 16, k = 4 t + l / 16) of step t.
 //
 // KC (k contiguous in memory: A, or B^T of the NT layout): LDS rows of KT +
-// 4 floats, each 16-k group stored with k = 4 t + q at 4 q + t, so one
-// ds_read_b128 gives a lane its elements of four consecutive steps; both the
-// reads (8 lanes on 8 rows, 4 KT + 16 bytes apart) and the scattering writes
-// touch every bank once.  Otherwise LDS rows are k rows of ROWS + pad floats
-// (= 16 mod 32: the two k of a half wave on opposite banks), read a step at
-// a time.
-template <bool KC, int ROWS, int KT, int NL, bool THIN = false>
+// 8 floats, each 16-k group stored with k = 4 t + q at 4 q + t, so one
+// ds_read_b128 gives a lane its elements of four consecutive steps.  Rows 8
+// floats off a multiple of 16 are what keeps those reads free of bank
+// conflicts (measured: 4.1-4.5 cycles an instruction, like contiguous
+// lanes; 4 off 8.0, 0 off 32: 128 x 11008 x 4096 123 -> 109 us, 1024^3 24.6 ->
+// 22.4); the scattering writes take 6.5 (4 off: 5.0-6.4).  Otherwise LDS rows
+// are k rows of ROWS + pad floats (= 16 mod 32: the two k of a half wave on
+// opposite banks), read a step at a time.
+template <class T, bool KC, int ROWS, int KT, int NL, bool THIN = false>
 struct FastTile {
-    static constexpr int kStride = KC ? KT + 4 : ROWS + ((48 - ROWS % 32) % 32);
+    using El = Elem<T>;
+    using Q = typename El::Q;
+    static constexpr int kStride = KC ? KT + 8 : ROWS + ((48 - ROWS % 32) % 32);
     static constexpr int kFloats = (KC ? ROWS : KT) * kStride;
     static constexpr int kVecs = ROWS * KT / 4;                     // float4 of the tile
     static constexpr int kVPT = (kVecs + NL - 1) / NL;              // per lane
@@ -56,12 +135,12 @@ struct FastTile {
 
     // this lane's global addresses at the next K-tile to load; rows past the
     // matrix read rows inside it (their outputs are never stored)
-    const float* p[kVPT];
+    const T* p[kVPT];
     long step;                                                      // one K-tile further
     int shift;                                                      // !KC: see fix_rows()
 
     __device__ __forceinline__ static bool on(int i) { return kVecs % NL == 0 || (int)threadIdx.x + i * NL < kVecs; }
-    __device__ __forceinline__ void init(const float* P, long ld, long rows, long r0, long k0) {
+    __device__ __forceinline__ void init(const T* P, long ld, long rows, long r0, long k0) {
         const int tid = threadIdx.x;
         step = KC ? KT : (long)KT * ld;
         shift = 0;
@@ -91,51 +170,45 @@ struct FastTile {
             else p[i] -= max(0, idx / kPer + 1 - kn) * ld;
         }
     }
-    __device__ __forceinline__ void load(v4f (&v)[kVPT], int i) const {
+    __device__ __forceinline__ void load(Q (&v)[kVPT], int i) const {
         if constexpr (THIN) {
             if (on(i)) v[i] = v4f{p[i][0], p[i][min(1, shift)], p[i][min(2, shift)], 0.0f};
         } else if (on(i)) {
-            const v4u t = *reinterpret_cast<const v4u*>(p[i]);
-            v[i] = v4f{t.x, t.y, t.z, t.w};
+            v[i] = El::load(p[i]);
         }
     }
     __device__ __forceinline__ void advance(long by) {
 #pragma unroll
         for (int i = 0; i < kVPT; i++) p[i] += by;
     }
-    __device__ __forceinline__ static v4f shifted(v4f v, int sh) {
-        if (sh & 1) v = v4f{v.y, v.z, v.w, 0.0f};
-        if (sh & 2) v = v4f{v.z, v.w, 0.0f, 0.0f};
-        if (sh & 4) v = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        return v;
-    }
-    __device__ __forceinline__ static void fix_k(v4f (&v)[kVPT], int kn) {
+    __device__ __forceinline__ static void fix_k(Q (&v)[kVPT], int kn) {
 #pragma unroll
         for (int i = 0; i < kVPT; i++) {
             const int idx = threadIdx.x + i * NL;
-            if constexpr (KC) v[i] = shifted(v[i], min(4, max(0, (idx % kPer) * 4 + 4 - kn)));
-            else v[i] = shifted(v[i], idx / kPer >= kn ? 4 : 0);
+            if constexpr (KC) v[i] = El::shifted(v[i], min(4, max(0, (idx % kPer) * 4 + 4 - kn)));
+            else v[i] = El::shifted(v[i], idx / kPer >= kn ? 4 : 0);
         }
     }
     // !KC, tiles past the last row: lanes that moved back to stay inside
     // the matrix put their rows where they belong
-    __device__ __forceinline__ void fix_rows(v4f (&v)[kVPT]) const {
+    __device__ __forceinline__ void fix_rows(Q (&v)[kVPT]) const {
 #pragma unroll
         for (int i = 0; i < kVPT; i++)
-            if constexpr (!THIN) v[i] = shifted(v[i], shift);
+            if constexpr (!THIN) v[i] = El::shifted(v[i], shift);
     }
-    __device__ __forceinline__ static void store(float* S, const v4f (&v)[kVPT], int i) {
+    __device__ __forceinline__ static void store(float* S, const Q (&q)[kVPT], int i) {
         const int idx = threadIdx.x + i * NL;
         if (!on(i)) return;
+        const v4f v = El::widen(q[i]);
         if constexpr (KC) {
             const int c = idx % kPer;
             float* s = S + (idx / kPer) * kStride + (c / 4) * 16 + c % 4;
-            s[0] = v[i].x;
-            s[4] = v[i].y;
-            s[8] = v[i].z;
-            s[12] = v[i].w;
+            s[0] = v.x;
+            s[4] = v.y;
+            s[8] = v.z;
+            s[12] = v.w;
         } else {
-            *reinterpret_cast<v4f*>(S + (idx / kPer) * kStride + (idx % kPer) * 4) = v[i];
+            *reinterpret_cast<v4f*>(S + (idx / kPer) * kStride + (idx % kPer) * 4) = v;
         }
     }
     // the lane's elements of steps 4 g .. 4 g + 3 (k = 16 g .. 16 g + 15)
@@ -166,29 +239,38 @@ struct FastGeom {
 };
 
 // alpha / beta, bias and activation of outputs (gm, gn .. gn + 3)
-template <bool FUSED>
-__device__ __forceinline__ void fast_epilogue(float* __restrict__ C, int M, int N, long gm, long gn, v4f acc,
+template <bool FUSED, class T>
+__device__ __forceinline__ void fast_epilogue(T* __restrict__ C, int M, int N, long gm, long gn, v4f acc,
                                               const FastGeom& g) {
     const int left = (int)min(4L, (long)N - gn);
     if (gm >= M || left <= 0) return;
-    float* cp = C + gm * N + gn;
+    T* cp = C + gm * N + gn;
     v4f v;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         // rac_kernels.hip:267-272
         v[r] = g.alpha * acc[r];
-        if (g.beta != 0.0f && r < left) v[r] = __builtin_fmaf(g.alpha, acc[r], g.beta * cp[r]);
+        if constexpr (!FUSED) {
+            if (g.beta != 0.0f && r < left) v[r] = __builtin_fmaf(g.alpha, acc[r], g.beta * cp[r]);
+        }
     }
     if constexpr (FUSED) {
         // rac_torch.cu:770-775
         if (g.ep.bias) {
+            const T* bp = reinterpret_cast<const T*>(g.ep.bias) + gn;
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                if (r < left) v[r] = v[r] + g.ep.bias[gn + r];
+                if (r < left) v[r] = v[r] + Elem<T>::get(bp + r);
         }
-        if (g.ep.pre) store4(g.ep.pre + gm * N + gn, v, left);
-        if (g.ep.act != kActNone) {
-            // one copy of the activation per tile: v rotates
+        if (g.ep.pre) Elem<float>::store(g.ep.pre + gm * N + gn, v, left);
+        if (g.ep.act == kActSilu && (g.iters == 24 || g.iters == 16)) {
+            // four interleaved exps (same bits): a quarter of the serial time
+            float x[4] = {v.x, v.y, v.z, v.w};
+            if (g.iters == 24) elt_vec<kEltSilu, 24, 4>(x, g.iters, g.ep.khinv);
+            else elt_vec<kEltSilu, 16, 4>(x, g.iters, g.ep.khinv);
+            v = v4f{x[0], x[1], x[2], x[3]};
+        } else if (g.ep.act != kActNone) {
+            // one copy of the activation: v rotates
 #pragma unroll 1
             for (int r = 0; r < 4; r++) {
                 const float x = act_rt(v.x, g.ep.act, g.iters, g.ep.khinv);
@@ -196,7 +278,7 @@ __device__ __forceinline__ void fast_epilogue(float* __restrict__ C, int M, int 
             }
         }
     }
-    store4(cp, v, left);
+    Elem<T>::store(cp, v, left);
 }
 
 // Output tile BM x BN, WR x WC waves, K-tiles of KT in two LDS buffers, PD
@@ -206,14 +288,13 @@ __device__ __forceinline__ void fast_epilogue(float* __restrict__ C, int M, int 
 // between them, 2 between them with the order held by scheduling barriers
 // (a lone wave per SIMD issues them in the shadow of its matrix
 // instructions: 32x4096x4096 on 32x32 tiles 34.7 -> 24.9 us).
-template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD, bool THIN>
-__global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const float* __restrict__ A,
-                                                                 const float* __restrict__ B, float* __restrict__ C,
-                                                                 FastGeom g)
+template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD, bool THIN, class T>
+__global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const T* __restrict__ A, const T* __restrict__ B,
+                                                                 T* __restrict__ C, FastGeom g)
 {
     constexpr int NL = 64 * WR * WC;
-    using TAt = FastTile<!TA, BM, KT, NL, TA && THIN && BM == 16>;
-    using TBt = FastTile<TB, BN, KT, NL, !TB && THIN && BN == 16>;
+    using TAt = FastTile<T, !TA, BM, KT, NL, TA && THIN && BM == 16>;
+    using TBt = FastTile<T, TB, BN, KT, NL, !TB && THIN && BN == 16>;
     constexpr int TM = BM / WR, TN = BN / WC, MT = TM / 16, NT = TN / 16;
     __shared__ __attribute__((aligned(16))) float sA[2][TAt::kFloats];
     __shared__ __attribute__((aligned(16))) float sB[2][TBt::kFloats];
@@ -284,7 +365,8 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const float* __
     ta.init(A, lda, M, m0, kbeg);
     tb.init(B, ldb, N, n0, kbeg);
     constexpr int VA = TAt::kVPT, VB = TBt::kVPT;
-    v4f va[PD][VA], vb[PD][VB];
+    typename TAt::Q va[PD][VA];
+    typename TBt::Q vb[PD][VB];
     const int kn = kend - kbeg, nfull = kn / KT, tail = kn - nfull * KT, nst = nfull + (tail ? 1 : 0);
     const bool edge_a = TA && m0 + BM > M, edge_b = !TB && n0 + BN > N;
     // before K-tile s is loaded / after (tiles past the last reload it: the
@@ -393,15 +475,26 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const float* __
 
     // the operands are passed B first, so a lane holds four consecutive
     // columns of one row: n = 4 (lane / 16) + r, m = lane % 16 of each tile
+    const long em = m0 + wm + lane % 16, en = n0 + wn + 4 * (lane / 16);
+    if constexpr (FUSED) {
+        // one copy of the epilogue: the accumulators rotate through it
+#pragma unroll 1
+        for (int i = 0; i < MT * NT; i++) {
+            const v4f x = acc[0][0];
+            fast_epilogue<true>(C, M, N, em + 16 * (i / NT), en + 16 * (i % NT), x, g);
 #pragma unroll
-    for (int i = 0; i < MT; i++)
+            for (int j = 0; j + 1 < MT * NT; j++) acc[j / NT][j % NT] = acc[(j + 1) / NT][(j + 1) % NT];
+        }
+    } else {
 #pragma unroll
-        for (int j = 0; j < NT; j++)
-            fast_epilogue<FUSED>(C, M, N, m0 + wm + 16 * i + lane % 16, n0 + wn + 16 * j + 4 * (lane / 16), acc[i][j],
-                                 g);
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) fast_epilogue<false>(C, M, N, em + 16 * i, en + 16 * j, acc[i][j], g);
+    }
 }
 
-template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD, bool THIN = false>
+template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD, bool THIN = false,
+          class T = float>
 static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
     FastGeom g{a.M, a.N, a.K, a.sa, a.sb, a.sc, a.alpha, a.beta, a.iters, a.ep, a.k_causal, a.k_causal ? a.k_side : 0,
                a.row0, 0, (a.M + BM - 1) / BM, a.batch, 0};
@@ -413,9 +506,9 @@ static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
     g.total = (long)g.tiles * g.batch;
     // a grid dimension holds fewer than 2^32 lanes
     const long gx = g.total < (1L << 22) ? g.total : (1L << 22);
-    hipLaunchKernelGGL((gemm_fast_kernel<TA, TB, FUSED, TRAP, BM, BN, WR, WC, KT, PD, SPREAD, THIN>),
-                       dim3((unsigned)gx, (unsigned)((g.total + gx - 1) / gx)), dim3(64 * WR * WC), 0, s, a.A, a.B,
-                       a.C, g);
+    hipLaunchKernelGGL((gemm_fast_kernel<TA, TB, FUSED, TRAP, BM, BN, WR, WC, KT, PD, SPREAD, THIN, T>),
+                       dim3((unsigned)gx, (unsigned)((g.total + gx - 1) / gx)), dim3(64 * WR * WC), 0, s,
+                       reinterpret_cast<const T*>(a.A), reinterpret_cast<const T*>(a.B), reinterpret_cast<T*>(a.C), g);
     return hipGetLastError();
 }
 
@@ -434,11 +527,11 @@ static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
 // needs at least the longest tile's time: 32 x 2048 x 128 x 2048 150 us on
 // 64x64 (64x128 159, 128x128 162, 32x64 227), 8 x 1000 x 64 x 1000 15.5 us
 // on 32x64 (64x64 22).
-template <bool TA, bool TB, bool FUSED, bool TRAP>
+template <bool TA, bool TB, bool FUSED, bool TRAP, class T = float>
 static hipError_t fast_tile(const GemmArgs& a, hipStream_t s) {
     struct Shape { int bm, bn; double eff, eff_causal; };
-    constexpr Shape shapes[5] = {{128, 128, 0.93, 0.80}, {64, 128, 0.91, 0.85}, {64, 64, 0.83, 0.88},
-                                 {32, 64, 0.81, 0.70}, {32, 32, 0.76, 0.65}};
+    constexpr Shape shapes[5] = {{128, 128, 0.93, 0.80}, {64, 128, 0.91, 0.85}, {64, 64, 0.85, 0.88},
+                                 {32, 64, 0.82, 0.70}, {32, 32, 0.78, 0.65}};
     const long cus = device_cus();
     const bool causal_k = a.k_causal && (a.k_side == 1 || a.k_side == 2);
     int best = 0;
@@ -460,20 +553,22 @@ static hipError_t fast_tile(const GemmArgs& a, hipStream_t s) {
         }
     }
     constexpr bool KC2 = !TA && TB, KC0 = TA && !TB;      // both / neither operand k-contiguous
+#define RAC_FAST(...) return fast_launch<TA, TB, FUSED, TRAP, __VA_ARGS__, false, T>(a, s)
     switch (best) {
     case 0:
-        if constexpr (KC2) return fast_launch<TA, TB, FUSED, TRAP, 128, 128, 2, 4, 16, 1, 0>(a, s);
-        else if constexpr (KC0) return fast_launch<TA, TB, FUSED, TRAP, 128, 128, 2, 4, 32, 1, 0>(a, s);
-        else return fast_launch<TA, TB, FUSED, TRAP, 128, 128, 2, 2, 16, 1, 0>(a, s);
+        if constexpr (KC2) RAC_FAST(128, 128, 2, 4, 16, 1, 0);
+        else if constexpr (KC0) RAC_FAST(128, 128, 2, 4, 32, 1, 0);
+        else RAC_FAST(128, 128, 2, 2, 16, 1, 0);
     case 1:
-        if constexpr (KC0) return fast_launch<TA, TB, FUSED, TRAP, 64, 64, 2, 2, 32, 1, 1>(a, s);
-        else return fast_launch<TA, TB, FUSED, TRAP, 64, 128, 2, 2, 16, 1, 1>(a, s);
+        if constexpr (KC0) RAC_FAST(64, 64, 2, 2, 32, 1, 1);
+        else RAC_FAST(64, 128, 2, 2, 16, 1, 1);
     case 2:
-        if constexpr (KC0) return fast_launch<TA, TB, FUSED, TRAP, 64, 64, 2, 2, 32, 1, 1>(a, s);
-        else return fast_launch<TA, TB, FUSED, TRAP, 64, 64, 2, 4, 64, 2, 2>(a, s);
-    case 3: return fast_launch<TA, TB, FUSED, TRAP, 32, 64, 2, 2, 64, 2, 2>(a, s);
-    default: return fast_launch<TA, TB, FUSED, TRAP, 32, 32, 2, 2, 64, 2, 2>(a, s);
+        if constexpr (KC0) RAC_FAST(64, 64, 2, 2, 32, 1, 1);
+        else RAC_FAST(64, 64, 2, 2, 64, 1, 2);
+    case 3: RAC_FAST(32, 64, 2, 2, 64, 2, 2);
+    default: RAC_FAST(32, 32, 2, 2, 64, 2, 2);
     }
+#undef RAC_FAST
 }
 
 // At most 16 rows (decode-time linears) or columns: one 16 x 16 block of
@@ -484,32 +579,38 @@ static hipError_t fast_tile(const GemmArgs& a, hipStream_t s) {
 // against 95.3 us; 1 x 11008 x 4096, 172 blocks: 31.5 against 27.8); pairs
 // of waves where those still fit one to a CU (4096 columns: 23.4 against
 // 26.9 us; 11008, 344 blocks: 39.6, a second pair shares the first's SIMDs).
-template <bool TA, bool TB, bool FUSED>
+template <bool TA, bool TB, bool FUSED, class T = float>
 static hipError_t fast_few(const GemmArgs& a, hipStream_t s) {
     const long cus = device_cus();
     const bool rows = a.M <= 16;
     const long n = rows ? a.N : a.M, b4 = (n + 63) / 64 * a.batch, b2 = (n + 31) / 32 * a.batch;
+#define RAC_FAST(...) return fast_launch<TA, TB, FUSED, false, __VA_ARGS__, T>(a, s)
     // fewer than 4 rows stored side by side (1 is a vector, read as k-contiguous)
     if constexpr (TA) {
-        if (a.M < 4) return fast_launch<TA, TB, FUSED, false, 16, 64, 1, 4, 64, 2, 2, true>(a, s);
+        if (a.M < 4) RAC_FAST(16, 64, 1, 4, 64, 2, 2, true);
     }
     if constexpr (!TB) {
-        if (a.N < 4) return fast_launch<TA, TB, FUSED, false, 64, 16, 4, 1, 64, 2, 2, true>(a, s);
+        if (a.N < 4) RAC_FAST(64, 16, 4, 1, 64, 2, 2, true);
     }
     if (rows) {
-        if (b2 <= cus) return fast_launch<TA, TB, FUSED, false, 16, 32, 1, 2, 128, 1, 2>(a, s);
-        if (b4 <= cus) return fast_launch<TA, TB, FUSED, false, 16, 64, 1, 4, 64, 2, 2>(a, s);
-        return fast_launch<TA, TB, FUSED, false, 16, 64, 1, 4, 128, 1, 2>(a, s);
+        if (b2 <= cus) RAC_FAST(16, 32, 1, 2, 128, 1, 2, false);
+        if (b4 <= cus) RAC_FAST(16, 64, 1, 4, 64, 2, 2, false);
+        RAC_FAST(16, 64, 1, 4, 128, 1, 2, false);
     }
-    if (b2 <= cus) return fast_launch<TA, TB, FUSED, false, 32, 16, 2, 1, 128, 1, 2>(a, s);
-    if (b4 <= cus) return fast_launch<TA, TB, FUSED, false, 64, 16, 4, 1, 64, 2, 2>(a, s);
-    return fast_launch<TA, TB, FUSED, false, 64, 16, 4, 1, 128, 1, 2>(a, s);
+    if (b2 <= cus) RAC_FAST(32, 16, 2, 1, 128, 1, 2, false);
+    if (b4 <= cus) RAC_FAST(64, 16, 4, 1, 64, 2, 2, false);
+    RAC_FAST(64, 16, 4, 1, 128, 1, 2, false);
+#undef RAC_FAST
 }
 
-template <bool TA, bool TB, bool FUSED>
+template <bool TA, bool TB, bool FUSED, class T = float>
 static hipError_t fast_shape(const GemmArgs& a, hipStream_t s) {
-    if (a.M <= 16 || a.N <= 16) return fast_few<TA, TB, FUSED>(a, s);
-    return fast_tile<TA, TB, FUSED, false>(a, s);
+    if (a.M <= 16 || a.N <= 16) return fast_few<TA, TB, FUSED, T>(a, s);
+    return fast_tile<TA, TB, FUSED, false, T>(a, s);
+}
+
+hipError_t gemm_fast_half_launch(int dtype, const GemmArgs& g, hipStream_t s) {
+    return dtype == 1 ? fast_shape<false, true, true, Bf16>(g, s) : fast_shape<false, true, true, F16>(g, s);
 }
 
 hipError_t gemm_fast_launch(int ta, int tb, const GemmArgs& g, hipStream_t s) {

@@ -34,6 +34,10 @@ struct GemmEpilogue {
 // C[M,N] = act(A[M,K] W[N,K]^T + bias) in one launch.
 hipError_t gemm_fused_launch(const float* A, const float* W, float* C, int M, int N, int K,
                              const GemmEpilogue& ep, int iters, int mode, hipStream_t s);
+// The same in FAST mode with input, weight, bias (may be null) and output in
+// bf16 (dtype 1) or fp16 (2), computed in fp32; K >= 4.
+hipError_t gemm_fused_half_launch(const void* A, const void* W, const void* bias, void* C, int M, int N, int K,
+                                  const GemmEpilogue& ep, int iters, int dtype, hipStream_t s);
 // d[i] = g[i] * act'(pre[i]) (rac_torch.cu:680-694).
 hipError_t act_grad_launch(const float* g, const float* pre, float* d, long count, int act, int iters,
                            hipStream_t s);

@@ -116,6 +116,40 @@ def _fused(x2: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out:
           "rac_fused_linear_dev")
 
 
+_HALF = {torch.bfloat16: 1, torch.float16: 2}
+
+
+def _fused_half(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], act: int, iters: int,
+                mode: int, want_pre: bool):
+    """The fused linear layer on bf16 / fp16 tensors as they are (FAST mode):
+    (out, pre) as widening them, the fp32 layer and casting its output back
+    give, or None where that form does not apply (mixed types, another MAC,
+    nothing to compute, fewer than 4 input features)."""
+    iters, mode = _resolve(iters, mode)
+    dt = _HALF.get(input.dtype)
+    has_bias = bias is not None and bias.numel() > 0
+    if (dt is None or mode != MODE_FAST or weight.dtype != input.dtype or not weight.is_cuda or weight.dim() != 2
+            or weight.size(1) < 4 or (has_bias and (bias.dtype != input.dtype or not bias.is_cuda))):
+        return None
+    out_features, in_features = weight.shape
+    if input.dim() == 0 or input.size(-1) != in_features or input.numel() == 0 or out_features == 0:
+        return None
+    if has_bias and bias.numel() != out_features:
+        return None
+    x2 = input.reshape(-1, in_features).contiguous()
+    w = weight.contiguous()
+    b = bias.contiguous() if has_bias else None
+    shape = list(input.shape)
+    shape[-1] = out_features
+    out = torch.empty(shape, device=x2.device, dtype=input.dtype)
+    pre = torch.empty(shape, device=x2.device, dtype=torch.float32) if want_pre else None
+    check(_lib.load().rac_fused_linear_half_dev(x2.data_ptr(), w.data_ptr(), b.data_ptr() if b is not None else None,
+                                                out.data_ptr(), pre.data_ptr() if pre is not None else None,
+                                                x2.size(0), out_features, in_features, act, iters, dt, _stream(out)),
+          "rac_fused_linear_half_dev")
+    return out, pre
+
+
 # ── reference surface (rac_torch_bind.cpp:68-199) ─────────────────────────
 
 def matmul_forward(A: torch.Tensor, B: torch.Tensor, iters: int = 0, mode: int = -1) -> torch.Tensor:
@@ -169,6 +203,9 @@ def linear_forward(input: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor
     _require_gpu(input, "input")
     orig_dtype = input.dtype
     if orig_dtype != torch.float32:
+        half = _fused_half(input, weight, bias, 0, iters, mode, False)
+        if half is not None:
+            return half[0]
         input = input.to(torch.float32)
         weight = weight.to(torch.float32)
         if bias is not None and bias.numel() > 0:
@@ -237,6 +274,9 @@ def fused_linear_forward(input: torch.Tensor, weight: torch.Tensor, bias: torch.
         raise RuntimeError("RAC: act must be 0(none), 1(relu), 2(gelu), 3(silu)")
     orig_dtype = input.dtype
     if orig_dtype != torch.float32:
+        half = _fused_half(input, weight, bias, int(act), iters, mode, return_pre)
+        if half is not None:
+            return half if return_pre else half[0]
         input = input.to(torch.float32)
         weight = weight.to(torch.float32)
         if bias is not None and bias.numel() > 0:
