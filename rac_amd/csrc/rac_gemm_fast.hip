@@ -516,7 +516,9 @@ static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
 // CU.  A CU works through BM x BN x K MACs of a tile at 128 per cycle times
 // the share `eff` of that rate which the tile sustains, and the fullest CU
 // has ceil(tiles / CUs) of them: large tiles reuse operands best but leave
-// CUs idle in the last round.  eff and the shapes inside a tile size are
+// CUs idle in the last round.  A CU that holds a single tile has nothing to
+// run while that waits (`eff_alone`; 301 x 5632 x 2048 NT: 220 tiles of 64x128
+// 86 us, 1760 of 32x32 68).  eff and the shapes inside a tile size are
 // measured (K 1000-11008, all layouts): e.g. 2048 x 11008 x 4096 NT 1.39 ms
 // on 64x128 (128x128: 1.47, 64x64: 1.46), 500 x 2048 x 5632 NT 99 us on
 // 64x64 (32x64: 101, 32x32: 105), 128 x 11008 x 4096 NT 107 us on 32x64
@@ -529,9 +531,9 @@ static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
 // on 32x64 (64x64 22).
 template <bool TA, bool TB, bool FUSED, bool TRAP, class T = float>
 static hipError_t fast_tile(const GemmArgs& a, hipStream_t s) {
-    struct Shape { int bm, bn; double eff, eff_causal; };
-    constexpr Shape shapes[5] = {{128, 128, 0.93, 0.80}, {64, 128, 0.91, 0.85}, {64, 64, 0.85, 0.88},
-                                 {32, 64, 0.82, 0.70}, {32, 32, 0.78, 0.65}};
+    struct Shape { int bm, bn; double eff, eff_alone, eff_causal; };
+    constexpr Shape shapes[5] = {{128, 128, 0.93, 0.75, 0.80}, {64, 128, 0.91, 0.68, 0.85}, {64, 64, 0.85, 0.83, 0.88},
+                                 {32, 64, 0.82, 0.70, 0.70}, {32, 32, 0.78, 0.65, 0.65}};
     const long cus = device_cus();
     const bool causal_k = a.k_causal && (a.k_side == 1 || a.k_side == 2);
     int best = 0;
@@ -545,7 +547,8 @@ static hipError_t fast_tile(const GemmArgs& a, hipStream_t s) {
         }
         t *= a.batch;
         const double work = (double)bm * bn;
-        double cost = (double)((t + cus - 1) / cus) * work / (i == 0 && a.K < 512 ? 0.80 : shapes[i].eff);
+        const double eff = t <= cus ? shapes[i].eff_alone : i == 0 && a.K < 512 ? 0.80 : shapes[i].eff;
+        double cost = (double)((t + cus - 1) / cus) * work / eff;
         if (causal_k) cost = std::max(0.5 * t / cus, 1.0) * work / shapes[i].eff_causal;
         if (i == 0 || cost < best_cost) {
             best = i;
