@@ -40,6 +40,15 @@ int rac_decode_attention_dev(const float *q, const float *k_cache, const float *
                              int n_heads, int n_kv_heads, int d_head, long t_cap, const int *pos,
                              float scale, int iters, void *stream);
 
+/* Causal attention of T new tokens (a prompt) over the cache: q [n_kv_heads,
+ * rep * T, d_head] with row r * T + t of group g holding head g * rep + r,
+ * token t at position start + t; out in the same layout; FAST products.
+ * workspace: n_kv_heads * rep * T * (start + T) floats.  At most 16777215
+ * query rows. */
+int rac_prefill_attention_dev(const float *q, const float *k_cache, const float *v_cache, float *out,
+                              float *workspace, int n_kv_heads, int rep, int T, int start, int d_head,
+                              long t_cap, float scale, int iters, void *stream);
+
 /* kv = [k (n_kv_heads * d_head) | v (n_kv_heads * d_head)] of the new token
  * written at position *pos of every head (:569-574); nothing is written
  * for a position outside [0, t_cap). */

@@ -97,6 +97,7 @@ _SIGNATURES = {
                                         _i, _vp]),
     # rac_decode.h — decode step pieces, cache position in device memory
     "rac_decode_attention_dev": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _l, _vp, _f, _i, _vp]),
+    "rac_prefill_attention_dev": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _l, _f, _i, _vp]),
     "rac_kv_append_dev": (_i, [_vp, _vp, _vp, _i, _i, _l, _vp, _vp]),
     "rac_position_advance_dev": (_i, [_vp, _i, _vp]),
     "rac_swiglu_dev": (_i, [_vp, _vp, _l, _i, _vp]),

@@ -490,6 +490,40 @@ RAC_EXPORT int rac_decode_attention_dev(const float* q, const float* k_cache, co
                      "rac_decode_attention_dev launch");
 }
 
+// Causal grouped-query attention of T new tokens over a cache
+// (bench_rac_transformer.c:508-548): row r T + t of key / value head g's
+// queries is head g rep + r, token t, at position start + t; keys and values
+// 0 .. start + T - 1 of the caches [n_kv_heads, t_cap, d_head].  FAST products
+// around the row softmax: score tiles past the diagonal are not computed, and
+// the softmax reads and exponentiates only what is not masked.
+RAC_EXPORT int rac_prefill_attention_dev(const float* q, const float* k_cache, const float* v_cache, float* out,
+                                         float* workspace, int n_kv_heads, int rep, int T, int start, int d_head,
+                                         long t_cap, float scale, int iters, void* stream) {
+    if (!q || !k_cache || !v_cache || !out || !workspace)
+        return fail(RAC_ERR_NULL_PTR, "rac_prefill_attention_dev: null buffer");
+    if (n_kv_heads <= 0 || rep <= 0 || T <= 0 || start < 0 || d_head <= 0 || (long)start + T > t_cap)
+        return fail(RAC_ERR_INVALID_DIM, "rac_prefill_attention_dev: bad sizes");
+    const long rows = (long)rep * T, total = (long)start + T;
+    if (n_kv_heads > 65535 || rows * n_kv_heads > 16777215L || total > 2147483647L / 16)
+        return fail(RAC_ERR_INVALID_DIM, "rac_prefill_attention_dev: too many query rows or positions");
+    const hipStream_t s = (hipStream_t)stream;
+    int rc = check_hip(gemm_launch(0, 1, q, k_cache, workspace, (int)rows, (int)total, d_head, scale, 0.0f, iters,
+                                   kModeFast, s, n_kv_heads, rows * d_head, t_cap * d_head, rows * total, 0, nullptr,
+                                   true, start, 3, T),
+                       "rac_prefill_attention scores launch");
+    if (rc) return rc;
+    SoftmaxMask mk;
+    mk.causal = 1;
+    mk.seq = T;
+    mk.row0 = start;
+    rc = check_hip(softmax_launch(workspace, workspace, rows * n_kv_heads, total, iters, s, mk),
+                   "rac_prefill_attention softmax launch");
+    if (rc) return rc;
+    return check_hip(gemm_launch(0, 0, workspace, v_cache, out, (int)rows, d_head, (int)total, 1.0f, 0.0f, iters,
+                                 kModeFast, s, n_kv_heads, rows * total, t_cap * d_head, rows * d_head),
+                     "rac_prefill_attention output launch");
+}
+
 // The new token's keys and values into the cache at *pos
 // (bench_rac_transformer.c:569-574).
 RAC_EXPORT int rac_kv_append_dev(const float* kv, float* k_cache, float* v_cache, int n_kv_heads, int d_head,
@@ -1054,7 +1088,7 @@ RAC_EXPORT int rac_attention_backward_dev(const float* q, const float* k, const 
                    "rac_attention_backward dV launch");
     if (rc || (!dq && !dk)) return rc;
     rc = check_hip(gemm_launch(0, 1, grad_out + off, v, workspace, c, t, d, 1.0f, 0.0f, iters, mode, s, bh, td, td, ct,
-                               0, flag, true, row0, 3),
+                               0, flag, true, row0, flag ? 3 : 0),
                    "rac_attention_backward dP launch");
     if (rc) return rc;
     rc = check_hip(attn_dscore_launch(P, workspace, (long)bh * c, t, c, row0, flag, s),

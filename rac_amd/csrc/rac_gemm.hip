@@ -535,15 +535,15 @@ static hipError_t dispatch(int ta, int tb, int mode, const GemmArgs& g, hipStrea
 hipError_t gemm_launch(int ta, int tb, const float* A, const float* B, float* C,
                        int M, int N, int K, float alpha, float beta, int iters, int mode,
                        hipStream_t s, int batch, long sa, long sb, long sc, int sched,
-                       const int* k_causal, bool exact_specials, int row0, int k_side) {
+                       const int* k_causal, bool exact_specials, int row0, int k_side, int period) {
     const GemmArgs g{A, B, C, M, N, K, alpha, beta, clamp_iters(iters), batch, sa, sb, sc,
-                     GemmEpilogue(), false, sched, k_causal, exact_specials ? 1 : 0, row0, k_side};
+                     GemmEpilogue(), false, sched, k_causal, exact_specials ? 1 : 0, row0, k_side, period};
     return dispatch(ta, tb, mode, g, s);
 }
 
 hipError_t gemm_fused_launch(const float* A, const float* W, float* C, int M, int N, int K,
                              const GemmEpilogue& ep, int iters, int mode, hipStream_t s) {
-    const GemmArgs g{A, W, C, M, N, K, 1.0f, 0.0f, clamp_iters(iters), 1, 0, 0, 0, ep, true, 0, nullptr, 1, 0, 0};
+    const GemmArgs g{A, W, C, M, N, K, 1.0f, 0.0f, clamp_iters(iters), 1, 0, 0, 0, ep, true, 0, nullptr, 1, 0, 0, 0};
     return dispatch(0, 1, mode, g, s);
 }
 
@@ -552,7 +552,7 @@ hipError_t gemm_fused_half_launch(const void* A, const void* W, const void* bias
     GemmEpilogue e = ep;
     e.bias = static_cast<const float*>(bias);                  // of the operands' type
     const GemmArgs g{static_cast<const float*>(A), static_cast<const float*>(W), static_cast<float*>(C), M, N, K, 1.0f,
-                     0.0f, clamp_iters(iters), 1, 0, 0, 0, e, true, 0, nullptr, 1, 0, 0};
+                     0.0f, clamp_iters(iters), 1, 0, 0, 0, e, true, 0, nullptr, 1, 0, 0, 0};
     return gemm_fast_half_launch(dtype, g, s);
 }
 

@@ -25,8 +25,9 @@ struct GemmArgs {
     // row0 + m*BM + BM - 1 (P V); 2, only from k = m*BM - row0 on (P^T dO: row
     // s of P^T is 0 before query position s, k = 0 being position row0); 3,
     // tiles wholly above the diagonal are left unwritten (dO V^T, rows from
-    // query position row0).  2 and 3 in FAST mode only.
+    // query position row0; without k_causal too).  2 and 3 in FAST mode only.
     int k_side;
+    int period;      // k_side 3: row m is at query position row0 + m % period (0: row0 + m)
 };
 
 // Column tiles of row tile r in a causal score trapezoid (query rows

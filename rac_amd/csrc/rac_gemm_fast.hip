@@ -232,7 +232,7 @@ struct FastGeom {
     GemmEpilogue ep;
     const int* k_causal;
     int k_side;           // 0: every k; 1-3: the causal limits of GemmArgs, when *k_causal holds 1
-    int row0;
+    int row0, period;
     int tiles, tiles_m;   // output tiles of one batch item, rows of them
     int batch;
     long total;           // tiles * batch
@@ -342,9 +342,14 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const T* __rest
     C += z * g.sc;
     int kbeg = 0, kend = g.K;
     bool any_k = true;
-    if (g.k_side && *g.k_causal == 1) {
+    if (g.k_side && (!g.k_causal || *g.k_causal == 1)) {
         if (g.k_side == 1) kend = (int)min((long)g.K, (long)g.row0 + m0 + BM);
-        else if (g.k_side == 3 && n0 > (long)g.row0 + m0 + BM - 1) return;
+        else if (g.k_side == 3) {
+            // the tile's last query position
+            long last = m0 + BM - 1;
+            if (g.period) last = m0 / g.period == last / g.period ? last % g.period : g.period - 1;
+            if (n0 > g.row0 + last) return;
+        }
         else if (g.k_side == 2) {
             kbeg = (int)min((long)g.K - 4, max(0L, m0 - g.row0));
             any_k = m0 - g.row0 < g.K;
@@ -496,8 +501,8 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const T* __rest
 template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD, bool THIN = false,
           class T = float>
 static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
-    FastGeom g{a.M, a.N, a.K, a.sa, a.sb, a.sc, a.alpha, a.beta, a.iters, a.ep, a.k_causal, a.k_causal ? a.k_side : 0,
-               a.row0, 0, (a.M + BM - 1) / BM, a.batch, 0};
+    FastGeom g{a.M, a.N, a.K, a.sa, a.sb, a.sc, a.alpha, a.beta, a.iters, a.ep, a.k_causal, a.k_causal || a.k_side == 3 ? a.k_side : 0,
+               a.row0, a.period, 0, (a.M + BM - 1) / BM, a.batch, 0};
     if constexpr (TRAP) {
         for (int r = 0; r < g.tiles_m; r++) g.tiles += trap_cols(g.row0, r, BM, BN, g.N);
     } else {
@@ -532,7 +537,7 @@ static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
 template <bool TA, bool TB, bool FUSED, bool TRAP, class T = float>
 static hipError_t fast_tile(const GemmArgs& a, hipStream_t s) {
     struct Shape { int bm, bn; double eff, eff_alone, eff_causal; };
-    constexpr Shape shapes[5] = {{128, 128, 0.93, 0.75, 0.80}, {64, 128, 0.91, 0.68, 0.85}, {64, 64, 0.85, 0.83, 0.88},
+    constexpr Shape shapes[5] = {{128, 128, 0.93, 0.75, 0.80}, {64, 128, 0.91, 0.68, 0.85}, {64, 64, 0.87, 0.83, 0.88},
                                  {32, 64, 0.82, 0.70, 0.70}, {32, 32, 0.78, 0.65, 0.65}};
     const long cus = device_cus();
     const bool causal_k = a.k_causal && (a.k_side == 1 || a.k_side == 2);

@@ -86,7 +86,7 @@ hipError_t gemm_launch(int ta, int tb, const float* A, const float* B, float* C,
                        int M, int N, int K, float alpha, float beta, int iters, int mode,
                        hipStream_t s, int batch = 1, long sa = 0, long sb = 0, long sc = 0,
                        int sched = 0, const int* k_causal = nullptr, bool exact_specials = true,
-                       int row0 = 0, int k_side = 1);
+                       int row0 = 0, int k_side = 1, int period = 0);
 // *flag = 1 if every x[i] is finite, else 0 (stream-ordered).
 hipError_t all_finite_launch(const float* x, long n, int* flag, hipStream_t s);
 // *flag = 1 if every element of the four arrays is below 2^58 in magnitude,

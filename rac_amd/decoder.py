@@ -152,14 +152,24 @@ class RACDecoder:
         cfg = self.cfg
         nkv, dh = cfg.n_kv_heads, cfg.d_head
         rep = cfg.n_heads // nkv
-        total = start + T
         # query rows of head group g: row r * T + t is head g * rep + r, token t
-        qg = q.view(T, nkv, rep, dh).permute(1, 2, 0, 3).reshape(nkv, rep * T, dh)
+        qg = q.unflatten(1, (nkv, rep, dh)).permute(1, 2, 0, 3).reshape(nkv, rep * T, dh).contiguous()
+        if nkv > 65535 or nkv * rep * T > 16777215:
+            return self._prefill_attention_composed(L, qg, start, T)
+        o = ext.prefill_attention(qg, self.k_cache[L], self.v_cache[L], T, start, self.scale, self.iters)
+        return o.view(nkv, rep, T, dh).permute(2, 0, 1, 3).reshape(T, cfg.d_model)
+
+    def _prefill_attention_composed(self, L: int, qg: torch.Tensor, start: int, T: int) -> torch.Tensor:
+        """The same stage by stage, for more query rows than one launch takes."""
+        cfg = self.cfg
+        nkv, dh = cfg.n_kv_heads, cfg.d_head
+        rep = cfg.n_heads // nkv
+        total = start + T
         kc = self.k_cache[L][:, :total, :]
         vc = self.v_cache[L][:, :total, :]
         s = ext.bmm(qg, kc, trans_b=True, alpha=self.scale, iters=self.iters, mode=ext.MODE_FAST)
-        t = torch.arange(T, device=q.device).repeat(rep).view(rep * T, 1)
-        j = torch.arange(total, device=q.device).view(1, total)
+        t = torch.arange(T, device=qg.device).repeat(rep).view(rep * T, 1)
+        j = torch.arange(total, device=qg.device).view(1, total)
         s.masked_fill_(j > start + t, float("-inf"))
         p = ext.softmax(s.view(nkv * rep * T, total), self.iters).view(nkv, rep * T, total)
         o = ext.bmm(p, vc, iters=self.iters, mode=ext.MODE_FAST)          # [nkv, rep * T, dh]
@@ -174,7 +184,7 @@ class RACDecoder:
         qkv = self._linear(h, w["qkv"])                                    # [T, d + 2 nkv dh]
         self.k_cache[L][:, start:start + T, :] = qkv[:, d:d + nkv * dh].reshape(T, nkv, dh).transpose(0, 1)
         self.v_cache[L][:, start:start + T, :] = qkv[:, d + nkv * dh:].reshape(T, nkv, dh).transpose(0, 1)
-        att = self._prefill_attention(L, qkv[:, :d].contiguous(), start, T)
+        att = self._prefill_attention(L, qkv[:, :d], start, T)
         x = x + self._linear(att, w["o"])
         h = ext.rmsnorm(x, lw.rms_ffn, cfg.eps)
         f = self._linear(h, w["g"], 3) * self._linear(h, w["u"])             # silu(gate) * up

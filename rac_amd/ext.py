@@ -929,6 +929,25 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     return out
 
 
+def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, T: int, start: int, scale: float,
+                      iters: int = 0) -> torch.Tensor:
+    """Causal attention of T new tokens at positions start .. start + T - 1
+    over the cache (bench_rac_transformer.c:508-548): q [n_kv_heads, rep * T,
+    d_head], row r * T + t of group g holding head g * rep + r, token t.
+    Returns the same layout."""
+    _require_f32(q, "q")
+    nkv, t_cap, dh = _require_cache(k_cache, v_cache)
+    if q.dim() != 3 or not q.is_contiguous() or q.size(0) != nkv or q.size(2) != dh or T <= 0 or q.size(1) % T:
+        raise RuntimeError("RAC: q must be a contiguous [n_kv_heads, rep * T, d_head] tensor")
+    out = torch.empty_like(q)
+    ws = torch.empty(q.size(0) * q.size(1) * (start + T), device=q.device, dtype=torch.float32)
+    check(_lib.load().rac_prefill_attention_dev(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
+                                                ws.data_ptr(), nkv, q.size(1) // T, int(T), int(start), dh, t_cap,
+                                                float(scale), _resolve_iters(iters), _stream(q)),
+          "rac_prefill_attention_dev")
+    return out
+
+
 def kv_append_(kv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pos: torch.Tensor) -> None:
     """Writes kv = [k | v] (2 * n_kv_heads * d_head values, contiguous) at
     cache position pos (read on the device)."""
