@@ -1,22 +1,21 @@
 // rac_rowops.hip — row-wise softmax (hyperbolic-CORDIC exp), RMSNorm and
 // LayerNorm (CORDIC-vectoring rsqrt) for gfx950.
 //
-// One 256-lane workgroup (4 wave64) per row.  When the row length is a
-// multiple of 4 and the row fits in registers (<= 16 float4 per lane), the
-// row is read from HBM exactly once into registers with 16-byte loads, the
-// reductions run as wave64 butterflies (ds_swizzle/DPP via __shfl_xor) plus a
-// 4-entry LDS exchange, and the result is written once: 1 read + 1 write per
-// element, the HBM minimum.  Other shapes take a strided loop that re-reads
-// the row (from L2 for rows up to a few MB).
+// A row that fits in registers (64 values per lane) is read from HBM exactly
+// once, reduced and written once: 1 read + 1 write per element, the HBM
+// minimum.  Longer rows take a strided loop that re-reads the row (from L2
+// for rows up to a few MB).  RowLayout says which lane holds what: 16-byte
+// groups where the row length and the pointers allow it, else single values,
+// and a workgroup (4 wave64, a 4-entry LDS exchange) or one wave per row.
 //
 // Arithmetic follows rac_cpu.c:258-271 (softmax), :548-574 (RMSNorm) and
 // :507-546 (LayerNorm) rounding for rounding, except the order of the row
-// sums: each lane adds its own values in order (the register path's lane l
-// holds the float4 groups l, l + 256, ...; the strided loop's, the elements
-// l, l + 256, ...), lanes combine by a wave64 XOR butterfly (offsets 32 ..
-// 1) and the four wave partials in order, instead of one left-to-right sum
-// (differences O(1e-7) relative).  That order is fixed, so results do not
-// depend on scheduling and a CPU model of it matches bit for bit.
+// sums: lane l of 256 adds the float4 groups l, l + 256, ... in order (where a
+// row cannot be read in float4 groups, the elements l, l + 256, ...), lanes
+// combine by a wave64 XOR butterfly (offsets 32 .. 1) and the four wave
+// partials in order, instead of one left-to-right sum (differences O(1e-7)
+// relative).  That order is fixed, whichever layout or loop ran, so results
+// do not depend on scheduling and a CPU model of it matches bit for bit.
 #include <hip/hip_runtime.h>
 #include <atomic>
 #include <type_traits>
@@ -64,21 +63,57 @@ __device__ __forceinline__ void exp_lane(float* v, int iters, float khinv) {
     }
 }
 
-// Softmax of the row a workgroup holds in registers: lane l holds the float4
-// groups l, l + 256, ... of the row (E = 4 VPT values, -inf past the row
-// end, whose exp is +0, so the max, the lane sums (s + 0 == s) and the
-// outputs are those of the elements that exist).  On return v holds the
-// outputs.  t is the row's query position (masked rows only).
+// Which elements of a row a lane holds: units of VEC values (4: 16-byte
+// groups; 1: single values, for row lengths that are no multiple of 4 and
+// unaligned pointers), unit l + LANES i for lane l of the W waves of the row.
+//
+// W = 4 is the order of the sums.  W = 1 (rows of up to 1024) has the same
+// bits: the units l, l + 64, l + 128, l + 192 that its lane l holds are those
+// of lane l of each of the four waves, so it keeps four sums apart, runs the
+// four butterflies side by side and adds them in order.  It needs no barriers
+// and leaves no wave without a row.
+template <int VEC_, int W_>
+struct RowLayout {
+    static constexpr int VEC = VEC_, W = W_, LANES = 64 * W_;
+    static constexpr int sums(int E) { return W == 4 ? 1 : E / VEC < 4 ? E / VEC : 4; }
+    static __device__ __forceinline__ int lane() { return W == 4 ? threadIdx.x : threadIdx.x & 63; }
+    static __device__ __forceinline__ int unit(int i) { return lane() + LANES * i; }
+    static __device__ __forceinline__ int index(int e) { return VEC * unit(e / VEC) + e % VEC; }
+    static constexpr int sum_of(int e) { return W == 4 ? 0 : (e / VEC) % 4; }
+    // the row this thread works on (W = 1: four to a workgroup)
+    static __device__ __forceinline__ long row() {
+        return W == 4 ? (long)blockIdx.x : 4L * blockIdx.x + threadIdx.x / 64;
+    }
+    static dim3 grid(long rows) { return dim3((unsigned)(W == 4 ? rows : (rows + 3) / 4)); }
+    // the row's sum of every lane's partial sums s[sums(E)]
+    template <int S, bool TRAIL = false, bool LDS_ONLY = false>
+    static __device__ __forceinline__ float total(const float* s, float* red) {
+        if constexpr (W == 4) {
+            return block_sum<TRAIL, LDS_ONLY>(s[0], red);
+        } else {
+            float r = wave_sum(s[0]);
+#pragma unroll
+            for (int i = 1; i < S; i++) r += wave_sum(s[i]);
+            return r;
+        }
+    }
+};
+
+// Softmax of the row a workgroup (or wave) holds in registers, E values per
+// lane, -inf past the row end, whose exp is +0, so the max, the lane sums
+// (s + 0 == s) and the outputs are those of the elements that exist.  On
+// return v holds the outputs.  t is the row's query position (masked rows
+// only).
 // First stage: masking (masked rows) and the lane's maximum.
-template <int VPT, bool MASKED, bool FULL>
-__device__ __forceinline__ float softmax_lane_max(float* v, long n4, long t, const SoftmaxMask& mk) {
+template <class L, int VPT, bool MASKED, bool FULL>
+__device__ __forceinline__ float softmax_lane_max(float* v, long n, long t, const SoftmaxMask& mk) {
     if constexpr (MASKED) {
 #pragma unroll
-        for (int i = 0; i < VPT; i++) {
-            const long idx = threadIdx.x + (long)i * kRowThreads;
-            if (FULL || idx < n4) {
+        for (int i = 0; i < 4 * VPT / L::VEC; i++) {
+            const long j = (long)L::VEC * L::unit(i);
+            if (FULL || j < n) {
 #pragma unroll
-                for (int c = 0; c < 4; c++) v[4 * i + c] = mask_score(v[4 * i + c], t, 4 * idx + c, mk);
+                for (int c = 0; c < L::VEC; c++) v[L::VEC * i + c] = mask_score(v[L::VEC * i + c], t, j + c, mk);
             }
         }
     }
@@ -89,29 +124,36 @@ __device__ __forceinline__ float softmax_lane_max(float* v, long n4, long t, con
     return m;
 }
 
-// The lane's first zero (zero_key) in the register layout: group i of lane l
-// is the row's float4 group l + 256 i, so the lane's values run in index
-// order.
-template <int VPT>
+// The lane's first zero (zero_key): a lane's values run in index order.
+template <class L, int VPT>
 __device__ __forceinline__ uint32_t lane_first_zero(const float* v) {
     uint32_t key = ~0u;
 #pragma unroll
     for (int e = 4 * VPT - 1; e >= 0; e--)
-        if (v[e] == 0.0f) key = zero_key<uint32_t>(4 * (threadIdx.x + kRowThreads * (e / 4)) + e % 4, v[e]);
+        if (v[e] == 0.0f) key = zero_key<uint32_t>(L::index(e), v[e]);
     return key;
 }
 
-// Exps of the lane's values against the row maximum m, and the lane's sum
-// of them (masked rows, and rows whose step count is known only at run time).
+// The lane's partial sums of its values.
+template <class L, int E>
+__device__ __forceinline__ void lane_sums(const float* v, float* s) {
+#pragma unroll
+    for (int i = 0; i < L::sums(E); i++) s[i] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < E; e++) s[L::sum_of(e)] += v[e];
+}
+
+// Exps of the lane's values against the row maximum m (masked rows, and rows
+// whose step count is known only at run time).
 template <int VPT, int NITER, bool MASKED>
-__device__ __forceinline__ float softmax_lane_exps(float* v, float m, int iters, float khinv) {
+__device__ __forceinline__ void softmax_lane_exps(float* v, float m, int iters, float khinv) {
     constexpr int E = 4 * VPT;
 #pragma unroll
     for (int e = 0; e < E; e++) v[e] = v[e] - m;
     if constexpr (MASKED) {
         // the exps of -inf are +0: a wave skips the runs of its values that
         // are -inf in every lane (past the diagonal of a causal row)
-        constexpr int G = E <= 8 ? 4 : 8;
+        constexpr int G = E % 8 || E == 8 ? 4 : 8;
 #pragma unroll
         for (int b = 0; b < E; b += G) {
             bool some = false;
@@ -127,10 +169,6 @@ __device__ __forceinline__ float softmax_lane_exps(float* v, float m, int iters,
     } else {
         exp_lane<NITER, E>(v, iters, khinv);
     }
-    float s = 0.0f;
-#pragma unroll
-    for (int e = 0; e < E; e++) s += v[e];
-    return s;
 }
 
 // Unmasked rows with a compile-time step count.  Every x - max is <= 0 or
@@ -157,7 +195,7 @@ struct RowExtent {
 // row_lds: the row in LDS in the same layout (the prefetching kernel), read
 // instead of v for the rare zero-maximum scan, so that scan holds no
 // registers of its own; null: scan v.
-template <int VPT, bool LDS_ONLY>
+template <class L, int VPT, bool LDS_ONLY>
 __device__ __forceinline__ RowExtent unmasked_row_extent(const float* v, float* red, uint32_t* zred,
                                                          const float* row_lds = nullptr) {
     constexpr int E = 4 * VPT;
@@ -167,18 +205,20 @@ __device__ __forceinline__ RowExtent unmasked_row_extent(const float* v, float* 
         mx = maximum(mx, v[e]);
         mn = fminf(mn, v[e]);
     }
-    mx = block_maximum<false, LDS_ONLY>(mx, red);
+    if constexpr (L::W == 1) mx = wave_maximum(mx);
+    else mx = block_maximum<false, LDS_ONLY>(mx, red);
     if (mx == 0.0f) {
         uint32_t key = ~0u;
         if (row_lds) {
             for (int e = 0; e < E && key == ~0u; e++) {
-                const int idx = 4 * (threadIdx.x + kRowThreads * (e / 4)) + e % 4;
+                const int idx = L::index(e);
                 if (row_lds[idx] == 0.0f) key = zero_key<uint32_t>(idx, row_lds[idx]);
             }
         } else {
-            key = lane_first_zero<VPT>(v);
+            key = lane_first_zero<L, VPT>(v);
         }
-        mx = first_zero_max<LDS_ONLY>(key, zred);
+        if constexpr (L::W == 1) mx = wave_first_zero_max(key);
+        else mx = first_zero_max<LDS_ONLY>(key, zred);
     }
     return {mx, mn};
 }
@@ -207,93 +247,94 @@ __device__ __forceinline__ void unmasked_exp_group(float* v, float khinv, bool f
 }
 
 template <int NITER, int E>
-__device__ __forceinline__ float unmasked_lane_exps(float* v, RowExtent r, float khinv) {
+__device__ __forceinline__ void unmasked_lane_exps(float* v, RowExtent r, float khinv) {
     const bool fused = __all((r.min - r.max) >= -86.0f);
 #pragma unroll
     for (int e = 0; e < E; e++) v[e] = v[e] - r.max;
     constexpr int G = E < 16 ? E : 16;
 #pragma unroll
-    for (int b = 0; b < E; b += G) unmasked_exp_group<NITER, G>(v + b, khinv, fused);
-    float s = 0.0f;
-#pragma unroll
-    for (int e = 0; e < E; e++) s += v[e];
-    if (!(__builtin_fabsf(r.max) < __builtin_inff())) s = __builtin_nanf("");
-    return s;
+    for (int b = 0; b + G <= E; b += G) unmasked_exp_group<NITER, G>(v + b, khinv, fused);
+}
+__device__ __forceinline__ float unmasked_row_sum(float s, RowExtent r) {
+    return __builtin_fabsf(r.max) < __builtin_inff() ? s : __builtin_nanf("");
 }
 
-// Second stage: row max, exps, row sum, scaling (m: the lane's maximum).
 // red: 2 kRowWaves floats (max and sum partials apart, so neither reduction
 // needs a trailing barrier; a kernel handles one row per workgroup).
-template <int VPT, int NITER, bool MASKED>
-__device__ __forceinline__ void softmax_row_finish(float* v, float m, int iters, float khinv,
-                                                   const SoftmaxMask& mk, float* red, uint32_t* zred) {
-    constexpr int E = 4 * VPT;
-    m = block_max<false>(m, red);
-    if (m == 0.0f) m = first_zero_max<false>(lane_first_zero<VPT>(v), zred);
-    float s = softmax_lane_exps<VPT, NITER, MASKED>(v, m, iters, khinv);
-    s = block_sum<false>(s, red + kRowWaves);
-    const float inv = inv_sum(s, MASKED ? mk.zero_guard : 0);
+template <class L, int VPT, int NITER, bool MASKED, bool FULL>
+__device__ __forceinline__ void softmax_row_regs(float* v, long n, long t, int iters, float khinv,
+                                                 const SoftmaxMask& mk, float* red, uint32_t* zred) {
+    constexpr int E = 4 * VPT, S = L::sums(E);
+    float s[S], inv;
+    if constexpr (!MASKED && NITER > 0) {
+        const RowExtent r = unmasked_row_extent<L, VPT, false>(v, red, zred);
+        unmasked_lane_exps<NITER, E>(v, r, khinv);
+        lane_sums<L, E>(v, s);
+        inv = inv_sum(unmasked_row_sum(L::template total<S>(s, red + kRowWaves), r), 0);
+    } else {
+        float m = softmax_lane_max<L, VPT, MASKED, FULL>(v, n, t, mk);
+        if constexpr (L::W == 1) {
+            m = wave_max(m);
+            if (m == 0.0f) m = wave_first_zero_max(lane_first_zero<L, VPT>(v));
+        } else {
+            m = block_max<false>(m, red);
+            if (m == 0.0f) m = first_zero_max<false>(lane_first_zero<L, VPT>(v), zred);
+        }
+        softmax_lane_exps<VPT, NITER, MASKED>(v, m, iters, khinv);
+        lane_sums<L, E>(v, s);
+        inv = inv_sum(L::template total<S>(s, red + kRowWaves), MASKED ? mk.zero_guard : 0);
+    }
 #pragma unroll
     for (int e = 0; e < E; e++) v[e] = v[e] * inv;
 }
 
-template <int VPT, int NITER, bool MASKED, bool FULL>
-__device__ __forceinline__ void softmax_row_regs(float* v, long n4, long t, int iters, float khinv,
-                                                 const SoftmaxMask& mk, float* red, uint32_t* zred) {
-    if constexpr (!MASKED && NITER > 0) {
-        const RowExtent r = unmasked_row_extent<VPT, false>(v, red, zred);
-        float s = unmasked_lane_exps<NITER, 4 * VPT>(v, r, khinv);
-        s = block_sum<false>(s, red + kRowWaves);
-        const float inv = inv_sum(s, 0);
-#pragma unroll
-        for (int e = 0; e < 4 * VPT; e++) v[e] = v[e] * inv;
-        return;
-    }
-    const float m = softmax_lane_max<VPT, MASKED, FULL>(v, n4, t, mk);
-    softmax_row_finish<VPT, NITER, MASKED>(v, m, iters, khinv, mk, red, zred);
-}
-
 // last: the last column needed (causal rows: the query position; the mask
-// puts -inf past it whatever was there).
-template <int VPT, bool FULL, bool MASKED = false>
-__device__ __forceinline__ void load_row_regs(const float* xrow, long n4, float* v, long last = 0) {
-    const float4* xr = reinterpret_cast<const float4*>(xrow);
+// puts -inf past it whatever was there).  pad: in place of what is not there.
+template <class L, int VPT, bool FULL, bool MASKED = false>
+__device__ __forceinline__ void load_row_regs(const float* xr, long n, float* v, float pad, long last = 0) {
 #pragma unroll
-    for (int i = 0; i < VPT; i++) {
-        const long idx = threadIdx.x + (long)i * kRowThreads;
-        float4 t = make_float4(-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff());
-        if ((FULL || idx < n4) && (!MASKED || 4 * idx <= last)) t = ld4_stream(&xr[idx]);
-        v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+    for (int i = 0; i < 4 * VPT / L::VEC; i++) {
+        const long j = (long)L::VEC * L::unit(i);
+        const bool in = (FULL || j < n) && (!MASKED || j <= last);
+        if constexpr (L::VEC == 4) {
+            float4 t = make_float4(pad, pad, pad, pad);
+            if (in) t = ld4_stream(reinterpret_cast<const float4*>(xr + j));
+            v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+        } else {
+            v[i] = in ? xr[j] : pad;
+        }
     }
 }
 
-template <int VPT, bool FULL>
-__device__ __forceinline__ void store_row_regs(float* yrow, long n4, const float* v) {
-    float4* yr = reinterpret_cast<float4*>(yrow);
+template <class L, int VPT, bool FULL>
+__device__ __forceinline__ void store_row_regs(float* yr, long n, const float* v) {
 #pragma unroll
-    for (int i = 0; i < VPT; i++) {
-        const long idx = threadIdx.x + (long)i * kRowThreads;
-        if (FULL || idx < n4) st4_stream(&yr[idx], make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]));
+    for (int i = 0; i < 4 * VPT / L::VEC; i++) {
+        const long j = (long)L::VEC * L::unit(i);
+        if (!FULL && j >= n) continue;
+        if constexpr (L::VEC == 4)
+            st4_stream(reinterpret_cast<float4*>(yr + j), make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]));
+        else
+            yr[j] = v[i];
     }
 }
 
-// One workgroup per row: the row is read once into registers (16-byte
-// loads), reduced, exponentiated and written once.
-// FULL: n == 1024 * VPT exactly, so no lane needs a bounds check.
-template <int VPT, int NITER, bool MASKED, bool FULL>
+// Rows held in registers: read once, reduced, exponentiated and written once.
+// FULL: n == 4 LANES VPT exactly, so no lane needs a bounds check.
+template <class L, int VPT, int NITER, bool MASKED, bool FULL>
 __global__ __launch_bounds__(kRowThreads) void softmax_reg_kernel(
-    const float* x, float* y, long n, int iters, float khinv,
+    const float* x, float* y, long rows, long n, int iters, float khinv,
     SoftmaxMask mk)
 {
     __shared__ float red[2 * kRowWaves];
     __shared__ uint32_t zred[kRowWaves];
-    const long row = blockIdx.x;
-    const long n4 = n / 4;
+    const long row = L::row();
+    if (L::W == 1 && row >= rows) return;
     float v[4 * VPT];
     const long t = MASKED ? mk.row0 + row % mk.seq : 0;
-    load_row_regs<VPT, FULL, MASKED>(x + row * n, n4, v, MASKED && mk.causal ? t : n);
-    softmax_row_regs<VPT, NITER, MASKED, FULL>(v, n4, t, iters, khinv, mk, red, zred);
-    store_row_regs<VPT, FULL>(y + row * n, n4, v);
+    load_row_regs<L, VPT, FULL, MASKED>(x + row * n, n, v, -__builtin_inff(), MASKED && mk.causal ? t : n);
+    softmax_row_regs<L, VPT, NITER, MASKED, FULL>(v, n, t, iters, khinv, mk, red, zred);
+    store_row_regs<L, VPT, FULL>(y + row * n, n, v);
 }
 
 // Unmasked rows of exactly 1024 VPT floats, persistent: workgroup g takes
@@ -304,7 +345,7 @@ __global__ __launch_bounds__(kRowThreads) void softmax_reg_kernel(
 // The row reductions use LDS-only barriers (lds_barrier): the previous
 // row's stores stay in flight across them; the barrier of the row sum
 // waits for the prefetch (an LDS write), which has had the exps to land.
-// Same arithmetic as softmax_reg_kernel<VPT, NITER, false, true>, so the
+// Same arithmetic as softmax_reg_kernel<RowLayout<4, 4>, VPT, ..>, so the
 // same bits.  Used where the exps are short (n = 8): at 16 and 24 steps the
 // one-row-per-workgroup kernel is faster (measured on 4096 x 4096: n = 8
 // 23.6 -> 22.2 us; n = 16 25.0 against 26.3, n = 24 31.1 against 32.2).
@@ -312,6 +353,7 @@ template <int VPT, int NITER>
 __global__ __launch_bounds__(kRowThreads, 6) void softmax_prefetch_kernel(
     const float* x, float* y, long rows, float khinv)
 {
+    using L = RowLayout<4, 4>;
     constexpr long n = 1024L * VPT;
     constexpr int E = 4 * VPT;
     __shared__ __attribute__((aligned(16))) float row_lds[n];
@@ -342,18 +384,20 @@ __global__ __launch_bounds__(kRowThreads, 6) void softmax_prefetch_kernel(
         }
         // every wave has read row_lds (its lane maximum needs the values)
         // once the barrier inside block_maximum is passed
-        const RowExtent r = unmasked_row_extent<VPT, true>(v, red, zred, row_lds);
+        const RowExtent r = unmasked_row_extent<L, VPT, true>(v, red, zred, row_lds);
         if (row + G < rows) prefetch(row + G);
-        float s = unmasked_lane_exps<NITER, E>(v, r, khinv);
+        unmasked_lane_exps<NITER, E>(v, r, khinv);
+        float s;
+        lane_sums<L, E>(v, &s);
         // the prefetch has landed before the barrier below (the LDS fence
         // waits for it too; this states it, and the operand keeps the wait
         // after the exps)
         asm volatile("s_waitcnt vmcnt(0)" : "+v"(s));
-        s = block_sum<false, true>(s, red + kRowWaves);
-        const float inv = inv_sum(s, 0);
+        s = L::total<1, false, true>(&s, red + kRowWaves);
+        const float inv = inv_sum(unmasked_row_sum(s, r), 0);
 #pragma unroll
         for (int e = 0; e < E; e++) v[e] = v[e] * inv;
-        store_row_regs<VPT, true>(y + row * n, n / 4, v);
+        store_row_regs<L, VPT, true>(y + row * n, n, v);
     }
 }
 
@@ -428,17 +472,58 @@ __global__ __launch_bounds__(kRowThreads) void softmax_loop_kernel(
 constexpr long kCuLdsBytes = 160L * 1024;
 constexpr int unmasked_reg_cap(int vpt) { return vpt <= 2 ? 0 : vpt == 4 ? 6 : vpt == 8 ? 4 : 3; }
 
-template <int VPT, int NITER, bool MASKED>
-static void softmax_reg_launch(dim3 grid, hipStream_t s, const float* x, float* y, long n, int iters,
+template <class L, int VPT, int NITER, bool MASKED>
+static void softmax_reg_launch(hipStream_t s, const float* x, float* y, long rows, long n, int iters,
                                float khinv, const SoftmaxMask& mk) {
-    constexpr int cap = (!MASKED && NITER > 0) ? unmasked_reg_cap(VPT) : 0;
+    constexpr int cap = (!MASKED && NITER > 0 && L::W == 4) ? unmasked_reg_cap(VPT) : 0;
     constexpr size_t lds = cap ? (size_t)(kCuLdsBytes / cap - 1024) : 0;
-    if (n == 4L * VPT * kRowThreads)
-        hipLaunchKernelGGL((softmax_reg_kernel<VPT, NITER, MASKED, true>), grid, dim3(kRowThreads), lds, s, x, y,
-                           n, iters, khinv, mk);
-    else
-        hipLaunchKernelGGL((softmax_reg_kernel<VPT, NITER, MASKED, false>), grid, dim3(kRowThreads), lds, s, x,
-                           y, n, iters, khinv, mk);
+    if constexpr (L::VEC == 4) {
+        if (n == 4L * VPT * L::LANES) {
+            hipLaunchKernelGGL((softmax_reg_kernel<L, VPT, NITER, MASKED, true>), L::grid(rows), dim3(kRowThreads),
+                               lds, s, x, y, rows, n, iters, khinv, mk);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((softmax_reg_kernel<L, VPT, NITER, MASKED, false>), L::grid(rows), dim3(kRowThreads), lds, s,
+                       x, y, rows, n, iters, khinv, mk);
+}
+
+// Calls f(layout, VPT) for the layout of rows of n values (vec: 16-byte
+// groups) and returns true, or returns false where a row does not fit.
+// A wave takes a row of up to 768 once there are 4 rows per CU (fewer rows
+// need the four waves each): softmax n = 16 against a workgroup per row
+// 16000 x 500 25.6 -> 15.1 us, 8192 x 100 13.7 -> 5.6, 4096 x 700 9.3 -> 7.7,
+// 1024 x 256 4.0 -> 2.9; RMSNorm 16000 x 500 19.6 -> 12.7, LayerNorm
+// 22.4 -> 13.1.  Past 768 its 16 values per lane leave too few waves in
+// flight until there are `wide` rows per CU (softmax 32: 4096 x 1000
+// 9.7 against 9.9, 16000 x 1000 29.3 against 26.5; the norms 16:
+// RMSNorm 2048 x 1000 4.95 against 5.25, 4096 x 1000 8.9 against 6.9).
+// Rows that cannot be read in 16-byte groups (the strided loop before):
+// softmax 4096 x 4095 69.5 -> 29.3 us (4096 x 4096: 25.1), RMSNorm 40.4 ->
+// 28.3, LayerNorm 49.3 -> 28.9.
+template <class F>
+static bool with_row_layout(long rows, long n, bool vec, long wide, F f) {
+    const long per_cu = rows / device_cus();
+    auto at = [&](auto vec_c) {
+        constexpr int VEC = decltype(vec_c)::value;
+        using L1 = RowLayout<VEC, 1>;
+        using L4 = RowLayout<VEC, 4>;
+#define RAC_VPT(L, k) f(L(), std::integral_constant<int, k>())
+        if (n <= 1024 && per_cu >= (n <= 768 ? 4 : wide)) {
+            if (n <= 256) RAC_VPT(L1, 1);
+            else if (n <= 512) RAC_VPT(L1, 2);
+            else if (n <= 768) RAC_VPT(L1, 3);
+            else RAC_VPT(L1, 4);
+        } else if (n <= 1024) RAC_VPT(L4, 1);
+        else if (n <= 2048) RAC_VPT(L4, 2);
+        else if (n <= 4096) RAC_VPT(L4, 4);
+        else if (n <= 8192) RAC_VPT(L4, 8);
+        else if (n <= 16384) RAC_VPT(L4, 16);
+        else return false;
+#undef RAC_VPT
+        return true;
+    };
+    return vec ? at(std::integral_constant<int, 4>()) : at(std::integral_constant<int, 1>());
 }
 
 template <int NITER, bool MASKED>
@@ -446,7 +531,6 @@ static hipError_t softmax_dispatch(const float* x, float* y, long rows, long n, 
                                    float khinv, hipStream_t s, const SoftmaxMask& mk) {
     const bool vec_ok = (n % 4 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0) &&
                         ((reinterpret_cast<uintptr_t>(y) & 15) == 0);
-    const long n4 = n / 4;
     dim3 grid((unsigned)rows), block(kRowThreads);
     if constexpr (!MASKED && NITER > 0 && NITER <= 8) {
         // short exps: the persistent prefetching kernel, where every
@@ -465,17 +549,9 @@ static hipError_t softmax_dispatch(const float* x, float* y, long rows, long n, 
                        prefetch_launch(std::integral_constant<int, 4>{})))
             return hipGetLastError();
     }
-    if (vec_ok && n4 <= 1 * kRowThreads)
-        softmax_reg_launch<1, NITER, MASKED>(grid, s, x, y, n, iters, khinv, mk);
-    else if (vec_ok && n4 <= 2 * kRowThreads)
-        softmax_reg_launch<2, NITER, MASKED>(grid, s, x, y, n, iters, khinv, mk);
-    else if (vec_ok && n4 <= 4 * kRowThreads)
-        softmax_reg_launch<4, NITER, MASKED>(grid, s, x, y, n, iters, khinv, mk);
-    else if (vec_ok && n4 <= 8 * kRowThreads)
-        softmax_reg_launch<8, NITER, MASKED>(grid, s, x, y, n, iters, khinv, mk);
-    else if (vec_ok && n4 <= 16 * kRowThreads)
-        softmax_reg_launch<16, NITER, MASKED>(grid, s, x, y, n, iters, khinv, mk);
-    else
+    if (!with_row_layout(rows, n, vec_ok, 32, [&](auto l, auto vpt) {
+            softmax_reg_launch<decltype(l), decltype(vpt)::value, NITER, MASKED>(s, x, y, rows, n, iters, khinv, mk);
+        }))
         hipLaunchKernelGGL((softmax_loop_kernel<NITER, MASKED>), grid, block, 0, s, x, y, n, iters, khinv, mk);
     return hipGetLastError();
 }
@@ -506,44 +582,43 @@ hipError_t softmax_launch(const float* x, float* y, long rows, long n, int iters
 
 // ── RMSNorm / LayerNorm ──────────────────────────────────────────────────
 
-template <int VPT>
+// The VEC values of a weight row at column j (gamma null: 1; beta null: 0).
+template <int VEC>
+__device__ __forceinline__ void load_weights(const float* w, long j, float none, float* v) {
+    if constexpr (VEC == 4) {
+        const float4 q = w ? *reinterpret_cast<const float4*>(w + j) : make_float4(none, none, none, none);
+        v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    } else {
+        v[0] = w ? w[j] : none;
+    }
+}
+
+template <class L, int VPT>
 __global__ __launch_bounds__(kRowThreads) void rmsnorm_reg_kernel(
     const float* __restrict__ x, float* __restrict__ y, const float* __restrict__ gamma,
-    float eps, long d, float khinv16)
+    float eps, long rows, long d, float khinv16)
 {
+    constexpr int E = 4 * VPT, S = L::sums(E);
     __shared__ float red[kRowWaves];
-    const long row = blockIdx.x;
-    const float4* xr = reinterpret_cast<const float4*>(x + row * d);
-    float4* yr = reinterpret_cast<float4*>(y + row * d);
-    const float4* g4 = reinterpret_cast<const float4*>(gamma);
-    const long d4 = d / 4;
-    float4 v[VPT];
+    const long row = L::row();
+    if (L::W == 1 && row >= rows) return;
+    float v[E], ss[S] = {};
+    load_row_regs<L, VPT, false>(x + row * d, d, v, 0.0f);
 #pragma unroll
-    for (int i = 0; i < VPT; i++) {
-        const long idx = threadIdx.x + (long)i * kRowThreads;
-        v[i] = (idx < d4) ? ld4_stream(&xr[idx]) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    float ss = 0.0f;
-#pragma unroll
-    for (int i = 0; i < VPT; i++) {
-        ss = __builtin_fmaf(v[i].x, v[i].x, ss);
-        ss = __builtin_fmaf(v[i].y, v[i].y, ss);
-        ss = __builtin_fmaf(v[i].z, v[i].z, ss);
-        ss = __builtin_fmaf(v[i].w, v[i].w, ss);
-    }
-    const float ms = block_sum(ss, red) / (float)d;
+    for (int e = 0; e < E; e++) ss[L::sum_of(e)] = __builtin_fmaf(v[e], v[e], ss[L::sum_of(e)]);
+    const float ms = L::template total<S>(ss, red) / (float)d;
     const float inv = rsqrt_cordic(ms + eps, khinv16);
 #pragma unroll
-    for (int i = 0; i < VPT; i++) {
-        const long idx = threadIdx.x + (long)i * kRowThreads;
-        if (idx < d4) {
-            const float4 g = gamma ? g4[idx] : make_float4(1.f, 1.f, 1.f, 1.f);
-            float4 o;
-            o.x = v[i].x * inv * g.x; o.y = v[i].y * inv * g.y;
-            o.z = v[i].z * inv * g.z; o.w = v[i].w * inv * g.w;
-            st4_stream(&yr[idx], o);
+    for (int i = 0; i < E / L::VEC; i++) {
+        const long j = (long)L::VEC * L::unit(i);
+        if (j < d) {
+            float g[L::VEC];
+            load_weights<L::VEC>(gamma, j, 1.0f, g);
+#pragma unroll
+            for (int c = 0; c < L::VEC; c++) v[L::VEC * i + c] = v[L::VEC * i + c] * inv * g[c];
         }
     }
+    store_row_regs<L, VPT, false>(y + row * d, d, v);
 }
 
 __global__ __launch_bounds__(kRowThreads) void rmsnorm_loop_kernel(
@@ -564,56 +639,41 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_loop_kernel(
     }
 }
 
-template <int VPT>
+template <class L, int VPT>
 __global__ __launch_bounds__(kRowThreads) void layernorm_reg_kernel(
     const float* __restrict__ x, float* __restrict__ y, const float* __restrict__ gamma,
-    const float* __restrict__ beta, float eps, long d, float khinv16)
+    const float* __restrict__ beta, float eps, long rows, long d, float khinv16)
 {
-    __shared__ float red[kRowWaves];
-    const long row = blockIdx.x;
-    const float4* xr = reinterpret_cast<const float4*>(x + row * d);
-    float4* yr = reinterpret_cast<float4*>(y + row * d);
-    const float4* g4 = reinterpret_cast<const float4*>(gamma);
-    const float4* b4 = reinterpret_cast<const float4*>(beta);
-    const long d4 = d / 4;
-    float4 v[VPT];
+    constexpr int E = 4 * VPT, S = L::sums(E);
+    __shared__ float red[2 * kRowWaves];
+    const long row = L::row();
+    if (L::W == 1 && row >= rows) return;
+    float v[E], sm[S], sv[S] = {};
+    load_row_regs<L, VPT, false>(x + row * d, d, v, 0.0f);
+    lane_sums<L, E>(v, sm);
+    const float mean = L::template total<S>(sm, red) / (float)d;
 #pragma unroll
-    for (int i = 0; i < VPT; i++) {
-        const long idx = threadIdx.x + (long)i * kRowThreads;
-        v[i] = (idx < d4) ? ld4_stream(&xr[idx]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int e = 0; e < E; e++) {
+        const float z = v[e] - mean;
+        if (L::index(e) < d) sv[L::sum_of(e)] = __builtin_fmaf(z, z, sv[L::sum_of(e)]);
     }
-    float sm = 0.0f;
-#pragma unroll
-    for (int i = 0; i < VPT; i++) { sm += v[i].x; sm += v[i].y; sm += v[i].z; sm += v[i].w; }
-    const float mean = block_sum(sm, red) / (float)d;
-    float sv = 0.0f;
-#pragma unroll
-    for (int i = 0; i < VPT; i++) {
-        const long idx = threadIdx.x + (long)i * kRowThreads;
-        if (idx < d4) {
-            float z;
-            z = v[i].x - mean; sv = __builtin_fmaf(z, z, sv);
-            z = v[i].y - mean; sv = __builtin_fmaf(z, z, sv);
-            z = v[i].z - mean; sv = __builtin_fmaf(z, z, sv);
-            z = v[i].w - mean; sv = __builtin_fmaf(z, z, sv);
-        }
-    }
-    const float var = block_sum(sv, red) / (float)d;
+    const float var = L::template total<S>(sv, red + kRowWaves) / (float)d;
     const float inv = rsqrt_cordic(var + eps, khinv16);
 #pragma unroll
-    for (int i = 0; i < VPT; i++) {
-        const long idx = threadIdx.x + (long)i * kRowThreads;
-        if (idx < d4) {
-            const float4 g = gamma ? g4[idx] : make_float4(1.f, 1.f, 1.f, 1.f);
-            const float4 b = beta ? b4[idx] : make_float4(0.f, 0.f, 0.f, 0.f);
-            float4 o;
-            o.x = __builtin_fmaf(g.x, (v[i].x - mean) * inv, b.x);
-            o.y = __builtin_fmaf(g.y, (v[i].y - mean) * inv, b.y);
-            o.z = __builtin_fmaf(g.z, (v[i].z - mean) * inv, b.z);
-            o.w = __builtin_fmaf(g.w, (v[i].w - mean) * inv, b.w);
-            st4_stream(&yr[idx], o);
+    for (int i = 0; i < E / L::VEC; i++) {
+        const long j = (long)L::VEC * L::unit(i);
+        if (j < d) {
+            float g[L::VEC], b[L::VEC];
+            load_weights<L::VEC>(gamma, j, 1.0f, g);
+            load_weights<L::VEC>(beta, j, 0.0f, b);
+#pragma unroll
+            for (int c = 0; c < L::VEC; c++) {
+                float& o = v[L::VEC * i + c];
+                o = __builtin_fmaf(g[c], (o - mean) * inv, b[c]);
+            }
         }
     }
+    store_row_regs<L, VPT, false>(y + row * d, d, v);
 }
 
 __global__ __launch_bounds__(kRowThreads) void layernorm_loop_kernel(
@@ -647,20 +707,12 @@ hipError_t rmsnorm_launch(const float* x, float* y, const float* gamma, float ep
                           long rows, long d, hipStream_t s) {
     const float k = host_consts().rsqrt_khinv;
     const bool vec_ok = (d % 4 == 0) && aligned16(x) && aligned16(y) && (!gamma || aligned16(gamma));
-    const long d4 = d / 4;
-    dim3 grid((unsigned)rows), block(kRowThreads);
-    if (vec_ok && d4 <= kRowThreads)
-        hipLaunchKernelGGL((rmsnorm_reg_kernel<1>), grid, block, 0, s, x, y, gamma, eps, d, k);
-    else if (vec_ok && d4 <= 2 * kRowThreads)
-        hipLaunchKernelGGL((rmsnorm_reg_kernel<2>), grid, block, 0, s, x, y, gamma, eps, d, k);
-    else if (vec_ok && d4 <= 4 * kRowThreads)
-        hipLaunchKernelGGL((rmsnorm_reg_kernel<4>), grid, block, 0, s, x, y, gamma, eps, d, k);
-    else if (vec_ok && d4 <= 8 * kRowThreads)
-        hipLaunchKernelGGL((rmsnorm_reg_kernel<8>), grid, block, 0, s, x, y, gamma, eps, d, k);
-    else if (vec_ok && d4 <= 16 * kRowThreads)
-        hipLaunchKernelGGL((rmsnorm_reg_kernel<16>), grid, block, 0, s, x, y, gamma, eps, d, k);
-    else
-        hipLaunchKernelGGL(rmsnorm_loop_kernel, grid, block, 0, s, x, y, gamma, eps, d, k);
+    if (!with_row_layout(rows, d, vec_ok, 16, [&](auto l, auto vpt) {
+            using L = decltype(l);
+            hipLaunchKernelGGL((rmsnorm_reg_kernel<L, decltype(vpt)::value>), L::grid(rows), dim3(kRowThreads), 0, s,
+                               x, y, gamma, eps, rows, d, k);
+        }))
+        hipLaunchKernelGGL(rmsnorm_loop_kernel, dim3((unsigned)rows), dim3(kRowThreads), 0, s, x, y, gamma, eps, d, k);
     return hipGetLastError();
 }
 
@@ -669,20 +721,12 @@ hipError_t layernorm_launch(const float* x, float* y, const float* gamma, const 
     const float k = host_consts().rsqrt_khinv;
     const bool vec_ok = (d % 4 == 0) && aligned16(x) && aligned16(y) &&
                         (!gamma || aligned16(gamma)) && (!beta || aligned16(beta));
-    const long d4 = d / 4;
-    dim3 grid((unsigned)rows), block(kRowThreads);
-    if (vec_ok && d4 <= kRowThreads)
-        hipLaunchKernelGGL((layernorm_reg_kernel<1>), grid, block, 0, s, x, y, gamma, beta, eps, d, k);
-    else if (vec_ok && d4 <= 2 * kRowThreads)
-        hipLaunchKernelGGL((layernorm_reg_kernel<2>), grid, block, 0, s, x, y, gamma, beta, eps, d, k);
-    else if (vec_ok && d4 <= 4 * kRowThreads)
-        hipLaunchKernelGGL((layernorm_reg_kernel<4>), grid, block, 0, s, x, y, gamma, beta, eps, d, k);
-    else if (vec_ok && d4 <= 8 * kRowThreads)
-        hipLaunchKernelGGL((layernorm_reg_kernel<8>), grid, block, 0, s, x, y, gamma, beta, eps, d, k);
-    else if (vec_ok && d4 <= 16 * kRowThreads)
-        hipLaunchKernelGGL((layernorm_reg_kernel<16>), grid, block, 0, s, x, y, gamma, beta, eps, d, k);
-    else
-        hipLaunchKernelGGL(layernorm_loop_kernel, grid, block, 0, s, x, y, gamma, beta, eps, d, k);
+    if (!with_row_layout(rows, d, vec_ok, 16, [&](auto l, auto vpt) {
+            using L = decltype(l);
+            hipLaunchKernelGGL((layernorm_reg_kernel<L, decltype(vpt)::value>), L::grid(rows), dim3(kRowThreads), 0, s,
+                               x, y, gamma, beta, eps, rows, d, k);
+        }))
+        hipLaunchKernelGGL(layernorm_loop_kernel, dim3((unsigned)rows), dim3(kRowThreads), 0, s, x, y, gamma, beta, eps, d, k);
     return hipGetLastError();
 }
 

@@ -150,13 +150,23 @@ __device__ __forceinline__ float block_max(float v, float* red) {
     return r;
 }
 
-template <bool LDS_ONLY, class K>
-__device__ __forceinline__ float first_zero_max(K key, K* zred) {
+template <class K>
+__device__ __forceinline__ K wave_min_key(K key) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         const K o = __shfl_xor(key, off, 64);
         key = o < key ? o : key;
     }
+    return key;
+}
+// first_zero_max of a row that one wave holds.
+template <class K>
+__device__ __forceinline__ float wave_first_zero_max(K key) {
+    return (wave_min_key(key) & 1) ? -0.0f : 0.0f;
+}
+template <bool LDS_ONLY, class K>
+__device__ __forceinline__ float first_zero_max(K key, K* zred) {
+    key = wave_min_key(key);
     if ((threadIdx.x & 63) == 0) zred[threadIdx.x / 64] = key;
     red_barrier<LDS_ONLY>();
     K k = zred[0];
