@@ -255,8 +255,9 @@ __device__ __forceinline__ void unmasked_lane_exps(float* v, RowExtent r, float 
 #pragma unroll
     for (int b = 0; b + G <= E; b += G) unmasked_exp_group<NITER, G>(v + b, khinv, fused);
 }
-__device__ __forceinline__ float unmasked_row_sum(float s, RowExtent r) {
-    return __builtin_fabsf(r.max) < __builtin_inff() ? s : __builtin_nanf("");
+__device__ __forceinline__ float unmasked_lane_sum(float s, RowExtent r) {
+    if (!(__builtin_fabsf(r.max) < __builtin_inff())) s = __builtin_nanf("");
+    return s;
 }
 
 // red: 2 kRowWaves floats (max and sum partials apart, so neither reduction
@@ -270,7 +271,8 @@ __device__ __forceinline__ void softmax_row_regs(float* v, long n, long t, int i
         const RowExtent r = unmasked_row_extent<L, VPT, false>(v, red, zred);
         unmasked_lane_exps<NITER, E>(v, r, khinv);
         lane_sums<L, E>(v, s);
-        inv = inv_sum(unmasked_row_sum(L::template total<S>(s, red + kRowWaves), r), 0);
+        s[0] = unmasked_lane_sum(s[0], r);
+        inv = inv_sum(L::template total<S>(s, red + kRowWaves), 0);
     } else {
         float m = softmax_lane_max<L, VPT, MASKED, FULL>(v, n, t, mk);
         if constexpr (L::W == 1) {
@@ -389,12 +391,13 @@ __global__ __launch_bounds__(kRowThreads, 6) void softmax_prefetch_kernel(
         unmasked_lane_exps<NITER, E>(v, r, khinv);
         float s;
         lane_sums<L, E>(v, &s);
+        s = unmasked_lane_sum(s, r);
         // the prefetch has landed before the barrier below (the LDS fence
         // waits for it too; this states it, and the operand keeps the wait
         // after the exps)
         asm volatile("s_waitcnt vmcnt(0)" : "+v"(s));
         s = L::total<1, false, true>(&s, red + kRowWaves);
-        const float inv = inv_sum(unmasked_row_sum(s, r), 0);
+        const float inv = inv_sum(s, 0);
 #pragma unroll
         for (int e = 0; e < E; e++) v[e] = v[e] * inv;
         store_row_regs<L, VPT, true>(y + row * n, n, v);
