@@ -373,9 +373,11 @@ __global__ __launch_bounds__(256) void all_finite_kernel(const float* __restrict
 
 __global__ void set_flag_kernel(int* flag, int v) { *flag = v; }
 
-// flag = 1 unless some element of the four arrays (n each) is 2^58 or more
-// in magnitude, infinite or NaN: then no product of two of them over up to
-// 4096 k overflows, and what a causal backward pass may skip is exactly zero.
+// flag = 1 unless some element of the four arrays (n each) is 2^57 or more
+// in magnitude, infinite or NaN: then a product of two of them over up to
+// 4096 k stays below 2^126, and its distance from a mean of such products
+// (dP - rowsum(dP P)) below 2^127, so what a causal backward pass may skip is
+// 0 times something finite.
 __global__ __launch_bounds__(256) void all_bounded_kernel(const float* __restrict__ a, const float* __restrict__ b,
                                                           const float* __restrict__ c, const float* __restrict__ d,
                                                           long n, int* __restrict__ flag) {
@@ -391,7 +393,7 @@ __global__ __launch_bounds__(256) void all_bounded_kernel(const float* __restric
     }
     if (blockIdx.x == 0 && threadIdx.x < n - 4 * n4)
         m = __builtin_elementwise_maximum(m, __builtin_fabsf(x[4 * n4 + threadIdx.x]));
-    if (!(m < 0x1p58f)) *flag = 0;
+    if (!(m < 0x1p57f)) *flag = 0;
 }
 
 hipError_t all_bounded_launch(const float* a, const float* b, const float* c, const float* d, long n, int* flag,

@@ -89,7 +89,7 @@ hipError_t gemm_launch(int ta, int tb, const float* A, const float* B, float* C,
                        int row0 = 0, int k_side = 1, int period = 0);
 // *flag = 1 if every x[i] is finite, else 0 (stream-ordered).
 hipError_t all_finite_launch(const float* x, long n, int* flag, hipStream_t s);
-// *flag = 1 if every element of the four arrays is below 2^58 in magnitude,
+// *flag = 1 if every element of the four arrays is below 2^57 in magnitude,
 // else 0.
 hipError_t all_bounded_launch(const float* a, const float* b, const float* c, const float* d, long n, int* flag,
                               hipStream_t s);

@@ -90,3 +90,23 @@ def test_attention_backward_unbounded_operands(which, value):
     ext.attention_backward(*ops[:3], P, ops[3], True, *got)
     for a, b in zip(got, want):
         assert torch.equal(a.isnan(), b.isnan())
+
+
+def test_attention_backward_overflowing_differences():
+    """Operands whose products are finite but whose dP - rowsum(dP P) is not:
+    0 times it is NaN past the diagonal too, so nothing may be skipped.  dP is
+    +-1.125 * 2^127 in alternate columns: row 0's sum is dP[0, 0] and
+    dP[0, 1] - dP[0, 0] overflows."""
+    from rac_amd import ext
+    q, k, v, g = inputs(1, 1, 8, 4096)
+    big = 1.5 * 2.0 ** 57
+    v = torch.full_like(v, big)
+    v[:, :, 1::2] = -big
+    g = torch.full_like(g, big)
+    _, P = ext.attention(q, k, v, None, True, iters=16, mode=ext.MODE_FAST, return_probs=True)
+    want = composed(q, k, v, P, g, ext.MODE_FAST)
+    assert want[1].isnan().any()
+    got = [torch.empty_like(q) for _ in range(3)]
+    ext.attention_backward(q, k, v, P, g, True, *got)
+    for a, b in zip(got, want):
+        assert torch.equal(a.isnan(), b.isnan())
