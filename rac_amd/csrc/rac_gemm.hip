@@ -160,8 +160,9 @@ __global__ __launch_bounds__(256) void gemm_kernel(
         uint32_t a_hi = 0u, a_lo_m1 = 0xffffffffu;
 
         // Global -> register staging of one K-tile; element (m, k) of op(A) and
-        // (k, n) of op(B), zero outside the matrix.  Index order is chosen so
-        // consecutive lanes read consecutive addresses.
+        // (k, n) of op(B), zero outside the matrix (FAST: -0 in A, so that the
+        // product -0 leaves a -0 accumulator as it is too).  Index order is
+        // chosen so consecutive lanes read consecutive addresses.
         auto load_tile = [&](int k0) {
 #pragma unroll
             for (int r = 0; r < Cfg::kALoads; r++) {
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(
                 if constexpr (TA) { kk = idx / BM; mm = idx % BM; }
                 else { mm = idx / BK; kk = idx % BK; }
                 const long gm = m0 + mm, gk = (long)k0 + kk;
-                float v = 0.0f;
+                float v = MODE == kModeFast ? -0.0f : 0.0f;
                 if (gm < M && gk < K) v = TA ? A[gk * M + gm] : A[gm * K + gk];
                 ra[r] = v;
             }
@@ -212,8 +213,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(
 
         // Causal P V: row t of P is exactly 0 beyond column t, and with every v
         // finite (*k_causal == 1, checked on the device) fma(0, v, acc) == acc
-        // (acc starts at +0 and can never become -0), so the K loop stops after
-        // the tile's last row (query position row0 + m0 + BM - 1).
+        // (a zero accumulator at most changes its sign), so the K loop stops
+        // after the tile's last row (query position row0 + m0 + BM - 1).
         int kend = K;
         if (k_causal && *k_causal == 1) kend = (int)min((long)K, (long)row0 + m0 + BM);
         load_tile(0);

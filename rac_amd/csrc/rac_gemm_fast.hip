@@ -29,7 +29,8 @@ typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
 // half-precision linear layer, widened (exactly) on the way to LDS and
 // rounded to nearest even on the way out: what converting whole tensors
 // before and after would give, without their passes over memory.
-// Q: four elements as loaded; shifted(): the first `sh` dropped, zeros behind.
+// Q: four elements as loaded; shifted(): the first `sh` dropped, zeros behind
+// (NEG: negative ones).
 struct Bf16 { uint16_t bits; };
 struct F16 { uint16_t bits; };
 typedef uint32_t u2a __attribute__((ext_vector_type(2), aligned(2)));
@@ -45,10 +46,12 @@ struct Elem<float> {
         return v4f{t.x, t.y, t.z, t.w};
     }
     static __device__ __forceinline__ v4f widen(Q v) { return v; }
+    template <bool NEG>
     static __device__ __forceinline__ Q shifted(Q v, int sh) {
-        if (sh & 1) v = v4f{v.y, v.z, v.w, 0.0f};
-        if (sh & 2) v = v4f{v.z, v.w, 0.0f, 0.0f};
-        if (sh & 4) v = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        constexpr float z = NEG ? -0.0f : 0.0f;
+        if (sh & 1) v = v4f{v.y, v.z, v.w, z};
+        if (sh & 2) v = v4f{v.z, v.w, z, z};
+        if (sh & 4) v = v4f{z, z, z, z};
         return v;
     }
     static __device__ __forceinline__ float get(const float* p) { return *p; }
@@ -69,8 +72,11 @@ struct Elem16 {
         const u2a t = *reinterpret_cast<const u2a*>(p);
         return u2v{t.x, t.y};
     }
+    template <bool NEG>
     static __device__ __forceinline__ Q shifted(Q v, int sh) {
-        const uint64_t x = sh >= 4 ? 0 : (((uint64_t)v.y << 32) | v.x) >> (16 * sh);
+        constexpr uint64_t z = NEG ? 0x8000800080008000u : 0;
+        if (sh <= 0) return v;
+        const uint64_t x = sh >= 4 ? z : (((uint64_t)v.y << 32) | v.x) >> (16 * sh) | z << (64 - 16 * sh);
         return u2v{(uint32_t)x, (uint32_t)(x >> 32)};
     }
 };
@@ -160,8 +166,9 @@ struct FastTile {
     }
     // The K-tile at hand has only `kn` (1 .. KT - 1) of its k, and the matrix
     // at least 4: addresses move back inside K; fix_k() then puts the
-    // elements where they belong and zeroes those past K (a zero product
-    // leaves an accumulator as it is: it starts at +0 and never becomes -0).
+    // elements where they belong and zeroes those past K, negative zeros in
+    // one operand: adding the product -0 leaves every accumulator as it is,
+    // the -0 of a chain of underflowed negative products too.
     __device__ __forceinline__ void retreat(int kn, long ld) {
 #pragma unroll
         for (int i = 0; i < kVPT; i++) {
@@ -181,12 +188,13 @@ struct FastTile {
 #pragma unroll
         for (int i = 0; i < kVPT; i++) p[i] += by;
     }
+    template <bool NEG>
     __device__ __forceinline__ static void fix_k(Q (&v)[kVPT], int kn) {
 #pragma unroll
         for (int i = 0; i < kVPT; i++) {
             const int idx = threadIdx.x + i * NL;
-            if constexpr (KC) v[i] = El::shifted(v[i], min(4, max(0, (idx % kPer) * 4 + 4 - kn)));
-            else v[i] = El::shifted(v[i], idx / kPer >= kn ? 4 : 0);
+            if constexpr (KC) v[i] = El::template shifted<NEG>(v[i], min(4, max(0, (idx % kPer) * 4 + 4 - kn)));
+            else v[i] = El::template shifted<NEG>(v[i], idx / kPer >= kn ? 4 : 0);
         }
     }
     // !KC, tiles past the last row: lanes that moved back to stay inside
@@ -194,7 +202,7 @@ struct FastTile {
     __device__ __forceinline__ void fix_rows(Q (&v)[kVPT]) const {
 #pragma unroll
         for (int i = 0; i < kVPT; i++)
-            if constexpr (!THIN) v[i] = El::shifted(v[i], shift);
+            if constexpr (!THIN) v[i] = El::template shifted<false>(v[i], shift);
     }
     __device__ __forceinline__ static void store(float* S, const Q (&q)[kVPT], int i) {
         const int idx = threadIdx.x + i * NL;
@@ -389,8 +397,8 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const T* __rest
     };
     auto fix = [&](int s, int slot) {
         if (tail && s == nfull) {
-            TAt::fix_k(va[slot], tail);
-            TBt::fix_k(vb[slot], tail);
+            TAt::template fix_k<true>(va[slot], tail);
+            TBt::template fix_k<false>(vb[slot], tail);
         }
         if constexpr (TA) if (edge_a) ta.fix_rows(va[slot]);
         if constexpr (!TB) if (edge_b) tb.fix_rows(vb[slot]);

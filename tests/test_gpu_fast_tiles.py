@@ -88,6 +88,36 @@ def test_fast_tile_specials(layout):
     assert np.array_equal(got[~np.isnan(ref)], ref[~np.isnan(ref)])
 
 
+UNDERFLOW = [(17, 17, 4), (20, 18, 1), (31, 32, 63), (33, 65, 80), (63, 129, 15), (129, 8200, 37), (300, 5633, 31),
+             (500, 2049, 70), (1000, 777, 131), (2049, 4095, 33), (1, 31, 130), (3, 2100, 129), (16, 33, 127),
+             (2100, 3, 129), (2, 2, 2), (2, 3, 70)]
+
+
+@pytest.mark.parametrize("layout", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("shape", UNDERFLOW)
+def test_fast_tile_negative_underflow(shape, layout):
+    """Products that all underflow negatively: every fmaf of the chain rounds
+    to -0, and the k that a tile adds past K must leave it so."""
+    M, N, K = shape
+    ta, tb = layout
+    print(f"fast tile underflow shape={shape} layout={layout}", flush=True)
+    A = np.full((K, M) if ta else (M, K), -1e-30, np.float32)
+    B = np.full((N, K) if tb else (K, N), 1e-30, np.float32)
+    got = run(A, B, np.zeros((M, N), np.float32), M, N, K, ta, tb, 1.0, 0.0)
+    assert (got.view(np.uint32) == 0x80000000).all()
+
+
+@pytest.mark.parametrize("shape", [(3, 70, 37), (33, 65, 80), (301, 5632, 130)])
+def test_half_linear_negative_underflow(shape):
+    """The same through the 16-bit linear layer."""
+    from rac_amd import ext
+    M, N, K = shape
+    x = torch.full((M, K), -1e-30, device=DEV, dtype=torch.bfloat16)
+    w = torch.full((N, K), 1e-30, device=DEV, dtype=torch.bfloat16)
+    out = ext.fused_linear_forward(x, w, None, 0, mode=ext.MODE_FAST)
+    assert (out.view(torch.int16) == -0x8000).all()
+
+
 @pytest.mark.parametrize("act", [0, 1, 2, 3])
 @pytest.mark.parametrize("shape", [(18, 35, 70), (130, 2050, 40), (700, 1027, 36)])
 def test_fast_tile_fused_epilogue(shape, act):
