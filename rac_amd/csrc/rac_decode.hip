@@ -249,10 +249,11 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
         if (wave + kDecWaves * u < n16) kload(wave + kDecWaves * u, kf[u]);
 
     // P V's values, group of 16 positions b: V[16 b + 4 t + lq][16 wave + li],
-    // the last, partial group apart (zero past the row)
+    // the last, partial group apart (-0 past the row: times the probability 0
+    // there it leaves every accumulator as it is, -0 too)
     const bool pv_wave = wave < DF;
     const int nf = n / 16;
-    v4f vr[kDecAhead], vt = {0.0f, 0.0f, 0.0f, 0.0f};
+    v4f vr[kDecAhead], vt = {-0.0f, -0.0f, -0.0f, -0.0f};
     const uint32_t voff = (uint32_t)(lq * DH + 16 * wave + li) * 4u;
     auto vload = [&](int b) {
         const char* base = reinterpret_cast<const char*>(V + (long)b * 16 * DH);

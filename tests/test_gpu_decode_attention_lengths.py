@@ -65,3 +65,16 @@ def test_decode_attention_special_rows(n):
     assert np.all(np.isinf(got[:, 5])) and np.all(np.isfinite(np.delete(got, 5, 1)))
     K[:, n // 2, 7] = np.nan
     assert np.all(np.isnan(run(q, K, V, n, heads, scale, 24)))
+
+
+@pytest.mark.parametrize("dh", [32, 64, 128, 80])
+@pytest.mark.parametrize("n", [3, 5, 16, 21, 40, 1030])
+def test_decode_attention_negative_underflow(n, dh):
+    """Equal probabilities times the smallest negative subnormal underflow to
+    -0 at every position: the group's positions past the row leave it so."""
+    heads, kv, t_cap = 2, 1, 1040
+    K = rl.gen_normal((kv, t_cap, dh), seed=1)
+    V = np.full((kv, t_cap, dh), -1e-45, F32)
+    print(f"decode attention underflow n={n} dh={dh}", flush=True)
+    got = run(np.zeros(heads * dh, F32), K, V, n, heads, F32(0.125), 24)
+    assert np.all(got.view(np.uint32) == 0x80000000)
