@@ -44,8 +44,8 @@ __device__ __forceinline__ void dec_exp4(float* v, int iters, float khinv) {
 // V tile staged in LDS for the P V chains: kDecTile floats (16 KB)
 constexpr int kDecTile = 4096;
 
-// Any d_head and alignment (the shapes the matrix-core kernel below does not
-// take): one workgroup per query head.
+// Any d_head (those the matrix-core kernel below does not take): one
+// workgroup per query head.
 // Scores: lane t computes positions t, t + 256, ... (one fmaf chain each).  Softmax:
 // lane l takes the groups l, l + 256, ... as the row kernel.  P V: the
 // value rows pass through LDS a tile at a time (every lane loads, the next
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kRowThreads) void decode_attention_kernel(
     if (tid < dh) o[tid] = acc;
 }
 
-// ── the same on the matrix cores (d_head 32, 64, 128; 16-byte rows) ──────
+// ── the same on the matrix cores (d_head 32, 64, 128) ────────────────────
 //
 // One workgroup of 16 waves per query head.  Every chain of the form above is
 // kept, four k per instruction: a 16x16x4 matrix instruction is four in-order
@@ -197,6 +197,9 @@ __global__ __launch_bounds__(kRowThreads) void decode_attention_kernel(
 // workgroup (one reading of the keys for them) were slower: 12.6 us at 516,
 // the exps of all four being on one CU.
 typedef float v4f __attribute__((ext_vector_type(4)));
+// the same at any 4-byte boundary (global_load / store_dwordx4 need no more):
+// every alignment of the queries, the caches and the output runs here
+typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kDecWaves = 16, kDecThreads = 64 * kDecWaves;
 constexpr int kDecExps = kDecodeMaxLen / kDecThreads;       // positions per lane at most
 
@@ -238,12 +241,12 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
 #pragma unroll
             for (int i = 0; i < VECS; i++) {
                 const int v = lane + 64 * i;
-                f[h * VECS + i] = *reinterpret_cast<const v4f*>(
+                f[h * VECS + i] = *reinterpret_cast<const v4u*>(
                     K + (long)min(16 * b + v / (KP / 4), n - 1) * DH + h * KP + 4 * (v % (KP / 4)));
             }
     };
     float* skw = sk[wave];
-    const v4f q4 = *reinterpret_cast<const v4f*>(q + (long)h * DH + 4 * (lane % (DH / 4)));
+    const v4f q4 = *reinterpret_cast<const v4u*>(q + (long)h * DH + 4 * (lane % (DH / 4)));
 #pragma unroll
     for (int u = 0; u < kDecTiles; u++)
         if (wave + kDecWaves * u < n16) kload(wave + kDecWaves * u, kf[u]);
@@ -428,12 +431,12 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
                 p = probs(min(b0 + u + 1, n16 - 1));
             }
         if (nf < n16) mac(p, vt);
-        if (li == 0) *reinterpret_cast<v4f*>(out + (long)h * DH + 16 * wave + 4 * lq) = acc;
+        if (li == 0) *reinterpret_cast<v4u*>(out + (long)h * DH + 16 * wave + 4 * lq) = acc;
     }
 }
 
 template <int NITER>
-static hipError_t decode_attention_dh(int dh, bool vec, const float* q, const float* kc, const float* vc,
+static hipError_t decode_attention_dh(int dh, const float* q, const float* kc, const float* vc,
                                       float* out, int n_heads, int rep, long t_cap, const int* pos, float scale,
                                       int iters, float khinv, hipStream_t s) {
 #define RAC_DEC_ATT(D, E)                                                                                         \
@@ -444,9 +447,9 @@ static hipError_t decode_attention_dh(int dh, bool vec, const float* q, const fl
         if (t_cap <= 2 * kDecThreads) RAC_DEC_ATT(D, 2); \
         else RAC_DEC_ATT(D, kDecExps);             \
     } while (0)
-    if (vec && dh == 64) RAC_DEC_ATT_LEN(64);
-    else if (vec && dh == 128) RAC_DEC_ATT_LEN(128);
-    else if (vec && dh == 32) RAC_DEC_ATT_LEN(32);
+    if (dh == 64) RAC_DEC_ATT_LEN(64);
+    else if (dh == 128) RAC_DEC_ATT_LEN(128);
+    else if (dh == 32) RAC_DEC_ATT_LEN(32);
     else
         hipLaunchKernelGGL((decode_attention_kernel<NITER>), dim3(n_heads), dim3(kRowThreads), 0, s, q, kc, vc, out,
                            rep, dh, t_cap, pos, scale, iters, khinv);
@@ -461,15 +464,11 @@ hipError_t decode_attention_launch(const float* q, const float* kc, const float*
     iters = clamp_iters(iters);
     const float khinv = host_consts().exp_khinv[iters];
     const int rep = n_heads / n_kv_heads;
-    // 16-byte loads of query and key rows, 16-byte stores of the output
-    const uintptr_t any = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kc) |
-                          reinterpret_cast<uintptr_t>(vc) | reinterpret_cast<uintptr_t>(out);
-    const bool vec = (any & 15) == 0;
     switch (iters) {
-        case 8: return decode_attention_dh<8>(dh, vec, q, kc, vc, out, n_heads, rep, t_cap, pos, scale, iters, khinv, s);
-        case 16: return decode_attention_dh<16>(dh, vec, q, kc, vc, out, n_heads, rep, t_cap, pos, scale, iters, khinv, s);
-        case 24: return decode_attention_dh<24>(dh, vec, q, kc, vc, out, n_heads, rep, t_cap, pos, scale, iters, khinv, s);
-        default: return decode_attention_dh<0>(dh, vec, q, kc, vc, out, n_heads, rep, t_cap, pos, scale, iters, khinv, s);
+        case 8: return decode_attention_dh<8>(dh, q, kc, vc, out, n_heads, rep, t_cap, pos, scale, iters, khinv, s);
+        case 16: return decode_attention_dh<16>(dh, q, kc, vc, out, n_heads, rep, t_cap, pos, scale, iters, khinv, s);
+        case 24: return decode_attention_dh<24>(dh, q, kc, vc, out, n_heads, rep, t_cap, pos, scale, iters, khinv, s);
+        default: return decode_attention_dh<0>(dh, q, kc, vc, out, n_heads, rep, t_cap, pos, scale, iters, khinv, s);
     }
 }
 

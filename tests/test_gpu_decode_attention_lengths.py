@@ -78,3 +78,28 @@ def test_decode_attention_negative_underflow(n, dh):
     print(f"decode attention underflow n={n} dh={dh}", flush=True)
     got = run(np.zeros(heads * dh, F32), K, V, n, heads, F32(0.125), 24)
     assert np.all(got.view(np.uint32) == 0x80000000)
+
+
+@pytest.mark.parametrize("dh", [32, 64, 128])
+@pytest.mark.parametrize("which", ["q", "k", "v", "out"])
+def test_decode_attention_alignment(dh, which):
+    """Any 4-byte boundary of the queries, either cache and the output gives
+    the bits of the 16-byte one, and writes the output's elements alone."""
+    from rac_amd import ext
+    heads, kv, t_cap, n = 4, 2, 300, 277
+    K, V = (rl.gen_normal((kv, t_cap, dh), seed=s) for s in (1, 2))
+    q = rl.gen_normal((heads * dh,), seed=3)
+    want = orc_decode_attention(q, K, V, n, heads, F32(0.125), 24)
+    pos = torch.tensor([n - 1], dtype=torch.int32, device="cuda")
+    for off in (1, 2, 3):
+        print(f"decode attention alignment dh={dh} {which} off={off}", flush=True)
+        t = {"q": torch.from_numpy(q), "k": torch.from_numpy(K), "v": torch.from_numpy(V),
+             "out": torch.zeros(heads * dh)}
+        buf = torch.full((t[which].numel() + 4,), float("nan"), device="cuda")
+        t = {name: x.cuda() for name, x in t.items()}
+        view = buf[off:off + t[which].numel()].view(t[which].shape)
+        view.copy_(t[which])
+        t[which] = view
+        ext.decode_attention(t["q"], t["k"], t["v"], pos, heads, 0.125, 24, out=t["out"])
+        assert np.array_equal(t["out"].cpu().numpy(), want)
+        assert torch.isnan(buf[:off]).all() and torch.isnan(buf[off + view.numel():]).all()
