@@ -191,20 +191,23 @@ __global__ __launch_bounds__(kRowThreads) void decode_attention_kernel(
 //            positions in flight from before the scores on, go straight to
 //            the instruction: 10-14 cycles per position of the chain, where a
 //            lane of the VALU form took ~35 (its fmaf, its LDS reads).
-// Replayed in a graph (32 heads over 4, d_head 64), before -> now: length 1
-// 4.0 -> 4.3, 256 8.6 -> 6.7, 516 14.7 -> 10.3, 2047 46.7 -> 29.1 us (d_head
-// 128: 4.4 -> 4.9, 11.8 -> 9.6, 21.5 -> 16.2, 75.3 -> 50.7).  Four heads to a
-// workgroup (one reading of the keys for them) were slower: 12.6 us at 516,
-// the exps of all four being on one CU.
+// The softmax loops over the lanes' positions, its values in LDS: held in
+// registers (2 or, in caches of more than 2048 positions, 8 to a lane) its
+// unrolled stages cost a short row the instruction fetches of all 8, d_head 64
+// at length 16 4.45 us against 3.96.
+// Replayed in a graph (32 heads over 4, d_head 64, any cache length), one
+// workgroup of 4 waves on the VALU before -> now: length 1 3.9 -> 3.7, 256 8.5
+// -> 6.3, 516 14.6 -> 9.8, 2047 46.7 -> 28.8 us (d_head 128: 4.3 -> 4.2, 11.7
+// -> 9.0, 21.3 -> 15.6, 75.7 -> 48.9).  Four heads to a workgroup (one reading
+// of the keys for them) were slower: 12.6 us at 516, the exps of all four
+// being on one CU.
 typedef float v4f __attribute__((ext_vector_type(4)));
 // the same at any 4-byte boundary (global_load / store_dwordx4 need no more):
 // every alignment of the queries, the caches and the output runs here
 typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kDecWaves = 16, kDecThreads = 64 * kDecWaves;
-constexpr int kDecExps = kDecodeMaxLen / kDecThreads;       // positions per lane at most
 
-// EMAX: lanes hold up to EMAX positions (caches of up to 1024 EMAX)
-template <int NITER, int DH, int EMAX>
+template <int NITER, int DH>
 __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
     const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
     float* __restrict__ out, int rep, long t_cap, const int* __restrict__ pos_dev, float scale, int iters,
@@ -214,7 +217,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
     // a wave's key staging: 16 rows of KP floats (a row, or half a long one)
     constexpr int KP = DH < 64 ? DH : 64, KR = KP + 8, PARTS = DH / KP, VECS = KP / 16;
     __shared__ __attribute__((aligned(16))) float sk[kDecWaves][16 * KR];
-    __shared__ __attribute__((aligned(16))) float sp[kDecThreads * EMAX];
+    __shared__ __attribute__((aligned(16))) float sp[kDecodeMaxLen];
     __shared__ __attribute__((aligned(16))) float rmax[kDecWaves];
     __shared__ __attribute__((aligned(16))) uint32_t rzero[kDecWaves];
     __shared__ float rsum[kRowWaves];
@@ -335,20 +338,16 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
 
     // row maximum; a zero maximum takes the sign of the row's first zero
     // (first_zero_max)
-    float e[EMAX];
     float m = -__builtin_inff();
-#pragma unroll
-    for (int i = 0; i < EMAX; i++) {
-        const int j = tid + kDecThreads * i;
-        e[i] = j < n ? sp[j] : -__builtin_inff();
-        m = fmaxf(m, e[i]);
-    }
+    for (int j = tid; j < n; j += kDecThreads) m = fmaxf(m, sp[j]);
     m = wave_max_valu(m);
     uint32_t key = ~0u;
     if (m == 0.0f) {
-#pragma unroll
-        for (int i = EMAX - 1; i >= 0; i--)
-            if (e[i] == 0.0f) key = zero_key<uint32_t>(tid + kDecThreads * i, e[i]);
+        for (int j = tid; j < n; j += kDecThreads)
+            if (sp[j] == 0.0f) {
+                key = zero_key<uint32_t>(j, sp[j]);
+                break;
+            }
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) key = min(key, (uint32_t)__shfl_xor((int)key, off, 64));
     }
@@ -367,19 +366,14 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
         m = (key & 1) ? -0.0f : 0.0f;
     }
 
-    // exps; a NaN score stays NaN and makes the row's sum, and every
-    // probability, NaN
-#pragma unroll
-    for (int i = 0; i < EMAX; i++) {
-        const int j = tid + kDecThreads * i;
-        if (j < 4 * n4) {
-            float v[1] = {e[i] - m};
-            const bool nan = v[0] != v[0];
-            if constexpr (NITER > 0) exp_cordic_vec<NITER, 1, kExpFlush | kExpNonPos>(v, khinv);
-            else v[0] = exp_cordic_rt(v[0], iters, khinv);
-            e[i] = nan ? __builtin_nanf("") : v[0];
-            sp[j] = e[i];
-        }
+    // exps, of the -inf up to the last group of four too; a NaN score stays
+    // NaN and makes the row's sum, and every probability, NaN
+    for (int j = tid; j < 4 * n4; j += kDecThreads) {
+        float v[1] = {sp[j] - m};
+        const bool nan = v[0] != v[0];
+        if constexpr (NITER > 0) exp_cordic_vec<NITER, 1, kExpFlush | kExpNonPos>(v, khinv);
+        else v[0] = exp_cordic_rt(v[0], iters, khinv);
+        sp[j] = nan ? __builtin_nanf("") : v[0];
     }
     __syncthreads();
     if (tid < kRowThreads) {
@@ -397,10 +391,11 @@ __global__ __launch_bounds__(kDecThreads) void decode_attention_mfma_kernel(
 #pragma unroll
     for (int i = 1; i < kRowWaves; i++) s += rsum[i];
     const float inv = 1.0f / s;
-#pragma unroll
-    for (int i = 0; i < EMAX; i++) {
-        const int j = tid + kDecThreads * i;
-        if (j < 16 * n16) sp[(j & ~15) + 4 * (j & 3) + ((j >> 2) & 3)] = j < n ? e[i] * inv : 0.0f;
+    // permuted within groups of 16, which a wave reads and writes as a whole
+    for (int j = tid; j < 16 * n16; j += kDecThreads) {
+        const float v = j < n ? sp[j] * inv : 0.0f;
+        own_lds();
+        sp[(j & ~15) + 4 * (j & 3) + ((j >> 2) & 3)] = v;
     }
     __syncthreads();
 
@@ -439,21 +434,15 @@ template <int NITER>
 static hipError_t decode_attention_dh(int dh, const float* q, const float* kc, const float* vc,
                                       float* out, int n_heads, int rep, long t_cap, const int* pos, float scale,
                                       int iters, float khinv, hipStream_t s) {
-#define RAC_DEC_ATT(D, E)                                                                                         \
-    hipLaunchKernelGGL((decode_attention_mfma_kernel<NITER, D, E>), dim3(n_heads), dim3(kDecThreads), 0, s, q, kc, \
+#define RAC_DEC_ATT(D)                                                                                         \
+    hipLaunchKernelGGL((decode_attention_mfma_kernel<NITER, D>), dim3(n_heads), dim3(kDecThreads), 0, s, q, kc, \
                        vc, out, rep, t_cap, pos, scale, iters, khinv)
-#define RAC_DEC_ATT_LEN(D)                         \
-    do {                                           \
-        if (t_cap <= 2 * kDecThreads) RAC_DEC_ATT(D, 2); \
-        else RAC_DEC_ATT(D, kDecExps);             \
-    } while (0)
-    if (dh == 64) RAC_DEC_ATT_LEN(64);
-    else if (dh == 128) RAC_DEC_ATT_LEN(128);
-    else if (dh == 32) RAC_DEC_ATT_LEN(32);
+    if (dh == 64) RAC_DEC_ATT(64);
+    else if (dh == 128) RAC_DEC_ATT(128);
+    else if (dh == 32) RAC_DEC_ATT(32);
     else
         hipLaunchKernelGGL((decode_attention_kernel<NITER>), dim3(n_heads), dim3(kRowThreads), 0, s, q, kc, vc, out,
                            rep, dh, t_cap, pos, scale, iters, khinv);
-#undef RAC_DEC_ATT_LEN
 #undef RAC_DEC_ATT
     return hipGetLastError();
 }

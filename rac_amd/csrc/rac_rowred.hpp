@@ -30,7 +30,7 @@ __device__ __forceinline__ float wave_max(float v) {
 // once lanes i and i ^ 2 OFF agree, i + OFF and i ^ OFF do.  The same pairs,
 // and bits, as a shuffle by OFF, whose trip through LDS takes ~100 cycles a
 // step: for kernels that wait on one row's reduction (the decode attention:
-// 4.26 -> 3.96 us at one position).  The row kernels, which have other rows'
+// 0.3 us of 4.0 at one position).  The row kernels, which have other rows'
 // waves to run meanwhile, keep the shuffles: softmax 4096 x 4096 was slower
 // without (n = 16 28.5 -> 30.9 us, n = 24 32.1 -> 36.1).
 template <int OFF, class Op>

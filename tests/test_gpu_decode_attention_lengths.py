@@ -1,7 +1,7 @@
 """GPU parity of the decode attention's matrix-core form (d_head 32, 64, 128)
-at cache lengths around its 16-position groups, the rounds of its 16 waves,
-its lanes' 1024 positions and the two LDS sizes, bit for bit against the
-oracle's composition; and with special keys and values next to the row's end.
+at cache lengths around its 16-position groups, the rounds of its 16 waves and
+its lanes' rounds of 1024 positions, bit for bit against the oracle's
+composition; and with special keys and values next to the row's end.
 """
 import numpy as np
 import pytest
