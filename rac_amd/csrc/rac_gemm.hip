@@ -487,8 +487,10 @@ static hipError_t launch_tiles(const GemmArgs& g, hipStream_t s) {
         // two 64x64 blocks per CU (2 waves per SIMD, 16 MAC chains each)
         // still beat 32x32 blocks (measured, same bits: 512-1023 blocks 5-6%
         // faster, e.g. the attention core's P V chunks 32 x 512 x 128 x K; at
-        // one block per CU 43% slower)
-        if (tiles >= 2 * device_cus())
+        // one block per CU 43% slower).  FAST comes here with a few k only,
+        // when the stores bound it: 4 blocks per CU (800 x 3913 x 1, 806
+        // blocks: 9.5 us on 64x64, 7.7 on 32x32)
+        if (tiles >= (MODE == kModeFast ? 4 : 2) * device_cus())
             return launch_cfg<MODE, NITER, TA, TB, FUSED, SCHED, 4>(g, s);
         return launch_cfg<MODE, NITER, TA, TB, FUSED, SCHED, 2>(g, s);
     }

@@ -39,7 +39,7 @@ def run(A, B, C0, M, N, K, ta, tb, alpha, beta):
     return Cd.cpu().numpy()
 
 
-SHAPES = [(17, 17, 4), (17, 33, 3), (20, 18, 1), (31, 32, 63), (33, 65, 64), (32, 31, 65), (63, 129, 15),
+SHAPES = [(17, 17, 4), (17, 33, 3), (20, 18, 1), (801, 3913, 1), (2050, 2041, 3), (31, 32, 63), (33, 65, 64), (32, 31, 65), (63, 129, 15),
           (65, 64, 129), (127, 200, 16), (128, 257, 17), (129, 8200, 37), (300, 5633, 31), (500, 2049, 70),
           (1000, 777, 131), (2047, 2177, 19), (2049, 4095, 33),
           # few rows or columns: one, the 2 and 3 of a thin operand, 16; blocks
