@@ -119,7 +119,8 @@ def test_half_linear_negative_underflow(shape):
 
 
 @pytest.mark.parametrize("act", [0, 1, 2, 3])
-@pytest.mark.parametrize("shape", [(18, 35, 70), (130, 2050, 40), (700, 1027, 36)])
+@pytest.mark.parametrize("shape", [(18, 35, 70), (130, 2050, 40), (700, 1027, 36), (1, 3, 40), (1, 11009, 64), (3, 2035, 70),
+                                   (550, 2, 33)])
 def test_fast_tile_fused_epilogue(shape, act):
     """Bias, the kept pre-activation and the activation: those of the plain
     product's output."""
