@@ -518,7 +518,15 @@ static hipError_t dispatch(int ta, int tb, int mode, const GemmArgs& g, hipStrea
         // 16-byte loads cannot read, and where both operands hold 2 or 3 rows
         // side by side
         const bool thin_a = ta && g.M > 1 && g.M < 4, thin_b = !tb && g.N > 1 && g.N < 4;
-        if (g.K >= 4 && !(thin_a && thin_b)) return gemm_fast_launch(ta, tb, g, s);
+        // and for up to 16 k, one K-tile, of up to 2^21 outputs, bound by the
+        // start of a launch, which is shorter there: 300 x 300 x 9 2.7 us against
+        // 3.1, 679 x 1739 x 16 4.6 against 6.3, 12 x 300 TN x 9 2.5 against 3.5;
+        // past them the stores dominate, which the other tiles make in 16 bytes
+        // (1166 x 3868 x 9 11.8 us against 8.2).  Not for SiLU, whose epilogue
+        // there has four exps in flight (300 x 300 x 9 7.3 us against 4.1).
+        const bool few_k = g.K <= 16 && (long)g.M * g.N * g.batch <= (1L << 21) && g.sched == 0 && !g.k_causal &&
+                           g.k_side != 3 && !(g.fused && g.ep.act == kActSilu);
+        if (g.K >= 4 && !(thin_a && thin_b) && !few_k) return gemm_fast_launch(ta, tb, g, s);
         return launch_layout<kModeFast, 0>(ta, tb, g, s);
     }
     // few rows or columns (schedule 2, the causal P V, is then the plain

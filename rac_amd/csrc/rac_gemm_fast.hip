@@ -277,24 +277,26 @@ __device__ __forceinline__ void fast_epilogue(T* __restrict__ C, int M, int N, l
         }
         if (g.ep.pre && in) Elem<float>::store(g.ep.pre + gm * N + gn, v, left);
         float x[4] = {v.x, v.y, v.z, v.w};
-        if (g.ep.act == kActRelu) {
-            elt_vec<kEltRelu, 0, 4>(x, 0, 0.0f);
+        if (g.ep.act == kActSilu) {
+            if (g.iters == 24) {
+                elt_vec<kEltSilu, 24, 4>(x, g.iters, g.ep.khinv);
+            } else if (g.iters == 16) {
+                elt_vec<kEltSilu, 16, 4>(x, g.iters, g.ep.khinv);
+            } else {
+                // one copy: x rotates
+#pragma unroll 1
+                for (int r = 0; r < 4; r++) {
+                    const float y = act_rt(x[0], kActSilu, g.iters, g.ep.khinv);
+                    x[0] = x[1];
+                    x[1] = x[2];
+                    x[2] = x[3];
+                    x[3] = y;
+                }
+            }
         } else if (g.ep.act == kActGelu) {
             elt_vec<kEltGelu, 0, 4>(x, 0, 0.0f);
-        } else if (g.ep.act == kActSilu && g.iters == 24) {
-            elt_vec<kEltSilu, 24, 4>(x, g.iters, g.ep.khinv);
-        } else if (g.ep.act == kActSilu && g.iters == 16) {
-            elt_vec<kEltSilu, 16, 4>(x, g.iters, g.ep.khinv);
-        } else if (g.ep.act == kActSilu) {
-            // other step counts, one copy: x rotates
-#pragma unroll 1
-            for (int r = 0; r < 4; r++) {
-                const float y = act_rt(x[0], kActSilu, g.iters, g.ep.khinv);
-                x[0] = x[1];
-                x[1] = x[2];
-                x[2] = x[3];
-                x[3] = y;
-            }
+        } else if (g.ep.act == kActRelu) {
+            elt_vec<kEltRelu, 0, 4>(x, 0, 0.0f);
         }
         v = v4f{x[0], x[1], x[2], x[3]};
         if (!in) return;
@@ -394,7 +396,9 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const T* __rest
     typename TAt::Q va[PD][VA];
     typename TBt::Q vb[PD][VB];
     const int kn = kend - kbeg, nfull = kn / KT, tail = kn - nfull * KT, nst = nfull + (tail ? 1 : 0);
-    const bool edge_a = TA && m0 + BM > M, edge_b = !TB && n0 + BN > N;
+    // only a vector across the edge holds rows of the matrix elsewhere than
+    // its lanes store them
+    const bool edge_a = TA && m0 + BM > M && M % 4, edge_b = !TB && n0 + BN > N && N % 4;
     // before K-tile s is loaded / after (tiles past the last reload it: the
     // loads stay unconditional, so the waits stay exact)
     auto before = [&](int s) {
@@ -434,7 +438,9 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const T* __rest
         }
     };
     // the MACs of the K-tile in LDS buffer `buf`; `staged`: with the
-    // next tile's staging, ahead of them (SPREAD 0) or spread over them
+    // next tile's staging, ahead of them (SPREAD 0) or spread over them; else
+    // the last tile's, the 16-k groups that it has
+    const int last_groups = (kn - (nst - 1) * KT + 15) / 16;
     auto compute = [&](int buf, auto staged, int slot, bool ld) {
         constexpr int Q = KT / 16, X = VA + VB;
         v4f fa[2][MT], fb[2][NT];
@@ -445,6 +451,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const T* __rest
         frags(buf, 0, fa[0], fb[0]);
 #pragma unroll
         for (int q = 0; q < Q; q++) {
+            if (Q > 1 && !decltype(staged)::value && q >= last_groups) break;
             if (q + 1 < Q) frags(buf, q + 1, fa[(q + 1) & 1], fb[(q + 1) & 1]);
 #pragma unroll
             for (int t = 0; t < 4; t++) {
@@ -462,7 +469,20 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const T* __rest
             }
         }
     };
-    if (any_k) {
+    if (KT > 16 && any_k && nst == 1) {
+        // all of K in one tile: no other to load (4 x 300 x 48 3.6 us, 3.9 with
+        // the last tile loaded again in its place)
+        before(0);
+#pragma unroll
+        for (int x = 0; x < VA; x++) ta.load(va[0], x);
+#pragma unroll
+        for (int x = 0; x < VB; x++) tb.load(vb[0], x);
+        fix(0, 0);
+#pragma unroll
+        for (int x = 0; x < VA + VB; x++) stage(0, 0, x, false);
+        __syncthreads();
+        compute(0, std::false_type(), 0, false);
+    } else if (any_k) {
 #pragma unroll
         for (int s = 0; s < PD; s++) {
             before(s);
@@ -583,6 +603,14 @@ static hipError_t fast_tile(const GemmArgs& a, hipStream_t s) {
     }
     constexpr bool KC2 = !TA && TB, KC0 = TA && !TB;      // both / neither operand k-contiguous
 #define RAC_FAST(...) return fast_launch<TA, TB, FUSED, TRAP, __VA_ARGS__, false, T>(a, s)
+    // Few k for many outputs: the 64-k tiles would load and stage mostly what
+    // is not there (1166 x 3868 x 24 16.3 us on 32x64 x 64 k, here 9.4; x 64
+    // 16.7 against 12.9; 679 x 1739 x 24 6.6 against 5.3).  With fewer outputs
+    // a CU has a tile or two, and one load of all k is the quicker start: 679
+    // x 1739 x 48 with a bias 6.6 us against 7.3, 280 x 7066 x 64 8.3 against
+    // 9.0; the two meet near 2^20 outputs at 32 k, 2^21 at 64.
+    if (!TRAP && best >= 2 && a.K <= 64 && (long)a.M * a.N * a.batch > (long)std::max(a.K, 32) << 15)
+        RAC_FAST(64, 64, 2, 2, 16, 1, 1);
     switch (best) {
     case 0:
         if constexpr (KC2) RAC_FAST(128, 128, 2, 4, 16, 1, 0);
@@ -620,6 +648,12 @@ static hipError_t fast_few(const GemmArgs& a, hipStream_t s) {
     }
     if constexpr (!TB) {
         if (a.N < 4) RAC_FAST(64, 16, 4, 1, 64, 2, 2, true);
+    }
+    // few k of a transposed A: K-tiles no longer than they are (12 x 300 x 24
+    // TN 2.9 us, on 128 k 3.6)
+    if constexpr (TA) {
+        if (rows && a.K <= 32) RAC_FAST(16, 32, 1, 2, 32, 1, 1, false);
+        if (a.K <= 32) RAC_FAST(32, 16, 2, 1, 32, 1, 1, false);
     }
     if (rows) {
         if (b2 <= cus) RAC_FAST(16, 32, 1, 2, 128, 1, 2, false);

@@ -48,6 +48,12 @@ SHAPES = [(17, 17, 4), (17, 33, 3), (20, 18, 1), (801, 3913, 1), (2050, 2041, 3)
           (33, 1, 64), (2100, 3, 129), (31, 16, 257), (8300, 2, 65), (16500, 7, 131)]
 
 
+# few k: the VALU tiles up to 16, one K-tile with all its 16-k groups or some,
+# the 16-k tiles of many outputs, short K-tiles of a transposed A's few rows
+SHAPES += [(300, 301, 15), (300, 299, 16), (299, 300, 17), (679, 1739, 32), (679, 1739, 33), (1167, 3867, 16),
+           (1167, 3868, 47), (2049, 1030, 64), (12, 300, 32), (13, 301, 33), (301, 7, 17), (4, 62, 48)]
+
+
 @pytest.mark.parametrize("layout", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("shape", SHAPES)
 def test_fast_tile_edges(shape, layout):
