@@ -20,10 +20,9 @@
 // and reads only 2 ds_read_b128 per 16 MACs; the rotations of those MACs
 // advance step-major, so independent FMA chains interleave in each wave's
 // instruction stream.  FAST mode (1 FMA per MAC) runs on the matrix cores
-// (rac_gemm_fast.hip), here only for what those cannot read (K < 4).
-// Launches with fewer than 2 blocks of 64x64 per CU step down to 32x32 (2x2
-// per lane) so
-// every SIMD holds several waves.  The next K-tile is
+// (rac_gemm_fast.hip), here only for few k (dispatch).  Launches with fewer
+// than 2 blocks of 64x64 per CU (FAST: 4) step down to 32x32 (2x2 per lane),
+// so every SIMD holds several waves.  The next K-tile is
 // prefetched into registers while the current one is computed.
 #include <hip/hip_runtime.h>
 #include <atomic>
@@ -512,30 +511,58 @@ static hipError_t launch_layout(int ta, int tb, const GemmArgs& g, hipStream_t s
     return launch_tiles<MODE, NITER, true, true, false>(g, s);
 }
 
+// FAST products of few rows or columns that the few-row kernels run better
+// than the matrix cores: their fold takes 4.6 cycles a k, a matrix instruction
+// 8, and they start sooner, but they spread a long K's loads over fewer lanes
+// and take more workgroups for the same outputs.  Both sides measured (us,
+// few-row kernel / matrix cores), NT unless noted: 4 x 2036 x 64 3.1 / 3.6, x
+// 200 3.8 / 4.7, x 400 5.2 / 5.8, x 512 5.5 / 5.7, x 700 7.0 / 7.2, x 1024 8.8 /
+// 8.1; 3 x 6874 (430 workgroups) x 200 4.1 / 4.8, x 400 5.8 / 6.0; but 1 x 4000
+// x 300 5.2 / 4.9, 16 x 6874 x 64 4.5 / 4.2, 1 x 11008 x 64 5.2 / 3.0.  One row
+// times a matrix stored k by k stays ahead while that is small: 1 x 62 x 4096
+// 25 / 32, 1 x 512 x 4096 24 / 26, 1 x 2048 x 1024 8.6 / 8.7, x 1500 12.4 / 11.9.
+// Batches of at most 16 x 16: 60000 of 8 x 8 x 8 112 / 580 (2000 of 4 x 4 x 4 5.9,
+// on the VALU tiles 7.2).
+static bool fast_few_rows(int tb, const GemmArgs& g) {
+    const long cus = device_cus();
+    const int r = g.M <= kSkinnyMaxRows ? g.M : g.N;
+    const long blocks = (long)((g.M <= kSkinnyMaxRows ? g.N : g.M) + 15) / 16 * g.batch;
+    if (r > kSkinnyMaxRows) return false;
+    if (g.M == 1 && !tb && blocks <= cus / 2 && (long)g.N * g.K * g.batch <= (1L << 21)) return true;
+    if (g.K <= 256 && ((g.M <= 16 && g.N <= 16) || (r >= 2 && r <= 8 && blocks <= 2 * cus))) return true;
+    return g.K <= 512 && blocks <= (r == 1 ? cus / 2 : cus);
+}
+
 static hipError_t dispatch(int ta, int tb, int mode, const GemmArgs& g, hipStream_t s) {
+    auto skinny = [&] {
+        return gemm_skinny_launch({g.A, g.B, g.C, g.M, g.N, g.K, g.alpha, g.beta, g.iters, g.batch, g.sa, g.sb, g.sc,
+                                   g.ep, g.fused, tb != 0, g.k_causal, g.exact_specials, g.row0}, mode, s);
+    };
     if (mode == kModeFast) {
-        // the matrix cores; the VALU tiles for fewer than 4 k, which the
-        // 16-byte loads cannot read, and where both operands hold 2 or 3 rows
-        // side by side
+        if (g.M == 1) ta = 0;                                // vectors
+        if (g.N == 1) tb = 1;
+        const bool plain = g.sched == 0 && !g.k_causal && g.k_side != 3;
+        const bool few_rows = plain && !ta && fast_few_rows(tb, g);
+        // up to 16 k, one K-tile, of up to 2^21 outputs are bound by the start of
+        // a launch, which is shortest on the VALU tiles: 300 x 300 x 9 2.7 us, on
+        // the matrix cores 3.1, 679 x 1739 x 16 4.6 against 6.3, 12 x 300 x 9 2.5
+        // against 3.5 (2.9 on the few-row kernel); past them the stores dominate,
+        // which the matrix-core tiles make in 16 bytes (1166 x 3868 x 9 11.8 us
+        // against 8.2).  Not for SiLU, whose epilogue there has four exps in
+        // flight (300 x 300 x 9 7.3 us against 4.1).
+        const bool few_k = plain && g.K <= 16 && (long)g.M * g.N * g.batch <= (1L << 21) &&
+                           !(g.fused && g.ep.act == kActSilu);
+        // and for fewer than 4 k, which the 16-byte loads cannot read, and where
+        // both operands hold 2 or 3 rows side by side
         const bool thin_a = ta && g.M > 1 && g.M < 4, thin_b = !tb && g.N > 1 && g.N < 4;
-        // and for up to 16 k, one K-tile, of up to 2^21 outputs, bound by the
-        // start of a launch, which is shorter there: 300 x 300 x 9 2.7 us against
-        // 3.1, 679 x 1739 x 16 4.6 against 6.3, 12 x 300 TN x 9 2.5 against 3.5;
-        // past them the stores dominate, which the other tiles make in 16 bytes
-        // (1166 x 3868 x 9 11.8 us against 8.2).  Not for SiLU, whose epilogue
-        // there has four exps in flight (300 x 300 x 9 7.3 us against 4.1).
-        const bool few_k = g.K <= 16 && (long)g.M * g.N * g.batch <= (1L << 21) && g.sched == 0 && !g.k_causal &&
-                           g.k_side != 3 && !(g.fused && g.ep.act == kActSilu);
+        if (few_rows && (!few_k || (g.M <= 16 && g.N <= 16 && g.batch > device_cus()))) return skinny();
         if (g.K >= 4 && !(thin_a && thin_b) && !few_k) return gemm_fast_launch(ta, tb, g, s);
         return launch_layout<kModeFast, 0>(ta, tb, g, s);
     }
     // few rows or columns (schedule 2, the causal P V, is then the plain
     // product with its causal K limit, which those kernels apply)
-    if ((g.sched == 0 || g.sched == 2) && !ta && (g.M <= kSkinnyMaxRows || g.N <= kSkinnyMaxRows)) {
-        const SkinnyArgs k{g.A, g.B, g.C, g.M, g.N, g.K, g.alpha, g.beta, g.iters, g.batch, g.sa, g.sb, g.sc,
-                           g.ep, g.fused, tb != 0, g.k_causal, g.exact_specials, g.row0};
-        return gemm_skinny_launch(k, mode, s);
-    }
+    if ((g.sched == 0 || g.sched == 2) && !ta && (g.M <= kSkinnyMaxRows || g.N <= kSkinnyMaxRows))
+        return skinny();
     if (mode == kModeShiftAdd) return launch_layout<kModeShiftAdd, 0>(ta, tb, g, s);
     switch (g.iters) {
         case 8: return launch_layout<kModeCordic, 8>(ta, tb, g, s);

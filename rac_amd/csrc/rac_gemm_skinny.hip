@@ -1,7 +1,8 @@
 // rac_gemm_skinny.hip — the RAC GEMM for products with few rows of op(A)
 // (M <= 16: decode-time linears, one token or a few) or few columns
-// (N <= 16: a matrix-vector product, a classifier head), CORDIC and SHIFTADD
-// MACs (FAST runs on the matrix cores, rac_gemm_fast.hip).
+// (N <= 16: a matrix-vector product, a classifier head): CORDIC and SHIFTADD,
+// and FAST where K is short (fast_few_rows in rac_gemm.hip; the others on the
+// matrix cores, rac_gemm_fast.hip).
 //
 // Each output is ONE accumulator over k = 0..K-1 in order (rac_fma_iters,
 // rac_kernels.hip:204-219), so such a product has only M * N serial chains.
@@ -18,9 +19,10 @@
 //     time: CORDIC the rotation of (a ^ sign(b), 0) and its gain correction
 //     p = R_n(.) * (1/K-hat(n)) (rac_kernels.hip:140-185; the literal chain
 //     for inputs outside the strength-reduced one's range, as gemm_kernel),
-//     SHIFTADD the shift-add product (rac_kernels.hip:85-122);
+//     SHIFTADD the shift-add product (rac_kernels.hip:85-122); FAST has no
+//     term to prepare;
 //   * lane m * CB + n folds output (m, n) over the tile's k in order:
-//     fma(p, |b|, acc) or acc + prod, exactly the MAC of
+//     fma(p, |b|, acc), acc + prod or fma(a, b, acc), exactly the MAC of
 //     gemm_kernel, so every result has the same bits as there and in the
 //     reference.
 // Every MAC's rotation or shift-add product is still computed, per MAC.
@@ -29,15 +31,20 @@
 
 namespace rac {
 
-// Where the per-MAC terms are computed.  With 256 outputs
+// Where the per-MAC terms are computed.  FAST has none.  With 256 outputs
 // per workgroup (one per lane) each lane computes its own MACs' terms and
 // folds them at once ("own"); with fewer, every lane computes terms for the
 // tile into LDS and the lanes owning outputs fold them ("shared").  k per
-// tile keeps the workgroup's LDS under 64 KB.
-template <int OUTS>
+// tile keeps the workgroup's LDS under 64 KB.  (512-k FAST tiles on grids
+// of one workgroup per CU were faster with the looped fold, 42 -> 31 us at
+// 1x4096x4096; with the read-ahead fold the 256-k tile is: 32.2 -> 29.9 us,
+// 4096x1x4096 31.8 -> 29.3 us, bit-identical.)
+template <int MODE, int OUTS>
 struct SkCfg {
-    static constexpr bool kShared = OUTS < 256;
-    static constexpr int kKT = !kShared ? 128 : (OUTS == 16 ? 256 : (OUTS <= 64 ? 128 : 64));
+    static constexpr bool kShared = MODE != kModeFast && OUTS < 256;
+    static constexpr bool kOwn = MODE != kModeFast && OUTS == 256;
+    static constexpr int kKT = MODE == kModeFast ? 256
+                               : kOwn ? 128 : (OUTS == 16 ? 256 : (OUTS <= 64 ? 128 : 64));
     static constexpr int kRow = kKT + 4;        // LDS row stride (16 rows cover all banks)
 };
 
@@ -70,8 +77,9 @@ __device__ __forceinline__ void sk_cordic_terms(const float* a, const float* b, 
 // Global -> registers: element (m0 + m, k) of A (row-major M x K) and
 // (k, n0 + n) of op(B) for the K-tile at k0, zero outside the matrices,
 // spread over lanes L0 .. L0 + NL - 1 (the others return: with L0 = 64 the
-// folding wave 0 issues no loads).
-template <int RB, int CB, int KT, bool TB, int L0 = 0, int NL = 256>
+// folding wave 0 issues no loads).  NEG (FAST): -0 in A past the matrix: the
+// product -0 leaves every accumulator as it is.
+template <int RB, int CB, int KT, bool TB, int L0 = 0, int NL = 256, bool NEG = false>
 __device__ __forceinline__ void sk_load(const float* __restrict__ A, const float* __restrict__ B, int M, int N,
                                         int K, long m0, long n0, int k0, float* ra, float* rb) {
     if ((int)threadIdx.x < L0) return;
@@ -80,7 +88,7 @@ __device__ __forceinline__ void sk_load(const float* __restrict__ A, const float
     for (int r = 0; r < (RB * KT + NL - 1) / NL; r++) {
         const int idx = tid + r * NL, kk = idx % KT;
         const long gm = m0 + idx / KT, gk = (long)k0 + kk;
-        ra[r] = (idx < RB * KT && gm < M && gk < K) ? A[gm * K + gk] : 0.0f;
+        ra[r] = (idx < RB * KT && gm < M && gk < K) ? A[gm * K + gk] : (NEG ? -0.0f : 0.0f);
     }
 #pragma unroll
     for (int r = 0; r < (CB * KT + NL - 1) / NL; r++) {
@@ -146,7 +154,7 @@ __device__ __forceinline__ void sk_terms(const float* sA, const float* sB, float
 
 // The serial fold of output (om, on) over kn k of a tile, in order: the
 // terms from sP row `prow` (SHARED), or computed here from sA row om (own
-// terms).  Zero k-padding leaves acc as is.
+// terms; FAST: the A element itself).  Zero k-padding leaves acc as is.
 template <int MODE, int NITER, int ROW, bool SHARED, bool RING>
 __device__ __forceinline__ float sk_fold(const float* sA, const float* sB, const float* sP, int om, int on,
                                          int prow, int kn, float acc, int iters, float kinv, bool lit) {
@@ -167,20 +175,23 @@ __device__ __forceinline__ float sk_fold(const float* sA, const float* sB, const
         }
         return acc;
     }
-    if constexpr (RING && SHARED) {
-        // Terms come from LDS, so the chain is fed by reads alone.  A full tile's fold is unrolled completely and its
+    if constexpr (RING && (SHARED || MODE == kModeFast)) {
+        // Terms (or FAST's A elements) come from LDS, so the chain is fed by
+        // reads alone.  A full tile's fold is unrolled completely and its
         // reads run D 4-k steps ahead of the FMAs through a ring of D
         // register pairs: step j folds pair j and reads pair j + D, and a
         // scheduling barrier after each step keeps that order (left to
         // itself the scheduler read one step ahead and waited on LDS every
         // 8 k; a dependent fmaf costs ~4.6 cycles on one wave).  2 D reads
         // in flight stay within the 15 the LDS counter tracks.  RING is set
-        // where it measured faster: the CORDIC pipeline on 512 lanes or with
-        // 64-output blocks (its VGPRs cost a wave per SIMD on wide grids).
+        // where it measured faster (sk_block): FAST blocks of at most 64
+        // outputs, and larger ones on grids of at most two workgroups per CU
+        // (the ring's VGPRs cost a wave per SIMD on wider ones), and the
+        // CORDIC pipeline on 512 lanes or with 64-output blocks.
         constexpr int KT = ROW - 4, D = 6;
         if (kn == KT) {
             const float* rowb = &sB[on * ROW];
-            const float* rowt = &sP[prow * ROW];
+            const float* rowt = SHARED ? &sP[prow * ROW] : &sA[om * ROW];
             float4 rb[D], rt[D];
 #pragma unroll
             for (int j = 0; j < D; j++) {
@@ -198,7 +209,8 @@ __device__ __forceinline__ float sk_fold(const float* sA, const float* sB, const
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     if constexpr (MODE == kModeCordic) acc = __builtin_fmaf(t[e], __builtin_fabsf(b[e]), acc);
-                    else acc = acc + t[e];
+                    else if constexpr (MODE == kModeShiftAdd) acc = acc + t[e];
+                    else acc = __builtin_fmaf(t[e], b[e], acc);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -220,15 +232,19 @@ __device__ __forceinline__ float sk_fold(const float* sA, const float* sB, const
             const float a[4] = {a4.x, a4.y, a4.z, a4.w};
             if constexpr (MODE == kModeCordic) {
                 sk_cordic_terms<NITER>(a, b, t4, iters, kinv, lit);
-            } else {
+            } else if constexpr (MODE == kModeShiftAdd) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) t4[e] = shiftadd_mul(a[e], b[e], iters);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) t4[e] = a[e];
             }
         }
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             if constexpr (MODE == kModeCordic) acc = __builtin_fmaf(t4[e], __builtin_fabsf(b[e]), acc);
-            else acc = acc + t4[e];
+            else if constexpr (MODE == kModeShiftAdd) acc = acc + t4[e];
+            else acc = __builtin_fmaf(t4[e], b[e], acc);
         }
     }
     return acc;
@@ -268,13 +284,13 @@ struct SkBlock {
     }
 };
 
-template <int MODE, int NITER, bool TB, bool FUSED, int RB, int CB, bool FEWCOL>
+template <int MODE, int NITER, bool TB, bool FUSED, int RB, int CB, bool FEWCOL, bool RING>
 __global__ __launch_bounds__(256) void gemm_skinny_kernel(
     const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N, int K,
     float alpha, float beta, int iters, float kinv, long sa, long sb, long sc, GemmEpilogue ep,
     const int* k_causal, int exact_specials, int row0)
 {
-    using Cfg = SkCfg<RB * CB>;
+    using Cfg = SkCfg<MODE, RB * CB>;
     constexpr int KT = Cfg::kKT, ROW = Cfg::kRow;
     constexpr bool kShared = Cfg::kShared;
     __shared__ __attribute__((aligned(16))) float sA[RB * ROW];
@@ -294,14 +310,23 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(
 
     const int om = tid / CB, on = tid % CB;           // output owned by lanes tid < RB * CB
     const bool owner = tid < RB * CB && om < blk.mv && on < blk.nv;
-    float ra[(RB * KT + 255) / 256], rb[(CB * KT + 255) / 256];
+    // FAST with one row (or column) of 16 outputs: wave 0 only folds, and
+    // waves 1-3 load and stage the tiles, so the next tile's loads are
+    // issued while wave 0 folds this one (per tile at 1x4096x4096 wave 0
+    // spent ~950 of 4300 cycles issuing its share of the loads before its
+    // fold).  Measured, bit-identical: 1x4096x4096 29.9 -> 29.3 us,
+    // 1x4096x11008 72.5 -> 66.6, 4096x1x4096 29.4 -> 28.4; with 4 rows it
+    // lost (30.3 -> 31.8 us), and the CORDIC pipeline, whose waves 1-3
+    // compute the terms, lost too (1x4096x4096 54.3 -> 63.7 us).
+    constexpr int L0 = (MODE == kModeFast && RB * CB <= 16) ? 64 : 0, NL = 256 - L0;
+    float ra[(RB * KT + NL - 1) / NL], rb[(CB * KT + NL - 1) / NL];
     float acc = 0.0f;
-    sk_load<RB, CB, KT, TB>(A, B, M, N, K, blk.m0, blk.n0, 0, ra, rb);
+    sk_load<RB, CB, KT, TB, L0, NL, MODE == kModeFast>(A, B, M, N, K, blk.m0, blk.n0, 0, ra, rb);
     for (int k0 = 0, t = 0; k0 < blk.kend; k0 += KT, t++) {
         __syncthreads();                                // previous tile's fold done with LDS
-        if (sk_store<MODE, RB, CB, KT, ROW, TB>(sA, sB, ra, rb) && exact_specials) lit[t & 1] = 1;
+        if (sk_store<MODE, RB, CB, KT, ROW, TB, L0, NL>(sA, sB, ra, rb) && exact_specials) lit[t & 1] = 1;
         __syncthreads();
-        if (k0 + KT < blk.kend) sk_load<RB, CB, KT, TB>(A, B, M, N, K, blk.m0, blk.n0, k0 + KT, ra, rb);
+        if (k0 + KT < blk.kend) sk_load<RB, CB, KT, TB, L0, NL, MODE == kModeFast>(A, B, M, N, K, blk.m0, blk.n0, k0 + KT, ra, rb);
         const bool lit_tile = MODE == kModeCordic && lit[t & 1] != 0;
         if constexpr (kShared) {
             sk_terms<MODE, NITER, RB, CB, KT, ROW>(sA, sB, sP, blk.mv, blk.nv, iters, kinv, lit_tile);
@@ -309,7 +334,7 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(
         }
         if (tid == 0) lit[(t + 1) & 1] = 0;            // tile t+1's flag: set after the loop-top barrier
         if (owner)
-            acc = sk_fold<MODE, NITER, ROW, kShared, false>(sA, sB, sP, om, on, tid, min(KT, blk.kend - k0), acc, iters,
+            acc = sk_fold<MODE, NITER, ROW, kShared, RING>(sA, sB, sP, om, on, tid, min(KT, blk.kend - k0), acc, iters,
                                                      kinv, lit_tile);
     }
     if (owner) sk_epilogue<FUSED>(C, N, blk.m0 + om, blk.n0 + on, acc, alpha, beta, ep, iters);
@@ -392,7 +417,7 @@ __global__ __launch_bounds__(NT) void gemm_skinny_pipe_kernel(
 }
 
 template <int MODE, int NITER, bool TB, bool FUSED, int RB, int CB, bool FEWCOL, bool PIPE,
-          int NT = 256>
+          bool RING = (MODE == kModeFast && RB * CB <= 64), int NT = 256>
 static hipError_t sk_launch(const SkinnyArgs& g, hipStream_t s) {
     const unsigned wgs = FEWCOL ? (unsigned)((g.M + RB - 1) / RB) : (unsigned)((g.N + CB - 1) / CB);
     const dim3 grid(wgs, 1, (unsigned)g.batch);
@@ -401,7 +426,7 @@ static hipError_t sk_launch(const SkinnyArgs& g, hipStream_t s) {
                            g.A, g.B, g.C, g.M, g.N, g.K, g.alpha, g.beta, g.iters, cordic_kinv(g.iters), g.sa, g.sb,
                            g.sc, g.ep, g.k_causal, g.exact_specials, g.row0);
     } else {
-        hipLaunchKernelGGL((gemm_skinny_kernel<MODE, NITER, TB, FUSED, RB, CB, FEWCOL>), grid, dim3(256), 0, s,
+        hipLaunchKernelGGL((gemm_skinny_kernel<MODE, NITER, TB, FUSED, RB, CB, FEWCOL, RING>), grid, dim3(256), 0, s,
                            g.A, g.B, g.C, g.M, g.N, g.K, g.alpha, g.beta, g.iters, cordic_kinv(g.iters), g.sa, g.sb,
                            g.sc, g.ep, g.k_causal, g.exact_specials, g.row0);
     }
@@ -409,16 +434,30 @@ static hipError_t sk_launch(const SkinnyArgs& g, hipStream_t s) {
 }
 
 // One output block shape (RB x CB): CORDIC takes the pipelined terms (<= 64
-// outputs); SHIFTADD's terms (a shift-add product each) outweigh its fold
-// and keep all four waves (pipelined on three: 1x4096x4096 213 -> 297 us).
+// outputs); SHIFTADD's
+// terms (a shift-add product each) outweigh its fold and keep all four
+// waves (pipelined on three: 1x4096x4096 213 -> 297 us).  The read-ahead
+// fold (RING), measured against the looped one, bit-identical: FAST
+// 1x11008x4096 50.7 -> 43.8 us, 8x4096x4096 34.0 -> 32.0, 16x4096x4096
+// 38.6 -> 36.4, 2048x10x4096 55.2 -> 43.2; CORDIC n = 16 4x4096x4096 175.7
+// -> 158.3.  With 2.7 workgroups per CU its VGPRs cost a wave per SIMD
+// (FAST 16x11008x4096 77.7 -> 83.2 us), and one-row CORDIC and SHIFTADD
+// gained nothing (CORDIC 1x4096x4096 54.3 -> 55.1, SHIFTADD 1x11008x4096
+// 271.7 -> 279.7 us), so they keep the loop.
 template <int MODE, int NITER, bool TB, bool FUSED, int RB, int CB, bool FEWCOL>
 static hipError_t sk_block(const SkinnyArgs& g, hipStream_t s) {
     const long wgs = (FEWCOL ? (long)((g.M + RB - 1) / RB) : (long)((g.N + CB - 1) / CB)) * g.batch;
-    if constexpr (MODE == kModeCordic && RB * CB <= 128) {
-        if (wgs <= device_cus()) return sk_launch<MODE, NITER, TB, FUSED, RB, CB, FEWCOL, true, 512>(g, s);
+    if constexpr (MODE == kModeCordic && RB * CB == 128) {
+        if (wgs <= device_cus()) return sk_launch<MODE, NITER, TB, FUSED, RB, CB, FEWCOL, true, false, 512>(g, s);
     }
-    if constexpr (MODE == kModeCordic && RB * CB <= 64)
-        return sk_launch<MODE, NITER, TB, FUSED, RB, CB, FEWCOL, true>(g, s);
+    if constexpr (RB * CB <= 64) {
+        if constexpr (MODE == kModeCordic) {
+            if (wgs <= device_cus()) return sk_launch<MODE, NITER, TB, FUSED, RB, CB, FEWCOL, true, false, 512>(g, s);
+            return sk_launch<MODE, NITER, TB, FUSED, RB, CB, FEWCOL, true>(g, s);
+        }
+    } else if constexpr (MODE == kModeFast) {
+        if (wgs <= 2 * device_cus()) return sk_launch<MODE, NITER, TB, FUSED, RB, CB, FEWCOL, false, true>(g, s);
+    }
     return sk_launch<MODE, NITER, TB, FUSED, RB, CB, FEWCOL, false>(g, s);
 }
 
@@ -428,17 +467,25 @@ static hipError_t sk_block(const SkinnyArgs& g, hipStream_t s) {
 // half as wide blocks double the workgroups (two waves per SIMD instead of
 // one): measured, bit-identical, 8x4096x4096 CORDIC n = 16 218 -> 177 us,
 // 16x4096x4096 330 -> 225 us, SHIFTADD 1.54 -> 0.85 ms and 2.97 -> 1.69
-// ms; on wider grids (N = 11008) the narrow blocks lost 6-29% (CORDIC).
+// ms, FAST 16 rows 52 -> 37 us; on wider grids (N = 11008) the narrow
+// blocks lost 6-29% (CORDIC, FAST), and FAST lost with 8 rows everywhere.
 // SHIFTADD, bound by its terms, takes them at 9-16 rows on any grid.  CORDIC
 // with 5-8 rows (or columns) now keeps 8 x 16 blocks on such grids, which
 // the 512-lane pipeline runs (8 x 8 blocks on 256 lanes: 175.8 us, 8 x 16
-// on 512: 160.4 us at 8x4096x4096 n = 16).
+// on 512: 160.4 us at 8x4096x4096 n = 16).  One
+// FAST row (or column) takes 8-wide blocks on such grids too: its fold is
+// one wave per workgroup, so twice the workgroups fold on twice the SIMDs
+// (1x4096x4096 29.1 -> 26.4 us, 1x4096x11008 66.7 -> 62.2; on the wider
+// 1x11008x4096 grid 43.9 -> 51.9, so that keeps 16).
 template <int MODE, int NITER, bool TB, bool FUSED>
 static hipError_t sk_shape(const SkinnyArgs& g, hipStream_t s) {
     const long cus = device_cus();
     if (g.M <= kSkinnyMaxRows) {                         // few rows, the grid over N
         const bool one_per_cu = (long)((g.N + 15) / 16) * g.batch <= cus;
-        if (g.M == 1) return sk_block<MODE, NITER, TB, FUSED, 1, 16, false>(g, s);
+        if (g.M == 1) {
+            if (MODE == kModeFast && one_per_cu) return sk_block<MODE, NITER, TB, FUSED, 1, 8, false>(g, s);
+            return sk_block<MODE, NITER, TB, FUSED, 1, 16, false>(g, s);
+        }
         if (g.M <= 4) return sk_block<MODE, NITER, TB, FUSED, 4, 16, false>(g, s);
         if (g.M <= 8) {
             // CORDIC keeps 8 x 16 blocks there: the 512-lane pipeline takes them
@@ -450,10 +497,13 @@ static hipError_t sk_shape(const SkinnyArgs& g, hipStream_t s) {
     }
     // few columns, the grid over M
     const bool one_per_cu = (long)((g.M + 15) / 16) * g.batch <= cus;
-    if (g.N == 1) return sk_block<MODE, NITER, TB, FUSED, 16, 1, true>(g, s);
+    if (g.N == 1) {
+        if (MODE == kModeFast && one_per_cu) return sk_block<MODE, NITER, TB, FUSED, 8, 1, true>(g, s);
+        return sk_block<MODE, NITER, TB, FUSED, 16, 1, true>(g, s);
+    }
     if (g.N <= 4) return sk_block<MODE, NITER, TB, FUSED, 16, 4, true>(g, s);
     if (g.N <= 8) {
-        if (one_per_cu) return sk_block<MODE, NITER, TB, FUSED, 8, 8, true>(g, s);
+        if (MODE != kModeFast && one_per_cu) return sk_block<MODE, NITER, TB, FUSED, 8, 8, true>(g, s);
         return sk_block<MODE, NITER, TB, FUSED, 16, 8, true>(g, s);
     }
     if (MODE == kModeShiftAdd || one_per_cu) return sk_block<MODE, NITER, TB, FUSED, 8, 16, true>(g, s);
@@ -468,6 +518,7 @@ static hipError_t sk_layout(const SkinnyArgs& g, hipStream_t s) {
 }
 
 hipError_t gemm_skinny_launch(const SkinnyArgs& g, int mode, hipStream_t s) {
+    if (mode == kModeFast) return sk_layout<kModeFast, 0>(g, s);
     if (mode == kModeShiftAdd) return sk_layout<kModeShiftAdd, 0>(g, s);
     switch (g.iters) {
         case 8: return sk_layout<kModeCordic, 8>(g, s);

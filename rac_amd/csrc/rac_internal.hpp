@@ -58,9 +58,10 @@ hipError_t act_grad_launch(const float* g, const float* pre, float* d, long coun
 // keeps the strength-reduced chain for every input (callers whose parity
 // bar is a summation bound, where subnormal-rounding differences of tiny
 // products are far below it).
-// The CORDIC and SHIFTADD products for M <= 16 rows or N <= 16 columns, A
-// row-major (not transposed): gemm_launch hands such launches (schedules 0
-// and 2) to the few-row / few-column kernels.
+// The same product for M <= 16 rows or N <= 16 columns, A row-major (not
+// transposed): gemm_launch hands such launches to the few-row / few-column
+// kernels, CORDIC and SHIFTADD those of schedules 0 and 2, FAST some of
+// schedule 0 (fast_few_rows).
 struct SkinnyArgs {
     const float* A;
     const float* B;

@@ -52,6 +52,9 @@ SHAPES = [(17, 17, 4), (17, 33, 3), (20, 18, 1), (801, 3913, 1), (2050, 2041, 3)
 # the 16-k tiles of many outputs, short K-tiles of a transposed A's few rows
 SHAPES += [(300, 301, 15), (300, 299, 16), (299, 300, 17), (679, 1739, 32), (679, 1739, 33), (1167, 3867, 16),
            (1167, 3868, 47), (2049, 1030, 64), (12, 300, 32), (13, 301, 33), (301, 7, 17), (4, 62, 48)]
+# few rows or columns of short K (the few-row kernels) and one past it
+SHAPES += [(1, 62, 200), (1, 2050, 511), (1, 2050, 1027), (3, 6874, 255), (3, 6874, 257), (4, 62, 512), (9, 301, 513),
+           (550, 12, 210), (2036, 2, 511), (16, 16, 256), (7, 16, 40), (1, 513, 4090)]
 
 
 @pytest.mark.parametrize("layout", [(0, 0), (0, 1), (1, 0), (1, 1)])
@@ -96,7 +99,7 @@ def test_fast_tile_specials(layout):
 
 UNDERFLOW = [(17, 17, 4), (20, 18, 1), (31, 32, 63), (33, 65, 80), (63, 129, 15), (129, 8200, 37), (300, 5633, 31),
              (500, 2049, 70), (1000, 777, 131), (2049, 4095, 33), (1, 31, 130), (3, 2100, 129), (16, 33, 127),
-             (2100, 3, 129), (2, 2, 2), (2, 3, 70)]
+             (2100, 3, 129), (2, 2, 2), (2, 3, 70), (1, 62, 35), (4, 62, 270), (16, 300, 33)]
 
 
 @pytest.mark.parametrize("layout", [(0, 0), (0, 1), (1, 0), (1, 1)])
