@@ -1078,7 +1078,7 @@ RAC_EXPORT int rac_attention_backward_dev(const float* q, const float* k, const 
     // the sizes the FAST tiles take with a causal limit (K and side-by-side
     // rows of at least 4), and head_dim within the bound check's 4096 terms
     int* flag = nullptr;
-    if (causal_unmasked && mode == kModeFast && t >= 4 && c >= 4 && d >= 4 && d <= 4096) {
+    if (causal_unmasked && mode == kModeFast && t >= kFastMinK && c >= kFastMinK && d >= kFastMinK && d <= 4096) {
         flag = reinterpret_cast<int*>(reinterpret_cast<char*>(workspace) + attention_scores_bytes(bh, t, c));
         rc = check_hip(all_bounded_launch(q, k, v, grad_out, bh * td, flag, s), "rac_attention_backward bound check");
         if (rc) return rc;

@@ -374,7 +374,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const T* __rest
             if (n0 > g.row0 + last) return;
         }
         else if (g.k_side == 2) {
-            kbeg = (int)min((long)g.K - 4, max(0L, m0 - g.row0));
+            kbeg = (int)min((long)g.K - kFastMinK, max(0L, m0 - g.row0));
             any_k = m0 - g.row0 < g.K;
         }
     }
@@ -542,6 +542,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_fast_kernel(const T* __rest
 template <bool TA, bool TB, bool FUSED, bool TRAP, int BM, int BN, int WR, int WC, int KT, int PD, int SPREAD, bool THIN = false,
           class T = float>
 static hipError_t fast_launch(const GemmArgs& a, hipStream_t s) {
+    static_assert(BM <= kFastMaxTile && BN <= kFastMaxTile, "causal operands are defined to kCausalMargin only");
     FastGeom g{a.M, a.N, a.K, a.sa, a.sb, a.sc, a.alpha, a.beta, a.iters, a.ep, a.k_causal, a.k_causal || a.k_side == 3 ? a.k_side : 0,
                a.row0, a.period, 0, (a.M + BM - 1) / BM, a.batch, 0};
     if constexpr (TRAP) {

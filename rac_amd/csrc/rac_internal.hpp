@@ -94,10 +94,16 @@ hipError_t all_finite_launch(const float* x, long n, int* flag, hipStream_t s);
 // else 0.
 hipError_t all_bounded_launch(const float* a, const float* b, const float* c, const float* d, long n, int* flag,
                               hipStream_t s);
+// The FAST tiles' largest side and the fewest k a launch of theirs takes.
+constexpr int kFastMaxTile = 128, kFastMinK = 4;
+// How far past its diagonal a row of a causal operand is read under the FAST
+// products' limits on k: the tile that holds the diagonal reaches kFastMaxTile
+// - 1 further, and a last few k may begin up to kFastMinK rows early.
+constexpr int kCausalMargin = kFastMaxTile - 1 + kFastMinK;
 // dS = P (dP - rowsum(dP P)) in place of dP, rows x seq each (query position
 // row0 + row % c); flag (may be null): when it holds 1, P is causal, only the
-// columns up to the query position are read, and the next 131 are written as
-// zeros.
+// columns up to the query position are read, and the next kCausalMargin are
+// written as zeros.
 hipError_t attn_dscore_launch(const float* P, float* dP, long rows, long seq, long c, long row0, const int* flag,
                               hipStream_t s);
 

@@ -741,8 +741,8 @@ hipError_t layernorm_launch(const float* x, float* y, const float* gamma, const 
 // W waves per row (1: rows of up to 512, four to a workgroup).  Bound by
 // memory: [32, 2048, 2048] in 155 us causal (804 MB: half of each matrix).
 // With *flag == 1 (causal P, nothing past the diagonal but zeros) row t reads
-// columns 0 .. t and also writes zeros to t + 131, as far as the products'
-// 128-wide tiles and their last 4 k look past the diagonal.
+// columns 0 .. t and also writes zeros to t + kCausalMargin, as far as the
+// products look past the diagonal.
 template <int W, int VPT>
 __global__ __launch_bounds__(256) void attn_dscore_kernel(const float* __restrict__ P, float* dP, long rows, long n,
                                                           long c, long row0, const int* flag) {
@@ -753,7 +753,7 @@ __global__ __launch_bounds__(256) void attn_dscore_kernel(const float* __restric
     if (W == 1 && row >= rows) return;
     const bool causal = flag && *flag == 1;
     const long t = row0 + row % c;
-    const long have = causal ? min(n, t + 1) : n, want = causal ? min(n, t + 132) : n;
+    const long have = causal ? min(n, t + 1) : n, want = causal ? min(n, t + 1 + kCausalMargin) : n;
     const float* p = P + row * n;
     float* d = dP + row * n;
     // 16-byte accesses at any 4-byte boundary
