@@ -1,7 +1,8 @@
 """GPU parity of the attention core's native backward (ext.attention_backward)
 against the same gradients composed from the RAC products and torch, whole
 and in chunks of query rows, causal (which skips the half past the diagonal)
-and not, at sizes around the products' 32 / 64 / 128 tiles.
+and not, at sizes around the products' tiles: 32x32 and the few-column ones in
+the first test, the larger ones in test_attention_backward_large_tiles.
 
 The products have the composition's bits for equal dS; dS itself sums each
 row in another order.  A row sum of T terms dP P with sum |dP P| <= max |dP|
@@ -72,6 +73,16 @@ def test_attention_backward(shape, rows, causal, mode):
         assert float((dv - want[2]).abs().max()) <= T * 2.0 ** -24 * float(g.abs().max()) * T ** 0.5
     assert float((dq - want[0]).abs().max()) <= 2 * eps * float(k.abs().max())
     assert float((dk - want[1]).abs().max()) <= 2 * eps * float(q.abs().max()) * T ** 0.5
+
+
+# 256 CUs give the causal products 64x64 tiles (the first three shapes and the
+# last two; 32x64 the fourth and fifth), and dP 64x64, 32x64, 64x128, 32x64,
+# 32x32, 128x128 and 32x32 ones; the chunks' first rows are on no tile's edge
+@pytest.mark.parametrize("shape,rows", [((1, 16, 1030, 100), 1030), ((1, 16, 1030, 100), 333), ((1, 32, 1000, 64), 1000),
+                                        ((1, 8, 1030, 128), 1030), ((1, 8, 1030, 128), 500),
+                                        ((1, 4, 2000, 600), 2000), ((1, 8, 1030, 516), 500)])
+def test_attention_backward_large_tiles(shape, rows):
+    test_attention_backward(shape, rows, True, "fast")
 
 
 @pytest.mark.parametrize("value", [float("inf"), float("nan"), 2.0 ** 100])
