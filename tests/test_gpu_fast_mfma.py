@@ -1,15 +1,15 @@
 """GPU parity of the FAST-mode GEMM on the matrix cores.
 
-FAST launches with at least a quarter as many 128x128 blocks as CUs, at
-least half of their outputs real, and K >= 128 run on
-v_mfma_f32_32x32x1_2b_f32, one instruction per k in k order; each
-output must equal the reference's fmaf chain (rac_kernels.hip:204-219, mode
-FAST) bit for bit, like the VALU tiles do.  Shapes below are chosen to take
-that path: ragged on every edge, K not a multiple of 4 (element loads), all
-dimensions multiples of 4 (16-byte loads), exact tiles, a base address off
-the 16-byte grid, batched launches with alpha / beta, the fused bias +
-activation epilogue, special operands (subnormal, infinite, NaN), launches
-of fewer blocks than CUs, and the config-5 attention core's P V chunks.
+FAST products of more than 16 rows and columns and more than 16 k (fewer only
+past 2^21 outputs) run on v_mfma_f32_16x16x4_f32, in output tiles of 32x32 to
+128x128 chosen by a cost rule; each output must equal the reference's fmaf
+chain (rac_kernels.hip:204-219, mode FAST) bit for bit, whatever the tile.
+Shapes below are ragged on every edge, with K no multiple of 4 and odd leading
+dimensions, all dimensions multiples of 4, exact tiles, a base address off the
+16-byte grid, batched launches with alpha / beta, the fused bias + activation
+epilogue, special operands (subnormal, infinite, NaN), launches of one tile to
+a CU, and the attention core's P V chunks.  The tiles named are those of 256
+CUs.
 """
 import numpy as np
 import pytest
@@ -73,12 +73,13 @@ def operands(M, N, K, ta, tb, seed):
     return As, Bs
 
 
-# (2100, 2100, 129): ragged tiles, K % 4 != 0 and N % 4 != 0 (element
-# loads); (2052, 2100, 260): every dimension a multiple of 4 (16-byte loads),
-# ragged tiles; (2048, 2176, 512): exact tiles.  These take wave tiles of
-# 64 x 64 (128 x 128 blocks); the 4000 x 4000 shapes fill one round of
-# 256 x 128 blocks and take 128 x 64 wave tiles (ragged on both edges).
-MF_SHAPES = [(2100, 2100, 129), (2052, 2100, 260), (2048, 2176, 512), (4000, 4000, 129), (4000, 4000, 260)]
+# (2100, 2100, 129): 32x64 tiles, K no multiple of 4; (2052, 2100, 260): 32x32,
+# every dimension a multiple of 4; (2048, 2176, 512): 32x32, exact; the 4000 x
+# 4000 shapes and (4003, 3999, 77), rows and columns past a multiple of 4:
+# 64x128 (64x64 in the TN layout, which has no 64x128); (2483, 2881, 517):
+# 128x128.
+MF_SHAPES = [(2100, 2100, 129), (2052, 2100, 260), (2048, 2176, 512), (4000, 4000, 129), (4000, 4000, 260),
+             (4003, 3999, 77), (2483, 2881, 517)]
 
 
 @pytest.mark.parametrize("layout", [(0, 0), (0, 1), (1, 0), (1, 1)])
@@ -96,7 +97,8 @@ def test_fast_mfma_bit_exact(shape, layout):
 @pytest.mark.parametrize("shape", [(2052, 2100, 260), (4000, 4000, 260)])
 @pytest.mark.parametrize("layout", [(0, 0), (0, 1), (1, 0)])
 def test_fast_mfma_unaligned_base(layout, shape):
-    """Dimensions that allow 16-byte loads, base addresses that do not."""
+    """Dimensions whose rows all start on the 16-byte grid, base addresses that
+    do not."""
     M, N, K = shape
     ta, tb = layout
     print(f"fast mfma unaligned layout={layout}", flush=True)
@@ -147,7 +149,7 @@ def test_fast_mfma_alpha_beta():
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
 def test_fast_mfma_batched(ta, tb):
-    """4 batch items of 1100 x 1100 (324 tiles): bmm with alpha, then
+    """4 batch items of 1100 x 1100 (32x64 tiles): bmm with alpha, then
     accumulating into the result with beta."""
     e = ext()
     Z, M, N, K = 4, 1100, 1100, 200
@@ -168,7 +170,7 @@ def test_fast_mfma_batched(ta, tb):
 @pytest.mark.parametrize("act", [0, 1, 3])
 def test_fast_mfma_fused_linear(act):
     """linear_forward and fused_linear_forward (bias + activation in the
-    epilogue) at an MFMA shape: pre-activations equal the unfused product
+    epilogue) on 32x32 tiles: pre-activations equal the unfused product
     plus bias, bit-exact vs the checker; outputs equal the activation kernel
     applied to them."""
     e = ext()
@@ -192,10 +194,9 @@ def test_fast_mfma_fused_linear(act):
 @pytest.mark.parametrize("causal", [True, False])
 def test_fast_attention_config5_mfma_products(causal):
     """The config-5 attention core in FAST mode: each 512-row chunk's P V
-    (32 heads of 512 x 128, 128 blocks, the causal K limit per row tile)
-    runs on the matrix cores; the output equals the one-chunk form (P V on
-    the VALU tiles) and the checker's composition on sampled heads, bit for
-    bit."""
+    (32 heads of 512 x 128, the causal K limit per row tile) equals the
+    one-chunk form's (32 heads of 2048 x 128) and the checker's composition
+    on sampled heads, bit for bit."""
     e = ext()
     shape = (1, 32, 2048, 128)
     q = rl.gen_normal(shape, seed=700)
@@ -211,8 +212,7 @@ def test_fast_attention_config5_mfma_products(causal):
 
 @pytest.mark.parametrize("Z,M,N,K", [(32, 512, 128, 600), (1, 1024, 1024, 1030), (8, 512, 512, 512)])
 def test_fast_mfma_few_blocks(Z, M, N, K):
-    """Launches of 64-128 blocks of 128 x 128 (fewer than the CUs) on the
-    matrix cores: bit-exact vs the checker."""
+    """Launches of one 64x64 tile to a CU: bit-exact vs the checker."""
     e = ext()
     A = rl.gen_uniform((Z, M, K), seed=Z + M)
     B = rl.gen_uniform((Z, K, N), seed=N + K)
@@ -242,9 +242,9 @@ def _attention_ws(q, k, v, mask, causal, chunk_rows):
 
 def test_fast_attention_chunks_mfma():
     """[1, 16, 512, 128] in FAST mode: the causal scores of each chunk of
-    query rows (the trapezoid of 128 x 128 tiles on or below the diagonal)
-    and P V run on the matrix cores for chunks of 64 rows and more; every
-    chunk size gives the one-chunk bits, which equal the checker's."""
+    query rows (the trapezoid of tiles on or below the diagonal) and P V run
+    on the matrix cores, and every chunk size gives the one-chunk bits, which
+    equal the checker's."""
     e = ext()
     shape = (1, 16, 512, 128)
     q = rl.gen_normal(shape, seed=720)
@@ -266,11 +266,11 @@ def test_fast_attention_chunks_mfma():
 
 @pytest.mark.parametrize("act", [0, 3])
 def test_fast_mfma_linear_backward(act):
-    """The FAST training products at MFMA sizes: fused_linear_backward's
+    """The FAST training products on 32x32 and 32x64 tiles: fused_linear_backward's
     grad_input (d W, NN) and grad_weight (d^T x, TN) bit-exact vs the
     checker, d = the activation gradient of the saved pre-activations."""
     e = ext()
-    M, N, K = 1024, 2304, 1030         # 144 / 72 / 162 blocks of 128 x 128
+    M, N, K = 1024, 2304, 1030
     x = rl.gen_normal((M, K), seed=31)
     w = rl.gen_normal((N, K), seed=32, std=0.05)
     b = rl.gen_normal(N, seed=33)
