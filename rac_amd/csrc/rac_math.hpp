@@ -383,6 +383,33 @@ __device__ __forceinline__ float exp_cordic_rt(float x, int n, float khinv) {
     return (x != x) ? x : res;
 }
 
+// G of them a step at a time: G independent chains in flight, not one after
+// the other.
+template <int G>
+__device__ __forceinline__ void exp_cordic_rt_vec(float* v, int n, float khinv) {
+    int k[G];
+    float p[G], z[G];
+#pragma unroll
+    for (int e = 0; e < G; e++) {
+        exp_reduce(v[e], k[e], z[e]);
+        p[e] = 1.0f;
+    }
+    for (int j = 0; j < n; j++) {
+        const float S = g_steps.hS[j], C = g_steps.hC[j];
+#pragma unroll
+        for (int e = 0; e < G; e++) {
+            const float ds = __builtin_copysignf(S, z[e]);
+            p[e] = __builtin_fmaf(ds, p[e], p[e]);
+            z[e] = __builtin_fmaf(-ds, C, z[e]);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < G; e++) {
+        const float res = exp_scale(p[e] * khinv, k[e]);
+        v[e] = (v[e] != v[e]) ? v[e] : res;
+    }
+}
+
 // ── rsqrt by hyperbolic vectoring ────────────────────────────────────────
 
 // Vectoring step J (d = -sign(Y)), constants forced to compile time.

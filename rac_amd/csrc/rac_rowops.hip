@@ -47,10 +47,13 @@ __device__ __forceinline__ float inv_sum(float s, int zero_guard) {
     return (zero_guard && !(s > 0.0f)) ? 0.0f : 1.0f / s;
 }
 
-// Exps of the E = 4*VPT row elements a lane holds.  Compile-time step
-// counts use the step-major form (all elements advance one step at a time:
-// independent chains interleave and constants are shared); bit-identical
-// to one exp_cordic call per element.
+// Exps of the E = 4*VPT row elements a lane holds, in the step-major form
+// (the elements of a group advance one step at a time: independent chains
+// interleave and constants are shared); bit-identical to one exp_cordic call
+// per element.  Step counts known only at run time too: one element after the
+// other, a wave's long lane of them was slower than four waves' short ones
+// (1024 x 600, 12 steps: 6.9 us before rows to a wave, 9.4 with them, now
+// 6.9; 4096 x 500 10.1 -> 6.4).
 template <int NITER, int E, int OPT = kExpFull>
 __device__ __forceinline__ void exp_lane(float* v, int iters, float khinv) {
     if constexpr (NITER > 0) {
@@ -58,8 +61,9 @@ __device__ __forceinline__ void exp_lane(float* v, int iters, float khinv) {
 #pragma unroll
         for (int b = 0; b < E; b += G) exp_cordic_vec<NITER, G, OPT>(v + b, khinv);
     } else {
+        constexpr int G = E % 8 ? 4 : 8;
 #pragma unroll
-        for (int e = 0; e < E; e++) v[e] = exp_cordic_rt(v[e], iters, khinv);
+        for (int b = 0; b < E; b += G) exp_cordic_rt_vec<G>(v + b, iters, khinv);
     }
 }
 

@@ -53,7 +53,7 @@ WIDTHS = [1, 2, 3, 4, 63, 65, 101, 255, 256, 257, 511, 516, 767, 768, 769, 772, 
 @pytest.mark.parametrize("iters", [8, 11, 16])
 def test_softmax_layouts(n, rows, iters):
     from rac_amd import ext
-    if rows > 3 and (n > 1100 or iters == 11):
+    if rows > 3 and n > 1100:
         pytest.skip("one layout there; the small row count covers it")
     x = case(rows, n)
     same(ext.softmax(dev(x), iters), rl.orc_softmax_lanes(x, iters))
