@@ -61,7 +61,7 @@ __device__ __forceinline__ void exp_lane(float* v, int iters, float khinv) {
 #pragma unroll
         for (int b = 0; b < E; b += G) exp_cordic_vec<NITER, G, OPT>(v + b, khinv);
     } else {
-        constexpr int G = E % 8 ? 4 : 8;
+        constexpr int G = E < 4 ? E : E % 8 ? 4 : 8;
 #pragma unroll
         for (int b = 0; b < E; b += G) exp_cordic_rt_vec<G>(v + b, iters, khinv);
     }
@@ -76,6 +76,11 @@ __device__ __forceinline__ void exp_lane(float* v, int iters, float khinv) {
 // of lane l of each of the four waves, so it keeps four sums apart, runs the
 // four butterflies side by side and adds them in order.  It needs no barriers
 // and leaves no wave without a row.
+// VPT counts the lane's values in fours, 0 is a single one (row_values): a
+// ragged row of up to LANES values.  Held in four, three of them empty, it
+// took longer than in the strided loop before (900 x 130, 24 steps, 4.08 ->
+// 4.43 us; masked, three of 33 x 33, 3.8 -> 4.2), now 3.5 and 3.5.
+constexpr int row_values(int vpt) { return vpt ? 4 * vpt : 1; }
 template <int VEC_, int W_>
 struct RowLayout {
     static constexpr int VEC = VEC_, W = W_, LANES = 64 * W_;
@@ -113,7 +118,7 @@ template <class L, int VPT, bool MASKED, bool FULL>
 __device__ __forceinline__ float softmax_lane_max(float* v, long n, long t, const SoftmaxMask& mk) {
     if constexpr (MASKED) {
 #pragma unroll
-        for (int i = 0; i < 4 * VPT / L::VEC; i++) {
+        for (int i = 0; i < row_values(VPT) / L::VEC; i++) {
             const long j = (long)L::VEC * L::unit(i);
             if (FULL || j < n) {
 #pragma unroll
@@ -125,6 +130,7 @@ __device__ __forceinline__ float softmax_lane_max(float* v, long n, long t, cons
 #pragma unroll
     for (int i = 0; i < VPT; i++)
         m = fmaxf(fmaxf(fmaxf(m, v[4 * i]), fmaxf(v[4 * i + 1], v[4 * i + 2])), v[4 * i + 3]);
+    if constexpr (VPT == 0) m = fmaxf(m, v[0]);
     return m;
 }
 
@@ -133,7 +139,7 @@ template <class L, int VPT>
 __device__ __forceinline__ uint32_t lane_first_zero(const float* v) {
     uint32_t key = ~0u;
 #pragma unroll
-    for (int e = 4 * VPT - 1; e >= 0; e--)
+    for (int e = row_values(VPT) - 1; e >= 0; e--)
         if (v[e] == 0.0f) key = zero_key<uint32_t>(L::index(e), v[e]);
     return key;
 }
@@ -151,13 +157,13 @@ __device__ __forceinline__ void lane_sums(const float* v, float* s) {
 // whose step count is known only at run time).
 template <int VPT, int NITER, bool MASKED>
 __device__ __forceinline__ void softmax_lane_exps(float* v, float m, int iters, float khinv) {
-    constexpr int E = 4 * VPT;
+    constexpr int E = row_values(VPT);
 #pragma unroll
     for (int e = 0; e < E; e++) v[e] = v[e] - m;
     if constexpr (MASKED) {
         // the exps of -inf are +0: a wave skips the runs of its values that
         // are -inf in every lane (past the diagonal of a causal row)
-        constexpr int G = E % 8 || E == 8 ? 4 : 8;
+        constexpr int G = E < 4 ? E : E % 8 || E == 8 ? 4 : 8;
 #pragma unroll
         for (int b = 0; b < E; b += G) {
             bool some = false;
@@ -202,7 +208,7 @@ struct RowExtent {
 template <class L, int VPT, bool LDS_ONLY>
 __device__ __forceinline__ RowExtent unmasked_row_extent(const float* v, float* red, uint32_t* zred,
                                                          const float* row_lds = nullptr) {
-    constexpr int E = 4 * VPT;
+    constexpr int E = row_values(VPT);
     float mx = v[0], mn = v[0];
 #pragma unroll
     for (int e = 1; e < E; e++) {
@@ -269,7 +275,7 @@ __device__ __forceinline__ float unmasked_lane_sum(float s, RowExtent r) {
 template <class L, int VPT, int NITER, bool MASKED, bool FULL>
 __device__ __forceinline__ void softmax_row_regs(float* v, long n, long t, int iters, float khinv,
                                                  const SoftmaxMask& mk, float* red, uint32_t* zred) {
-    constexpr int E = 4 * VPT, S = L::sums(E);
+    constexpr int E = row_values(VPT), S = L::sums(E);
     float s[S], inv;
     if constexpr (!MASKED && NITER > 0) {
         const RowExtent r = unmasked_row_extent<L, VPT, false>(v, red, zred);
@@ -299,7 +305,7 @@ __device__ __forceinline__ void softmax_row_regs(float* v, long n, long t, int i
 template <class L, int VPT, bool FULL, bool MASKED = false>
 __device__ __forceinline__ void load_row_regs(const float* xr, long n, float* v, float pad, long last = 0) {
 #pragma unroll
-    for (int i = 0; i < 4 * VPT / L::VEC; i++) {
+    for (int i = 0; i < row_values(VPT) / L::VEC; i++) {
         const long j = (long)L::VEC * L::unit(i);
         const bool in = (FULL || j < n) && (!MASKED || j <= last);
         if constexpr (L::VEC == 4) {
@@ -315,7 +321,7 @@ __device__ __forceinline__ void load_row_regs(const float* xr, long n, float* v,
 template <class L, int VPT, bool FULL>
 __device__ __forceinline__ void store_row_regs(float* yr, long n, const float* v) {
 #pragma unroll
-    for (int i = 0; i < 4 * VPT / L::VEC; i++) {
+    for (int i = 0; i < row_values(VPT) / L::VEC; i++) {
         const long j = (long)L::VEC * L::unit(i);
         if (!FULL && j >= n) continue;
         if constexpr (L::VEC == 4)
@@ -336,7 +342,7 @@ __global__ __launch_bounds__(kRowThreads) void softmax_reg_kernel(
     __shared__ uint32_t zred[kRowWaves];
     const long row = L::row();
     if (L::W == 1 && row >= rows) return;
-    float v[4 * VPT];
+    float v[row_values(VPT)];
     const long t = MASKED ? mk.row0 + row % mk.seq : 0;
     load_row_regs<L, VPT, FULL, MASKED>(x + row * n, n, v, -__builtin_inff(), MASKED && mk.causal ? t : n);
     softmax_row_regs<L, VPT, NITER, MASKED, FULL>(v, n, t, iters, khinv, mk, red, zred);
@@ -515,13 +521,15 @@ static bool with_row_layout(long rows, long n, bool vec, long wide, F f) {
         constexpr int VEC = decltype(vec_c)::value;
         using L1 = RowLayout<VEC, 1>;
         using L4 = RowLayout<VEC, 4>;
-#define RAC_VPT(L, k) f(L(), std::integral_constant<int, k>())
+#define RAC_VPT(L, k) f(L(), std::integral_constant<int, (k) == 0 && VEC == 4 ? 1 : (k)>())
         if (n <= 1024 && per_cu >= (n <= 768 ? 4 : wide)) {
-            if (n <= 256) RAC_VPT(L1, 1);
+            if (VEC == 1 && n <= 64) RAC_VPT(L1, 0);
+            else if (n <= 256) RAC_VPT(L1, 1);
             else if (n <= 512) RAC_VPT(L1, 2);
             else if (n <= 768) RAC_VPT(L1, 3);
             else RAC_VPT(L1, 4);
-        } else if (n <= 1024) RAC_VPT(L4, 1);
+        } else if (VEC == 1 && n <= 256) RAC_VPT(L4, 0);
+        else if (n <= 1024) RAC_VPT(L4, 1);
         else if (n <= 2048) RAC_VPT(L4, 2);
         else if (n <= 4096) RAC_VPT(L4, 4);
         else if (n <= 8192) RAC_VPT(L4, 8);
@@ -605,7 +613,7 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_reg_kernel(
     const float* __restrict__ x, float* __restrict__ y, const float* __restrict__ gamma,
     float eps, long rows, long d, float khinv16)
 {
-    constexpr int E = 4 * VPT, S = L::sums(E);
+    constexpr int E = row_values(VPT), S = L::sums(E);
     __shared__ float red[kRowWaves];
     const long row = L::row();
     if (L::W == 1 && row >= rows) return;
@@ -651,7 +659,7 @@ __global__ __launch_bounds__(kRowThreads) void layernorm_reg_kernel(
     const float* __restrict__ x, float* __restrict__ y, const float* __restrict__ gamma,
     const float* __restrict__ beta, float eps, long rows, long d, float khinv16)
 {
-    constexpr int E = 4 * VPT, S = L::sums(E);
+    constexpr int E = row_values(VPT), S = L::sums(E);
     __shared__ float red[2 * kRowWaves];
     const long row = L::row();
     if (L::W == 1 && row >= rows) return;
