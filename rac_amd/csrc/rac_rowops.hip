@@ -318,16 +318,17 @@ __device__ __forceinline__ void load_row_regs(const float* xr, long n, float* v,
     }
 }
 
+template <int VEC>
+__device__ __forceinline__ void store_unit(float* y, const float* v) {
+    if constexpr (VEC == 4) st4_stream(reinterpret_cast<float4*>(y), make_float4(v[0], v[1], v[2], v[3]));
+    else *y = *v;
+}
 template <class L, int VPT, bool FULL>
 __device__ __forceinline__ void store_row_regs(float* yr, long n, const float* v) {
 #pragma unroll
     for (int i = 0; i < row_values(VPT) / L::VEC; i++) {
         const long j = (long)L::VEC * L::unit(i);
-        if (!FULL && j >= n) continue;
-        if constexpr (L::VEC == 4)
-            st4_stream(reinterpret_cast<float4*>(yr + j), make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]));
-        else
-            yr[j] = v[i];
+        if (FULL || j < n) store_unit<L::VEC>(yr + j, v + L::VEC * i);
     }
 }
 
@@ -608,12 +609,19 @@ __device__ __forceinline__ void load_weights(const float* w, long j, float none,
     }
 }
 
+// Rows of 64 values a lane store each unit as it is done, which frees its
+// registers; shorter ones all at the end: behind a store in between, the next
+// weights' load waits for it (8192 x 700 7.7 us against 8.5; but wide 1000 x
+// 15001 47.1 stored at the end, 43.0 so).
+constexpr bool wide_row(int vpt) { return vpt >= 16; }
+
 template <class L, int VPT>
 __global__ __launch_bounds__(kRowThreads) void rmsnorm_reg_kernel(
     const float* __restrict__ x, float* __restrict__ y, const float* __restrict__ gamma,
     float eps, long rows, long d, float khinv16)
 {
     constexpr int E = row_values(VPT), S = L::sums(E);
+    constexpr bool kWide = wide_row(VPT);
     __shared__ float red[kRowWaves];
     const long row = L::row();
     if (L::W == 1 && row >= rows) return;
@@ -621,7 +629,7 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_reg_kernel(
     load_row_regs<L, VPT, false>(x + row * d, d, v, 0.0f);
 #pragma unroll
     for (int e = 0; e < E; e++) ss[L::sum_of(e)] = __builtin_fmaf(v[e], v[e], ss[L::sum_of(e)]);
-    const float ms = L::template total<S>(ss, red) / (float)d;
+    const float ms = L::template total<S, kWide>(ss, red) / (float)d;
     const float inv = rsqrt_cordic(ms + eps, khinv16);
 #pragma unroll
     for (int i = 0; i < E / L::VEC; i++) {
@@ -631,9 +639,10 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_reg_kernel(
             load_weights<L::VEC>(gamma, j, 1.0f, g);
 #pragma unroll
             for (int c = 0; c < L::VEC; c++) v[L::VEC * i + c] = v[L::VEC * i + c] * inv * g[c];
+            if constexpr (kWide) store_unit<L::VEC>(y + row * d + j, v + L::VEC * i);
         }
     }
-    store_row_regs<L, VPT, false>(y + row * d, d, v);
+    if constexpr (!kWide) store_row_regs<L, VPT, false>(y + row * d, d, v);
 }
 
 __global__ __launch_bounds__(kRowThreads) void rmsnorm_loop_kernel(
@@ -660,6 +669,7 @@ __global__ __launch_bounds__(kRowThreads) void layernorm_reg_kernel(
     const float* __restrict__ beta, float eps, long rows, long d, float khinv16)
 {
     constexpr int E = row_values(VPT), S = L::sums(E);
+    constexpr bool kWide = wide_row(VPT);
     __shared__ float red[2 * kRowWaves];
     const long row = L::row();
     if (L::W == 1 && row >= rows) return;
@@ -667,10 +677,17 @@ __global__ __launch_bounds__(kRowThreads) void layernorm_reg_kernel(
     load_row_regs<L, VPT, false>(x + row * d, d, v, 0.0f);
     lane_sums<L, E>(v, sm);
     const float mean = L::template total<S>(sm, red) / (float)d;
+    // one bounds check a unit: one for each value cost a wide row 34 registers
+    // and a wave per SIMD (1000 x 16384 28.0 us, 21.2 so)
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-        const float z = v[e] - mean;
-        if (L::index(e) < d) sv[L::sum_of(e)] = __builtin_fmaf(z, z, sv[L::sum_of(e)]);
+    for (int i = 0; i < E / L::VEC; i++) {
+        if ((long)L::VEC * L::unit(i) < d) {
+#pragma unroll
+            for (int e = L::VEC * i; e < L::VEC * (i + 1); e++) {
+                const float z = v[e] - mean;
+                sv[L::sum_of(e)] = __builtin_fmaf(z, z, sv[L::sum_of(e)]);
+            }
+        }
     }
     const float var = L::template total<S>(sv, red + kRowWaves) / (float)d;
     const float inv = rsqrt_cordic(var + eps, khinv16);
@@ -686,9 +703,10 @@ __global__ __launch_bounds__(kRowThreads) void layernorm_reg_kernel(
                 float& o = v[L::VEC * i + c];
                 o = __builtin_fmaf(g[c], (o - mean) * inv, b[c]);
             }
+            if constexpr (kWide) store_unit<L::VEC>(y + row * d + j, v + L::VEC * i);
         }
     }
-    store_row_regs<L, VPT, false>(y + row * d, d, v);
+    if constexpr (!kWide) store_row_regs<L, VPT, false>(y + row * d, d, v);
 }
 
 __global__ __launch_bounds__(kRowThreads) void layernorm_loop_kernel(
