@@ -108,15 +108,25 @@ struct RowLayout {
     }
 };
 
+// Attention rows: with a causal limit or a mask, or (kGuarded) neither, only
+// the zero guard of the sum.  The latter have no runs of -inf to look for,
+// which took 8 heads of 2048 from 52.0 to 54.5 us, 49.0 without it; past
+// 4096 the exps in the search's groups of 8 hold fewer registers and win all
+// the same (1 x 6000 57.8 us against 61.0, 1 x 9000 145 against 209).
+// Under a mask that search gains where the mask holds -inf (8 x 512 10.2 ->
+// 7.9 us, 8 x 2048 78.1 -> 75.5) and costs where all of it is finite (8 x 2048
+// 80.3 -> 86.4, 16 x 1024 43.4 -> 45.5).
+constexpr int kGuarded = 1, kMasked = 2;
+
 // Softmax of the row a workgroup (or wave) holds in registers, E values per
 // lane, -inf past the row end, whose exp is +0, so the max, the lane sums
 // (s + 0 == s) and the outputs are those of the elements that exist.  On
 // return v holds the outputs.  t is the row's query position (masked rows
 // only).
 // First stage: masking (masked rows) and the lane's maximum.
-template <class L, int VPT, bool MASKED, bool FULL>
+template <class L, int VPT, int MASKED, bool FULL>
 __device__ __forceinline__ float softmax_lane_max(float* v, long n, long t, const SoftmaxMask& mk) {
-    if constexpr (MASKED) {
+    if constexpr (MASKED == kMasked) {
 #pragma unroll
         for (int i = 0; i < row_values(VPT) / L::VEC; i++) {
             const long j = (long)L::VEC * L::unit(i);
@@ -155,12 +165,12 @@ __device__ __forceinline__ void lane_sums(const float* v, float* s) {
 
 // Exps of the lane's values against the row maximum m (masked rows, and rows
 // whose step count is known only at run time).
-template <int VPT, int NITER, bool MASKED>
+template <int VPT, int NITER, int MASKED>
 __device__ __forceinline__ void softmax_lane_exps(float* v, float m, int iters, float khinv) {
     constexpr int E = row_values(VPT);
 #pragma unroll
     for (int e = 0; e < E; e++) v[e] = v[e] - m;
-    if constexpr (MASKED) {
+    if constexpr (MASKED == kMasked) {
         // the exps of -inf are +0: a wave skips the runs of its values that
         // are -inf in every lane (past the diagonal of a causal row)
         constexpr int G = E < 4 ? E : E % 8 || E == 8 ? 4 : 8;
@@ -272,7 +282,7 @@ __device__ __forceinline__ float unmasked_lane_sum(float s, RowExtent r) {
 
 // red: 2 kRowWaves floats (max and sum partials apart, so neither reduction
 // needs a trailing barrier; a kernel handles one row per workgroup).
-template <class L, int VPT, int NITER, bool MASKED, bool FULL>
+template <class L, int VPT, int NITER, int MASKED, bool FULL>
 __device__ __forceinline__ void softmax_row_regs(float* v, long n, long t, int iters, float khinv,
                                                  const SoftmaxMask& mk, float* red, uint32_t* zred) {
     constexpr int E = row_values(VPT), S = L::sums(E);
@@ -334,7 +344,7 @@ __device__ __forceinline__ void store_row_regs(float* yr, long n, const float* v
 
 // Rows held in registers: read once, reduced, exponentiated and written once.
 // FULL: n == 4 LANES VPT exactly, so no lane needs a bounds check.
-template <class L, int VPT, int NITER, bool MASKED, bool FULL>
+template <class L, int VPT, int NITER, int MASKED, bool FULL>
 __global__ __launch_bounds__(kRowThreads) void softmax_reg_kernel(
     const float* x, float* y, long rows, long n, int iters, float khinv,
     SoftmaxMask mk)
@@ -345,7 +355,7 @@ __global__ __launch_bounds__(kRowThreads) void softmax_reg_kernel(
     if (L::W == 1 && row >= rows) return;
     float v[row_values(VPT)];
     const long t = MASKED ? mk.row0 + row % mk.seq : 0;
-    load_row_regs<L, VPT, FULL, MASKED>(x + row * n, n, v, -__builtin_inff(), MASKED && mk.causal ? t : n);
+    load_row_regs<L, VPT, FULL, MASKED == kMasked>(x + row * n, n, v, -__builtin_inff(), MASKED && mk.causal ? t : n);
     softmax_row_regs<L, VPT, NITER, MASKED, FULL>(v, n, t, iters, khinv, mk, red, zred);
     store_row_regs<L, VPT, FULL>(y + row * n, n, v);
 }
@@ -486,7 +496,7 @@ __global__ __launch_bounds__(kRowThreads) void softmax_loop_kernel(
 constexpr long kCuLdsBytes = 160L * 1024;
 constexpr int unmasked_reg_cap(int vpt) { return vpt <= 2 ? 0 : vpt == 4 ? 6 : vpt == 8 ? 4 : 3; }
 
-template <class L, int VPT, int NITER, bool MASKED>
+template <class L, int VPT, int NITER, int MASKED>
 static void softmax_reg_launch(hipStream_t s, const float* x, float* y, long rows, long n, int iters,
                                float khinv, const SoftmaxMask& mk) {
     constexpr int cap = (!MASKED && NITER > 0 && L::W == 4) ? unmasked_reg_cap(VPT) : 0;
@@ -542,7 +552,7 @@ static bool with_row_layout(long rows, long n, bool vec, long wide, F f) {
     return vec ? at(std::integral_constant<int, 4>()) : at(std::integral_constant<int, 1>());
 }
 
-template <int NITER, bool MASKED>
+template <int NITER, int MASKED>
 static hipError_t softmax_dispatch(const float* x, float* y, long rows, long n, int iters,
                                    float khinv, hipStream_t s, const SoftmaxMask& mk) {
     const bool vec_ok = (n % 4 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0) &&
@@ -566,9 +576,10 @@ static hipError_t softmax_dispatch(const float* x, float* y, long rows, long n, 
             return hipGetLastError();
     }
     if (!with_row_layout(rows, n, vec_ok, 32, [&](auto l, auto vpt) {
-            softmax_reg_launch<decltype(l), decltype(vpt)::value, NITER, MASKED>(s, x, y, rows, n, iters, khinv, mk);
+            if constexpr (MASKED != kGuarded || decltype(vpt)::value <= 4)
+                softmax_reg_launch<decltype(l), decltype(vpt)::value, NITER, MASKED>(s, x, y, rows, n, iters, khinv, mk);
         }))
-        hipLaunchKernelGGL((softmax_loop_kernel<NITER, MASKED>), grid, block, 0, s, x, y, n, iters, khinv, mk);
+        hipLaunchKernelGGL((softmax_loop_kernel<NITER, MASKED != 0>), grid, block, 0, s, x, y, n, iters, khinv, mk);
     return hipGetLastError();
 }
 
@@ -579,9 +590,11 @@ static hipError_t softmax_mask_dispatch(const float* x, float* y, long rows, lon
         SoftmaxMask m2 = mk;
         if (m2.seq <= 0) m2.seq = n;   // square scores: row length = sequence length
         if (m2.mask_ld <= 0) m2.mask_ld = n;
-        return softmax_dispatch<NITER, true>(x, y, rows, n, iters, khinv, s, m2);
+        if (mk.mask || mk.causal || n > 4096)
+            return softmax_dispatch<NITER, kMasked>(x, y, rows, n, iters, khinv, s, m2);
+        return softmax_dispatch<NITER, kGuarded>(x, y, rows, n, iters, khinv, s, m2);
     }
-    return softmax_dispatch<NITER, false>(x, y, rows, n, iters, khinv, s, mk);
+    return softmax_dispatch<NITER, 0>(x, y, rows, n, iters, khinv, s, mk);
 }
 
 hipError_t softmax_launch(const float* x, float* y, long rows, long n, int iters, hipStream_t s,

@@ -85,10 +85,10 @@ def test_masked_softmax_layouts(T):
     s = rl.gen_normal((1030 // T + 1 if T < 300 else 4, T, T), seed=T)
     s[0, 0] = 0.0
     mask = rl.gen_normal((T, T), seed=T + 1)
-    for causal, m in ((True, None), (True, mask), (False, mask)):
+    for causal, m in ((True, None), (True, mask), (False, mask), (False, None)):
         got = ext.softmax_masked_(dev(s), None if m is None else dev(m), causal, 16)
         for b in range(s.shape[0]):
-            same(got[b], rl.orc_softmax_lanes(s[b], 16, causal=causal, mask=m))
+            same(got[b], rl.orc_softmax_lanes(s[b], 16, causal=causal, mask=m, zero_guard=True))
 
 
 @pytest.mark.parametrize("rows,n", [(3, 260), (1030, 500), (3, 2000), (1030, 768)])
