@@ -357,25 +357,29 @@ __global__ __launch_bounds__(256) void q8_gemv_generic_kernel(const float* __res
 
 // One input row on the fast path: the workgroup shape by the number of
 // rows.  16 rows per workgroup while that still gives two workgroups per
-// CU; below, 4 rows (8 when a row has fewer than 64 blocks, or when every
-// workgroup computes the norm first) so that small matrices spread over
-// every CU (measured on MI355X with weights streamed from HBM: 2048 x 5632
-// in 6.0 us instead of 8.3; 2560 x 2048 behind a norm in 5.6 on 8 rows, 5.9 on
-// 4).  Rows of 16-31 blocks in chunks of 16 (512 x 512 2.7 us, in chunks of 8
-// with 32 rows 3.4; 3072 x 512 behind a norm 4.0 against 4.7).  The shape only
-// changes which lane computes what.
+// CU; below, 4 rows (8 when a row has fewer than 64 blocks) so that small
+// matrices spread over every CU (measured on MI355X with weights streamed
+// from HBM: 2048 x 5632 in 6.0 us instead of 8.3).  Where every workgroup
+// computes the norm first, 8 rows halve that work, but their chunks of 32
+// blocks double the steps that a row takes one after the other: the two meet
+// at a number of workgroups that grows with the square root of K (us, 8 rows /
+// 4: 1500 x 2048 4.4 / 4.6, 1000 4.3 / 4.0; 2100 x 4096 7.1 / 7.4, 1000 6.5 /
+// 5.6; 4000 x 8192 12.8 / 14.6, 2560 11.2 / 11.2, 1024 9.9 / 7.8; 3000 x 16384
+// 21.0 / 20.0).  Rows of 16-31 blocks in chunks of 16 (512 x 512 2.7 us, in
+// chunks of 8 with 32 rows 3.4; 3072 x 512 behind a norm 4.0 against 4.7).  The
+// shape only changes which lane computes what.
 template <bool NORM, int EPI>
 static void q8_launch_row(const float* x, const uint8_t* w, const float* bias, float* out, int N, int K, int act,
                           const Q8Fuse& fz, hipStream_t s) {
     const int nb = K / kQ8Block;
-    const long cus = device_cus();
+    const long cus = device_cus(), wg8 = (N + 7) / 8;
 #define RAC_Q8_ROW(CB, R)                                                                                   \
     hipLaunchKernelGGL((q8_gemv_kernel<1, CB, R, NORM, EPI>), dim3((unsigned)((N + R - 1) / R)), dim3(256), 0, \
                        s, x, w, bias, out, 1, N, K, act, fz)
     if (nb < 16) RAC_Q8_ROW(8, 32);
     else if (nb < 32) RAC_Q8_ROW(16, 16);
     else if ((N + 15) / 16 >= 2 * cus) RAC_Q8_ROW(32, 16);
-    else if (nb >= 64 && !NORM) RAC_Q8_ROW(64, 4);
+    else if (nb >= 64 && (!NORM || 160 * wg8 * wg8 <= cus * cus * nb)) RAC_Q8_ROW(64, 4);
     else RAC_Q8_ROW(32, 8);
 #undef RAC_Q8_ROW
 }
