@@ -443,7 +443,9 @@ static hipError_t sk_launch(const SkinnyArgs& g, hipStream_t s) {
 // -> 158.3.  With 2.7 workgroups per CU its VGPRs cost a wave per SIMD
 // (FAST 16x11008x4096 77.7 -> 83.2 us), and one-row CORDIC and SHIFTADD
 // gained nothing (CORDIC 1x4096x4096 54.3 -> 55.1, SHIFTADD 1x11008x4096
-// 271.7 -> 279.7 us), so they keep the loop.
+// 271.7 -> 279.7 us), so they keep the loop.  (The FAST figures here and
+// below are of long K, which the matrix cores run now; the forms they chose
+// serve the short K that fast_few_rows in rac_gemm.hip still sends here.)
 template <int MODE, int NITER, bool TB, bool FUSED, int RB, int CB, bool FEWCOL>
 static hipError_t sk_block(const SkinnyArgs& g, hipStream_t s) {
     const long wgs = (FEWCOL ? (long)((g.M + RB - 1) / RB) : (long)((g.N + CB - 1) / CB)) * g.batch;

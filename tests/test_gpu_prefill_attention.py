@@ -48,3 +48,20 @@ def test_prefill_attention_matches_its_stages(nkv, rep, T, start, dh):
         got = ext.prefill_attention(q, kc, vc, T, start, scale, 16)
         assert torch.isfinite(got).all()
         assert torch.equal(got, want)
+
+
+def test_prefill_attention_composed_form():
+    """RACDecoder's form for more query rows than the native call takes: the
+    same result."""
+    from types import SimpleNamespace
+
+    from rac_amd import ext
+    from rac_amd.decoder import RACDecoder
+    nkv, rep, T, start, dh = 2, 3, 37, 11, 16
+    kc, vc = (torch.from_numpy(rl.gen_normal((nkv, 64, dh), seed=s)).to(DEV) for s in (2, 3))
+    dec = SimpleNamespace(cfg=SimpleNamespace(n_kv_heads=nkv, n_heads=nkv * rep, d_head=dh, d_model=nkv * rep * dh),
+                          k_cache=[kc], v_cache=[vc], scale=ext.attention_scale(dh), iters=16)
+    q = torch.from_numpy(rl.gen_normal((T, nkv * rep * dh), seed=1)).to(DEV)
+    qg = q.view(T, nkv, rep, dh).permute(1, 2, 0, 3).reshape(nkv, rep * T, dh).contiguous()
+    want = RACDecoder._prefill_attention_composed(dec, 0, qg, start, T)
+    assert torch.equal(RACDecoder._prefill_attention(dec, 0, q, start, T), want)
