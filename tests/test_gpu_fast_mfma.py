@@ -116,7 +116,7 @@ SPECIALS = np.array([0.0, -0.0, 1e-45, -3e-39, 2.0 ** -126, -(2.0 ** -110), 3e38
 @pytest.mark.parametrize("layout", [(0, 0), (1, 1)])
 def test_fast_mfma_special_values(layout, shape):
     """Subnormal, huge, infinite and NaN operands through the matrix cores:
-    every finite output bit-exact, NaN exactly where the checker has NaN."""
+    every finite output bit-exact, NaN exactly where the oracle has NaN."""
     M, N, K = shape
     ta, tb = layout
     rng = np.random.default_rng(5)
@@ -171,7 +171,7 @@ def test_fast_mfma_batched(ta, tb):
 def test_fast_mfma_fused_linear(act):
     """linear_forward and fused_linear_forward (bias + activation in the
     epilogue) on 32x32 tiles: pre-activations equal the unfused product
-    plus bias, bit-exact vs the checker; outputs equal the activation kernel
+    plus bias, bit-exact against the oracle; outputs equal the activation kernel
     applied to them."""
     e = ext()
     M, N, K = 2050, 2049, 300
@@ -195,7 +195,7 @@ def test_fast_mfma_fused_linear(act):
 def test_fast_attention_config5_mfma_products(causal):
     """The config-5 attention core in FAST mode: each 512-row chunk's P V
     (32 heads of 512 x 128, the causal K limit per row tile) equals the
-    one-chunk form's (32 heads of 2048 x 128) and the checker's composition
+    one-chunk form's (32 heads of 2048 x 128) and the oracle's composition
     on sampled heads, bit for bit."""
     e = ext()
     shape = (1, 32, 2048, 128)
@@ -212,7 +212,7 @@ def test_fast_attention_config5_mfma_products(causal):
 
 @pytest.mark.parametrize("Z,M,N,K", [(32, 512, 128, 600), (1, 1024, 1024, 1030), (8, 512, 512, 512)])
 def test_fast_mfma_few_blocks(Z, M, N, K):
-    """Launches of one 64x64 tile to a CU: bit-exact vs the checker."""
+    """Launches of one 64x64 tile to a CU: bit-exact against the oracle."""
     e = ext()
     A = rl.gen_uniform((Z, M, K), seed=Z + M)
     B = rl.gen_uniform((Z, K, N), seed=N + K)
@@ -244,7 +244,7 @@ def test_fast_attention_chunks_mfma():
     """[1, 16, 512, 128] in FAST mode: the causal scores of each chunk of
     query rows (the trapezoid of tiles on or below the diagonal) and P V run
     on the matrix cores, and every chunk size gives the one-chunk bits, which
-    equal the checker's."""
+    equal the oracle's."""
     e = ext()
     shape = (1, 16, 512, 128)
     q = rl.gen_normal(shape, seed=720)
